@@ -220,12 +220,11 @@ void free_batch(ehd_batch* bt)
     if (bt->st) (void)hipStreamDestroy(bt->st);
 }
 
-// Divisors of ny/2 up to the largest line count that fits, largest first.
-std::vector<int> x_candidates(int ny, int maxl)
+// The largest line count of a block and up to three halvings of it.
+std::vector<int> x_candidates(int maxl)
 {
     std::vector<int> c;
-    for (int l = maxl; l >= 1 && c.size() < 4; --l)
-        if ((ny / 2) % l == 0) c.push_back(l);
+    for (int l = maxl; l >= 1 && c.size() < 4; l /= 2) c.push_back(l);
     return c;
 }
 
@@ -288,7 +287,7 @@ int tune(ehd_batch* bt)
         const PoissonShape ps = poisson_shape(bt->prec, gr.g.nx, gr.g.ny, gr.g.max_n + 2);
         double best = 1e30;
         int bl = 0, by = 0;
-        for (int xl : x_candidates(gr.g.ny, ps.max_x_lines))
+        for (int xl : x_candidates(ps.max_x_lines))
             for (int yl : {ps.max_y_lines, ps.max_y_lines / 2, ps.max_y_lines / 4}) {
                 if (yl < 1) continue;
                 gr.g.lpb = xl;

@@ -15,14 +15,17 @@
 // with the wall potential carried by phi_L(z) = V (1 - z/(nz-1)), which the
 // second-difference operator annihilates (the lifting terms V/dz^2 of
 // poisson.cu:99,119 only ever reach mode (0,0)).  The DFTs are Stockham
-// mixed-radix FFTs in LDS (radix 4, 2, 3, 5 butterflies; any other prime
-// factor is done as a direct DFT stage).
+// mixed-radix FFTs in LDS with register butterflies of up to 16 points
+// (radices 2 to 5, 7 to 9, 11, 13, 16); a larger prime factor is a stage of
+// half the products of the direct DFT.
 //
 // Spectral layout: [z-1][kx][ky], kx in [0, nx/2], ky fastest.
 // FP32S path: the spectra are float; mode (0,0) is solved in FP64 and kept
 // as the per-plane mean phibar[z] (FP64), and phi holds phi - phibar in
 // float, so that E = -grad(phi) loses no digits to the large wall potential.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "ehd_internal.h"
 #include "fft_plan.h"
@@ -76,110 +79,6 @@ __device__ __forceinline__ cplx<T> root(const cplx<T>* tw, int m, int sign)
     cplx<T> w = tw[m];
     if (sign > 0) w.y = -w.y;
     return w;
-}
-
-// Stockham FFT of nlines lines (line l at buf[l*ldl]) held in LDS, ping-pong
-// between A and B.  sign -1 forward, +1 inverse, unnormalised.  Returns the
-// buffer that holds the result.  Every thread of the block must call it.
-template <typename T>
-__device__ cplx<T>* lds_fft(cplx<T>* A, cplx<T>* B, int n, int nlines, int ldl, const FftPlan& pl,
-                            const cplx<T>* __restrict__ tw, int sign)
-{
-    const int tid = threadIdx.x, nthr = blockDim.x;
-    const T sg = (T)sign;
-    cplx<T>* in = A;
-    cplx<T>* out = B;
-    int Ns = 1;
-    for (int st = 0; st < pl.nst; ++st) {
-        const int R = pl.rad[st];
-        const int nb = n / R;
-        const int tstep = n / (Ns * R);
-        if (R == 2 || R == 4) {
-            for (int w = tid; w < nlines * nb; w += nthr) {
-                const int l = w / nb, j = w - l * nb, k = j % Ns;
-                const cplx<T>* src = in + l * ldl + j;
-                cplx<T>* dst = out + l * ldl + (j / Ns) * Ns * R + k;
-                if (R == 2) {
-                    cplx<T> a = src[0];
-                    cplx<T> b = cmul(src[nb], root(tw, k * tstep, sign));
-                    dst[0] = cadd(a, b);
-                    dst[Ns] = csub(a, b);
-                } else {
-                    cplx<T> a = src[0];
-                    cplx<T> b = cmul(src[nb], root(tw, k * tstep, sign));
-                    cplx<T> c = cmul(src[2 * nb], root(tw, 2 * k * tstep, sign));
-                    cplx<T> d = cmul(src[3 * nb], root(tw, 3 * k * tstep, sign));
-                    cplx<T> t0 = cadd(a, c), t1 = csub(a, c), t2 = cadd(b, d), t3 = csub(b, d);
-                    // W4 = exp(sign*i*pi/2) = i*sign
-                    cplx<T> it3 = cis(t3, sg);
-                    dst[0] = cadd(t0, t2);
-                    dst[Ns] = cadd(t1, it3);
-                    dst[2 * Ns] = csub(t0, t2);
-                    dst[3 * Ns] = csub(t1, it3);
-                }
-            }
-        } else if (R == 3) {
-            const T s3 = (T)0.86602540378443864676;  // sin(2 pi/3)
-            for (int w = tid; w < nlines * nb; w += nthr) {
-                const int l = w / nb, j = w - l * nb, k = j % Ns;
-                const cplx<T>* src = in + l * ldl + j;
-                cplx<T>* dst = out + l * ldl + (j / Ns) * Ns * R + k;
-                cplx<T> a = src[0];
-                cplx<T> b = cmul(src[nb], root(tw, k * tstep, sign));
-                cplx<T> c = cmul(src[2 * nb], root(tw, 2 * k * tstep, sign));
-                cplx<T> t1 = cadd(b, c);
-                cplx<T> t2 = {a.x - (T)0.5 * t1.x, a.y - (T)0.5 * t1.y};
-                cplx<T> t3 = csub(b, c);
-                cplx<T> r = cis(cplx<T>{s3 * t3.x, s3 * t3.y}, sg);
-                dst[0] = cadd(a, t1);
-                dst[Ns] = cadd(t2, r);
-                dst[2 * Ns] = csub(t2, r);
-            }
-        } else if (R == 5) {
-            const T c1 = (T)0.30901699437494742410, c2 = (T)-0.80901699437494742410;
-            const T s1 = (T)0.95105651629515357212, s2 = (T)0.58778525229247312917;
-            for (int w = tid; w < nlines * nb; w += nthr) {
-                const int l = w / nb, j = w - l * nb, k = j % Ns;
-                const cplx<T>* src = in + l * ldl + j;
-                cplx<T>* dst = out + l * ldl + (j / Ns) * Ns * R + k;
-                cplx<T> a = src[0];
-                cplx<T> b = cmul(src[nb], root(tw, k * tstep, sign));
-                cplx<T> c = cmul(src[2 * nb], root(tw, 2 * k * tstep, sign));
-                cplx<T> d = cmul(src[3 * nb], root(tw, 3 * k * tstep, sign));
-                cplx<T> e = cmul(src[4 * nb], root(tw, 4 * k * tstep, sign));
-                cplx<T> t1 = cadd(b, e), t2 = cadd(c, d), t3 = csub(b, e), t4 = csub(c, d);
-                cplx<T> m1 = {a.x + c1 * t1.x + c2 * t2.x, a.y + c1 * t1.y + c2 * t2.y};
-                cplx<T> m2 = {a.x + c2 * t1.x + c1 * t2.x, a.y + c2 * t1.y + c1 * t2.y};
-                cplx<T> n1 = cis(cplx<T>{s1 * t3.x + s2 * t4.x, s1 * t3.y + s2 * t4.y}, sg);
-                cplx<T> n2 = cis(cplx<T>{s2 * t3.x - s1 * t4.x, s2 * t3.y - s1 * t4.y}, sg);
-                dst[0] = cadd(a, cadd(t1, t2));
-                dst[Ns] = cadd(m1, n1);
-                dst[2 * Ns] = cadd(m2, n2);
-                dst[3 * Ns] = csub(m2, n2);
-                dst[4 * Ns] = csub(m1, n1);
-            }
-        } else {
-            // direct DFT stage for any other prime: one thread per output
-            for (int w = tid; w < nlines * n; w += nthr) {
-                const int l = w / n, o = w - l * n;
-                const int k = o % Ns, q = (o / Ns) % R, jb = o / (Ns * R);
-                const int j = jb * Ns + k;
-                const cplx<T>* src = in + l * ldl + j;
-                cplx<T> acc = {(T)0, (T)0};
-                for (int r = 0; r < R; ++r) {
-                    cplx<T> v = cmul(src[r * nb], root(tw, (r * k * tstep) % n, sign));
-                    acc = cadd(acc, cmul(v, root(tw, ((r * q) % R) * nb, sign)));
-                }
-                out[l * ldl + o] = acc;
-            }
-        }
-        __syncthreads();
-        cplx<T>* tmp = in;
-        in = out;
-        out = tmp;
-        Ns *= R;
-    }
-    return in;
 }
 
 // ---------------------------------------------------------------------------
@@ -253,6 +152,68 @@ __device__ __forceinline__ void dft4(cplx<T>& a, cplx<T>& b, cplx<T>& c, cplx<T>
     d = csub(t1, it3);
 }
 
+// cos and sin of 2 pi m / R, m = 1 .. R/2, of the odd radices done by pairs
+template <int R>
+struct Roots;
+template <>
+struct Roots<7> {
+    static constexpr double c[3] = {0.6234898018587335305250, -0.2225209339563144042889, -0.9009688679024191262361};
+    static constexpr double s[3] = {0.7818314824680298087084, 0.9749279121818236070181, 0.4338837391175581204758};
+};
+template <>
+struct Roots<9> {
+    static constexpr double c[4] = {0.7660444431189780352024, 0.1736481776669303488517, -0.5, -0.9396926207859083840541};
+    static constexpr double s[4] = {0.6427876096865393263226, 0.9848077530122080593667, 0.8660254037844386467637,
+                                    0.3420201433256687330441};
+};
+template <>
+struct Roots<11> {
+    static constexpr double c[5] = {0.8412535328311811688618, 0.4154150130018864255293, -0.1423148382732851404438,
+                                    -0.6548607339452850640569, -0.9594929736144973898904};
+    static constexpr double s[5] = {0.5406408174555975821076, 0.9096319953545183714117, 0.9898214418809327323761,
+                                    0.7557495743542582837740, 0.2817325568414296977114};
+};
+template <>
+struct Roots<13> {
+    static constexpr double c[6] = {0.8854560256532098959004, 0.5680647467311558025118, 0.1205366802553230533491,
+                                    -0.3546048870425356259696, -0.7485107481711010986346, -0.9709418174260520271570};
+    static constexpr double s[6] = {0.4647231720437685456560, 0.8229838658936563945796, 0.9927088740980539928008,
+                                    0.9350162426854148234398, 0.6631226582407952023768, 0.2393156642875577671488};
+};
+
+// DFT of odd length R from the sums and differences of the pairs (r, R - r):
+// X_q, X_{R-q} = (x_0 + sum_r cos(2 pi r q/R) s_r) +- i sg sum_r sin(2 pi r q/R) d_r,
+// half the products of the direct sum
+template <typename T, int R>
+__device__ __forceinline__ void bfly_pairs(cplx<T>* v, T sg)
+{
+    constexpr int H = R / 2;
+    cplx<T> s[H], d[H], x0 = v[0];
+#pragma unroll
+    for (int r = 1; r <= H; ++r) {
+        s[r - 1] = cadd(v[r], v[R - r]);
+        d[r - 1] = csub(v[r], v[R - r]);
+        v[0] = cadd(v[0], s[r - 1]);
+    }
+#pragma unroll
+    for (int q = 1; q <= H; ++q) {
+        cplx<T> a = x0, b = {(T)0, (T)0};
+#pragma unroll
+        for (int r = 1; r <= H; ++r) {
+            const int m = (r * q) % R, n = m <= H ? m : R - m;   // n = 0 only for R = 9
+            const T c = n > 0 ? (T)Roots<R>::c[n > 0 ? n - 1 : 0] : (T)1;
+            const T sn = n > 0 ? (T)(m <= H ? Roots<R>::s[n > 0 ? n - 1 : 0] : -Roots<R>::s[n > 0 ? n - 1 : 0]) : (T)0;
+            a.x += c * s[r - 1].x;
+            a.y += c * s[r - 1].y;
+            b.x += sn * d[r - 1].x;
+            b.y += sn * d[r - 1].y;
+        }
+        const cplx<T> ib = cis(b, sg);
+        v[q] = cadd(a, ib);
+        v[R - q] = csub(a, ib);
+    }
+}
+
 template <typename T, int R>
 __device__ __forceinline__ void bfly(cplx<T>* v, T sg)
 {
@@ -308,6 +269,8 @@ __device__ __forceinline__ void bfly(cplx<T>* v, T sg)
         v[0] = cadd(a, t1);
         v[1] = cadd(t2, r);
         v[2] = csub(t2, r);
+    } else if constexpr (R == 7 || R == 9 || R == 11 || R == 13) {
+        bfly_pairs<T, R>(v, sg);
     } else {
         static_assert(R == 5, "radix");
         const T c1 = (T)0.30901699437494742410, c2 = (T)-0.80901699437494742410;
@@ -330,10 +293,12 @@ __device__ __forceinline__ void bfly(cplx<T>* v, T sg)
 // stage then spread over the banks instead of a few of them.
 __host__ __device__ constexpr int padi(int i) { return i + (i >> 4); }
 // LDS line pitch (complex elements): long enough for the padded line and
-// = 1 mod 32, so that threads walking across lines hit distinct banks.
+// = 1 mod 32 (runtime plans: odd), so that threads walking across lines hit
+// distinct banks.
 __host__ __device__ constexpr int lds_pitch(int N, int n)
 {
-    const int len = N > 0 ? padi(N - 1) + 1 : n;
+    if (N == 0) return n | 1;
+    const int len = padi(N - 1) + 1;
     return ((len + 30) / 32) * 32 + 1;
 }
 
@@ -387,18 +352,193 @@ __device__ __forceinline__ void ct_run(const LD& ld, const SF& sf, cplx<T>* buf,
     }
 }
 
+// ---------------------------------------------------------------------------
+// Runtime-planned FFT (every other size): a Stockham FFT of nl <= 2^lg lines
+// in LDS, ping-pong between two buffers, one register butterfly per thread
+// and turn.  The lines run fastest over the threads (line pitch odd), so the
+// reads and writes of a stage hit distinct banks whatever its strides, the
+// twiddles are broadcasts, and the only divisions left are by the stage's Ns,
+// done by a multiplication.
+
+// a / b of a magic number from fft_magic(b): exact for a < 2^16
+__device__ __forceinline__ int fdiv(int a, unsigned magic) { return (int)__umulhi((unsigned)a, magic); }
+
+template <typename T, int R>
+__device__ __forceinline__ void rt_stage(const cplx<T>* in, cplx<T>* out, int nl, int lg, int ldl, int nb, int Ns,
+                                         unsigned mNs, const cplx<T>* __restrict__ tw, int sign)
+{
+    const T sg = (T)sign;
+    const int tstep = Ns > 1 ? fdiv(nb, mNs) : nb;   // n / (Ns R)
+    for (int w = threadIdx.x; w < (nb << lg); w += blockDim.x) {
+        const int l = w & ((1 << lg) - 1), j = w >> lg;
+        if (l >= nl) continue;
+        const cplx<T>* src = in + l * ldl + j;
+        cplx<T> v[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] = src[r * nb];
+        int o = j * R;
+        if (Ns > 1) {
+            const int jq = fdiv(j, mNs), k = j - jq * Ns;
+            o = jq * Ns * R + k;
+#pragma unroll
+            for (int r = 1; r < R; ++r) v[r] = cmul(v[r], root(tw, r * k * tstep, sign));
+        }
+        bfly<T, R>(v, sg);
+        cplx<T>* dst = out + l * ldl + o;
+#pragma unroll
+        for (int r = 0; r < R; ++r) dst[r * Ns] = v[r];
+    }
+}
+
+// A stage of any other prime R (17 and up): the pairs (r, R - r) become their
+// sums and differences in place (after the twiddles), then every thread forms
+// PQ output pairs q, R - q of one butterfly; the roots are the same for all
+// lines (broadcasts), each sum and difference serves PQ outputs.
+// 122 = 61 * 2, FP64, 122x122x101, one y pass: 114 us with one thread per
+// output and a modulo per term, 20 us so (the x passes 88 and 84, now 24 and 21).
+template <typename T>
+__device__ __forceinline__ void rt_prime_stage(cplx<T>* in, cplx<T>* out, int R, int nl, int lg, int ldl, int nb,
+                                               unsigned mnb, int Ns, unsigned mNs, const cplx<T>* __restrict__ tw,
+                                               int sign)
+{
+    constexpr int PQ = 4;
+    const T sg = (T)sign;
+    const int H = R >> 1, tstep = Ns > 1 ? fdiv(nb, mNs) : nb, lm = (1 << lg) - 1;
+    for (int w = threadIdx.x; w < ((nb * H) << lg); w += blockDim.x) {
+        const int l = w & lm, e = w >> lg, r = fdiv(e, mnb) + (nb == 1 ? e : 0) + 1;
+        const int j = nb == 1 ? 0 : e - (r - 1) * nb;
+        if (l >= nl) continue;
+        cplx<T>* p = in + l * ldl + j;
+        cplx<T> a = p[r * nb], b = p[(R - r) * nb];
+        if (Ns > 1) {
+            const int k = j - fdiv(j, mNs) * Ns;
+            a = cmul(a, root(tw, r * k * tstep, sign));
+            b = cmul(b, root(tw, (R - r) * k * tstep, sign));
+        }
+        p[r * nb] = cadd(a, b);
+        p[(R - r) * nb] = csub(a, b);
+    }
+    __syncthreads();
+    const int ng = (H + PQ) / PQ;    // groups of PQ outputs over q = 0..H
+    for (int w = threadIdx.x; w < ((nb * ng) << lg); w += blockDim.x) {
+        const int l = w & lm, e = w >> lg, g = nb == 1 ? e : fdiv(e, mnb), j = e - g * nb;
+        if (l >= nl) continue;
+        const cplx<T>* p = in + l * ldl + j;
+        const cplx<T> x0 = p[0];
+        cplx<T> a[PQ], b[PQ];
+        int m[PQ], q[PQ];
+#pragma unroll
+        for (int i = 0; i < PQ; ++i) {
+            a[i] = x0;
+            b[i] = {(T)0, (T)0};
+            q[i] = min(g * PQ + i, H);
+            m[i] = 0;
+        }
+        for (int r = 1; r <= H; ++r) {
+            const cplx<T> s = p[r * nb], d = p[(R - r) * nb];
+#pragma unroll
+            for (int i = 0; i < PQ; ++i) {
+                m[i] += q[i];
+                m[i] -= m[i] >= R ? R : 0;
+                const cplx<T> c = tw[m[i] * nb];   // cos, -sin of 2 pi r q / R
+                a[i].x += c.x * s.x;
+                a[i].y += c.x * s.y;
+                b[i].x -= c.y * d.x;
+                b[i].y -= c.y * d.y;
+            }
+        }
+        const int jq = Ns > 1 ? fdiv(j, mNs) : j, k = Ns > 1 ? j - jq * Ns : 0;
+        cplx<T>* dst = out + l * ldl + jq * Ns * R + k;
+#pragma unroll
+        for (int i = 0; i < PQ; ++i) {
+            const cplx<T> ib = cis(b[i], sg);
+            if (g * PQ + i <= H) {
+                dst[q[i] * Ns] = cadd(a[i], ib);
+                if (q[i] > 0) dst[(R - q[i]) * Ns] = csub(a[i], ib);
+            }
+        }
+    }
+}
+
+// Runs plan pl on the lines A[l*ldl ..], l < nl; returns the buffer (A or B)
+// that holds the result.  Unnormalised, sign -1 forward, +1 inverse.  Every
+// thread of the block must call it, with A's writes behind a barrier.
+template <typename T>
+__device__ cplx<T>* rt_fft(cplx<T>* A, cplx<T>* B, const FftPlan& pl, int nl, int lg, int ldl,
+                           const cplx<T>* __restrict__ tw, int sign)
+{
+    cplx<T>* in = A;
+    cplx<T>* out = B;
+    int Ns = 1;
+    for (int st = 0; st < pl.nst; ++st) {
+        const int R = pl.rad[st], nb = pl.nb[st];
+        const unsigned mNs = pl.mns[st];
+        switch (R) {
+        case 2: rt_stage<T, 2>(in, out, nl, lg, ldl, nb, Ns, mNs, tw, sign); break;
+        case 3: rt_stage<T, 3>(in, out, nl, lg, ldl, nb, Ns, mNs, tw, sign); break;
+        case 4: rt_stage<T, 4>(in, out, nl, lg, ldl, nb, Ns, mNs, tw, sign); break;
+        case 5: rt_stage<T, 5>(in, out, nl, lg, ldl, nb, Ns, mNs, tw, sign); break;
+        case 7: rt_stage<T, 7>(in, out, nl, lg, ldl, nb, Ns, mNs, tw, sign); break;
+        case 8: rt_stage<T, 8>(in, out, nl, lg, ldl, nb, Ns, mNs, tw, sign); break;
+        case 9: rt_stage<T, 9>(in, out, nl, lg, ldl, nb, Ns, mNs, tw, sign); break;
+        case 11: rt_stage<T, 11>(in, out, nl, lg, ldl, nb, Ns, mNs, tw, sign); break;
+        case 13: rt_stage<T, 13>(in, out, nl, lg, ldl, nb, Ns, mNs, tw, sign); break;
+        case 16: rt_stage<T, 16>(in, out, nl, lg, ldl, nb, Ns, mNs, tw, sign); break;
+        default: rt_prime_stage<T>(in, out, R, nl, lg, ldl, nb, pl.mnb[st], Ns, mNs, tw, sign); break;
+        }
+        __syncthreads();
+        cplx<T>* tmp = in;
+        in = out;
+        out = tmp;
+        Ns *= R;
+    }
+    return in;
+}
+
+// A thread's turn over the count elements of a block's contiguous rows of n:
+// U loads ld(l, i) in flight, then their stores st(l, i, v); mn = fft_magic(n)
+template <int U, typename V, class LD, class ST>
+__device__ __forceinline__ void rows_copy(int count, int n, unsigned mn, const LD& ld, const ST& st)
+{
+    for (int e0 = threadIdx.x; e0 < count; e0 += U * blockDim.x) {
+        V v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int e = e0 + u * blockDim.x, l = fdiv(e, mn);
+            if (e < count) v[u] = ld(l, e - l * n);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int e = e0 + u * blockDim.x, l = fdiv(e, mn);
+            if (e < count) st(l, e - l * n, v[u]);
+        }
+    }
+}
+
+// a compile-time plan needs no argument (and no work on the host)
+struct NoPlan {};
+template <int N>
+using PlanArg = std::conditional_t<(N > 0), NoPlan, FftPlan>;
+template <int N>
+PlanArg<N> plan_arg(int n)
+{
+    if constexpr (N > 0) return NoPlan{};
+    else return make_fft_plan(n);
+}
+
 // Spectral layout (both precisions): [z-1][kx][ky], ky fastest, kx in
 // [0, nx/2]: the y transforms run over contiguous lines and the z solve over
 // contiguous modes m = kx*ny + ky.
 
 // (1a) R2C along x of s = -q/eps on interior rows, two real rows per complex
-// line.  A block takes 2*lpb consecutive rows y0.. of one plane; lpb divides
-// ny/2.  The spectrum is written transposed, 2*lpb consecutive ky per kx.
+// line.  A block takes up to 2*lpb = 2^(lg+1) consecutive rows y0.. of one
+// plane (the last block of a plane what is left).  The spectrum is written
+// transposed, 2*lpb consecutive ky per kx.
 // LDS: twiddles (nx), line buffers (lpb lines; two for the runtime plan).
 template <typename T, int N>
 __global__ void __launch_bounds__(256) fftx_fwd_kernel(const PoissonJob* __restrict__ jobs,
-                                                       const cplx<T>* __restrict__ tw, FftPlan pl, int nx_rt,
-                                                       int ny, int lpb)
+                                                       const cplx<T>* __restrict__ tw, PlanArg<N> pl, int nx_rt,
+                                                       int ny, int lpb, int lg)
 {
     const PoissonJob& J = jobs[blockIdx.y];
     const int nx = N > 0 ? N : nx_rt;
@@ -407,10 +547,11 @@ __global__ void __launch_bounds__(256) fftx_fwd_kernel(const PoissonJob* __restr
     extern __shared__ unsigned char smem_raw[];
     cplx<T>* tws = reinterpret_cast<cplx<T>*>(smem_raw);
     cplx<T>* A = tws + nx;
-    const int groups = ny / (2 * lpb);
+    const int groups = (ny / 2 + lpb - 1) / lpb;
     const int zi = blockIdx.x / groups;              // interior plane index z-1
     if (zi >= J.n) return;                           // a shorter box of the batch
     const int y0 = (blockIdx.x - zi * groups) * 2 * lpb;
+    const int nl = min(lpb, (ny - y0) / 2);
     EHD_GLOBAL const T* qp = gptr((const T*)J.q) + (size_t)(zi + 1) * nx * ny + (size_t)y0 * nx;
     EHD_GLOBAL cplx<T>* spec = gptr((cplx<T>*)J.spec);
     const double neps = -1.0 / J.eps;
@@ -423,22 +564,25 @@ __global__ void __launch_bounds__(256) fftx_fwd_kernel(const PoissonJob* __restr
                     (T)((double)qp[(size_t)(2 * l + 1) * N + i] * neps)};
         };
         auto sf = [](int, int, cplx<T>) {};
-        ct_run<T, N, 0, 1, false, false>(ld, sf, A, lpb, ldl, tws, -1);
+        ct_run<T, N, 0, 1, false, false>(ld, sf, A, nl, ldl, tws, -1);
         res = A;
     } else {
         cplx<T>* B = A + lpb * ldl;
-        for (int w = threadIdx.x; w < lpb * nx; w += blockDim.x) {
-            const int l = w / nx, i = w - l * nx;
-            A[l * ldl + i] = {(T)((double)qp[(size_t)(2 * l) * nx + i] * neps),
-                              (T)((double)qp[(size_t)(2 * l + 1) * nx + i] * neps)};
-        }
+        rows_copy<4, cplx<T>>(
+            nl * nx, nx, pl.mn,
+            [&](int l, int i) -> cplx<T> {
+                return {(T)((double)qp[(size_t)(2 * l) * nx + i] * neps),
+                        (T)((double)qp[(size_t)(2 * l + 1) * nx + i] * neps)};
+            },
+            [&](int l, int i, cplx<T> v) { A[l * ldl + i] = v; });
         __syncthreads();
-        res = lds_fft<T>(A, B, nx, lpb, ldl, pl, tws, -1);
+        res = rt_fft<T>(A, B, pl, nl, lg, ldl, tws, -1);
     }
-    const int rows = 2 * lpb;
+    const int rows = 2 << lg;
     EHD_GLOBAL cplx<T>* out = spec + (size_t)zi * nxh * ny + y0;
     for (int w = threadIdx.x; w < nxh * rows; w += blockDim.x) {
-        const int k = w / rows, r = w - k * rows;
+        const int k = w >> (lg + 1), r = w & (rows - 1);
+        if (r >= 2 * nl) continue;
         const int l = r >> 1;
         const int kn = (nx - k) % nx;
         const cplx<T> zk = res[l * ldl + (N > 0 ? padi(k) : k)];
@@ -454,7 +598,7 @@ __global__ void __launch_bounds__(256) fftx_fwd_kernel(const PoissonJob* __restr
 // A block takes G consecutive lines.
 template <typename T, int N>
 __global__ void __launch_bounds__(256) ffty_kernel(const PoissonJob* __restrict__ jobs, const cplx<T>* __restrict__ tw,
-                                                   FftPlan pl, int ny_rt, int nxh, int G, int sign)
+                                                   PlanArg<N> pl, int ny_rt, int nxh, int G, int lg, int sign)
 {
     const PoissonJob& J = jobs[blockIdx.y];
     const int ny = N > 0 ? N : ny_rt;
@@ -475,16 +619,14 @@ __global__ void __launch_bounds__(256) ffty_kernel(const PoissonJob* __restrict_
         ct_run<T, N, 0, 1, false, true>(ld, sf, A, nl, ldl, tws, sign);
     } else {
         cplx<T>* B = A + G * ldl;
-        for (int w = threadIdx.x; w < nl * ny; w += blockDim.x) {
-            const int l = w / ny, i = w - l * ny;
-            A[l * ldl + i] = ldc(base + (size_t)l * ny + i);
-        }
+        rows_copy<4, cplx<T>>(
+            nl * ny, ny, pl.mn, [&](int l, int i) { return ldc(base + (size_t)l * ny + i); },
+            [&](int l, int i, cplx<T> v) { A[l * ldl + i] = v; });
         __syncthreads();
-        cplx<T>* res = lds_fft<T>(A, B, ny, nl, ldl, pl, tws, sign);
-        for (int w = threadIdx.x; w < nl * ny; w += blockDim.x) {
-            const int l = w / ny, i = w - l * ny;
-            stc(base + (size_t)l * ny + i, res[l * ldl + i]);
-        }
+        cplx<T>* res = rt_fft<T>(A, B, pl, nl, lg, ldl, tws, sign);
+        rows_copy<4, cplx<T>>(
+            nl * ny, ny, pl.mn, [&](int l, int i) { return res[l * ldl + i]; },
+            [&](int l, int i, cplx<T> v) { stc(base + (size_t)l * ny + i, v); });
     }
 }
 
@@ -743,14 +885,14 @@ __global__ void __launch_bounds__(NT) zsolve_kernel(const PoissonJob* __restrict
 }
 
 // (3b) C2R along x, two real rows per complex line, scaled by 1/(nx*ny), plus
-// the wall potential (F64) or nothing (FP32S fluctuation).  A block takes
-// 2*lpb consecutive rows y0.. of one plane; the transposed spectrum is read
+// the wall potential (F64) or nothing (FP32S fluctuation).  A block takes up
+// to 2*lpb consecutive rows y0.. of one plane; the transposed spectrum is read
 // as (row 2l, row 2l+1) pairs, coalesced along ky, and rebuilt in LDS as
 // Z = A + i B with the Hermitian half.
 template <typename T, int N>
 __global__ void __launch_bounds__(256) fftx_inv_kernel(const PoissonJob* __restrict__ jobs,
-                                                       const cplx<T>* __restrict__ tw, FftPlan pl, int nx_rt,
-                                                       int ny, int lpb, int add_linear)
+                                                       const cplx<T>* __restrict__ tw, PlanArg<N> pl, int nx_rt,
+                                                       int ny, int lpb, int lg, int add_linear)
 {
     const PoissonJob& J = jobs[blockIdx.y];
     const int nx = N > 0 ? N : nx_rt;
@@ -759,10 +901,11 @@ __global__ void __launch_bounds__(256) fftx_inv_kernel(const PoissonJob* __restr
     extern __shared__ unsigned char smem_raw[];
     cplx<T>* tws = reinterpret_cast<cplx<T>*>(smem_raw);
     cplx<T>* A = tws + nx;
-    const int groups = ny / (2 * lpb);
+    const int groups = (ny / 2 + lpb - 1) / lpb;
     const int zi = blockIdx.x / groups;
     if (zi >= J.n) return;                           // a shorter box of the batch
     const int y0 = (blockIdx.x - zi * groups) * 2 * lpb;
+    const int nl = min(lpb, (ny - y0) / 2);
     const int z = zi + 1;
     const int nz = J.n + 2;
     const double voltage = J.voltage;
@@ -772,13 +915,15 @@ __global__ void __launch_bounds__(256) fftx_inv_kernel(const PoissonJob* __restr
     EHD_GLOBAL const cplx<T>* in = spec + (size_t)zi * nxh * ny + y0;
     // XI_LOADS row pairs in flight per thread before the LDS stores
     constexpr int XI_LOADS = 4;
-    for (int w0 = threadIdx.x; w0 < nxh * lpb; w0 += blockDim.x * XI_LOADS) {
+    // lanes beyond a last block's lines fill theirs with copies of its last one
+    const int lanes = 1 << lg;
+    for (int w0 = threadIdx.x; w0 < nxh * lanes; w0 += blockDim.x * XI_LOADS) {
         cplx<T> av[XI_LOADS], bv[XI_LOADS];
 #pragma unroll
         for (int u = 0; u < XI_LOADS; ++u) {
             const int w = w0 + u * blockDim.x;
-            if (w < nxh * lpb) {
-                const int k = w / lpb, l = w - k * lpb;
+            const int k = w >> lg, l = min(w & (lanes - 1), nl - 1);
+            if (w < nxh * lanes) {
                 av[u] = ldc(in + (size_t)k * ny + 2 * l);
                 bv[u] = ldc(in + (size_t)k * ny + 2 * l + 1);
             }
@@ -786,8 +931,8 @@ __global__ void __launch_bounds__(256) fftx_inv_kernel(const PoissonJob* __restr
 #pragma unroll
         for (int u = 0; u < XI_LOADS; ++u) {
             const int w = w0 + u * blockDim.x;
-            if (w < nxh * lpb) {
-                const int k = w / lpb, l = w - k * lpb;
+            const int k = w >> lg, l = w & (lanes - 1);
+            if (w < nxh * lanes) {
                 cplx<T> a = av[u], b = bv[u];
                 if (k == 0 || 2 * k == nx) {
                     a.y = (T)0;
@@ -812,16 +957,16 @@ __global__ void __launch_bounds__(256) fftx_inv_kernel(const PoissonJob* __restr
             row0[(size_t)(2 * l) * N + i] = (T)((double)v.x * inv + lin);
             row0[(size_t)(2 * l + 1) * N + i] = (T)((double)v.y * inv + lin);
         };
-        ct_run<T, N, 0, 1, true, true>(ld, sf, A, lpb, ldl, tws, +1);
+        ct_run<T, N, 0, 1, true, true>(ld, sf, A, nl, ldl, tws, +1);
     } else {
         cplx<T>* B = A + lpb * ldl;
-        cplx<T>* res = lds_fft<T>(A, B, nx, lpb, ldl, pl, tws, +1);
-        for (int w = threadIdx.x; w < lpb * nx; w += blockDim.x) {
-            const int l = w / nx, i = w - l * nx;
-            const cplx<T> v = res[l * ldl + i];
-            row0[(size_t)(2 * l) * nx + i] = (T)((double)v.x * inv + lin);
-            row0[(size_t)(2 * l + 1) * nx + i] = (T)((double)v.y * inv + lin);
-        }
+        cplx<T>* res = rt_fft<T>(A, B, pl, nl, lg, ldl, tws, +1);
+        rows_copy<4, cplx<T>>(
+            nl * nx, nx, pl.mn, [&](int l, int i) { return res[l * ldl + i]; },
+            [&](int l, int i, cplx<T> v) {
+                row0[(size_t)(2 * l) * nx + i] = (T)((double)v.x * inv + lin);
+                row0[(size_t)(2 * l + 1) * nx + i] = (T)((double)v.y * inv + lin);
+            });
     }
 }
 
@@ -838,32 +983,41 @@ __global__ void __launch_bounds__(256) phi_walls_kernel(const PoissonJob* __rest
 
 constexpr size_t kMaxLds = 65536;
 
-// Largest line count per block for an x pass: divides ny/2, one butterfly per
-// thread per stage (compile-time plan), LDS within kMaxLds.
+int pow2_floor(int v)
+{
+    int p = 1;
+    while (2 * p <= v) p *= 2;
+    return p;
+}
+
+// Lines per block of a pass that fit its LDS and, with a compile-time plan,
+// one butterfly per thread and stage; a power of two (the lanes count lines
+// by shifts), at most 16 with a runtime plan.  0: not even one line fits.
+template <typename T, int N>
+int lines_that_fit(int n)
+{
+    const size_t cs = sizeof(cplx<T>);
+    const int ldl = lds_pitch(N, n), bufs = N > 0 ? 1 : 2;
+    int l = N > 0 ? pow2_floor(256 / ct_max_nb(N > 0 ? N : 1)) : 16;
+    while (l > 0 && (size_t)n * cs + (size_t)bufs * l * ldl * cs > kMaxLds) l /= 2;
+    return l;
+}
+
+// Largest line count per block for an x pass: the power of two that holds a
+// plane's ny/2 row pairs cut evenly among as few blocks as fit.
 template <typename T, int N>
 int x_lines_per_block(int nx, int ny)
 {
-    const size_t cs = sizeof(cplx<T>);
-    const int ldl = lds_pitch(N, nx);
-    const int bufs = N > 0 ? 1 : 2;
-    const int cap = N > 0 ? 256 / ct_max_nb(N) : 16;
-    int best = 0;
-    for (int l = 1; l <= ny / 2 && l <= cap; ++l) {
-        if ((ny / 2) % l) continue;
-        if ((size_t)nx * cs + (size_t)bufs * l * ldl * cs <= kMaxLds) best = l;
-    }
-    return best;
+    const int fit = lines_that_fit<T, N>(nx), half = ny / 2;
+    if (fit == 0) return 0;
+    const int groups = (half + fit - 1) / fit, l = (half + groups - 1) / groups;
+    return pow2_floor(2 * l - 1);
 }
 
 template <typename T, int N>
 int y_lines_per_block(int ny)
 {
-    const size_t cs = sizeof(cplx<T>);
-    const int ldl = lds_pitch(N, ny);
-    const int bufs = N > 0 ? 1 : 2;
-    int g = N > 0 ? 256 / ct_max_nb(N) : 16;
-    while (g > 1 && (size_t)ny * cs + (size_t)bufs * g * ldl * cs > kMaxLds) --g;
-    return ((size_t)ny * cs + (size_t)bufs * g * ldl * cs <= kMaxLds) ? g : 0;
+    return lines_that_fit<T, N>(ny);
 }
 
 // z-solve partition: P (16, 8 or 32) threads per mode with chunks of at most
@@ -883,28 +1037,73 @@ int zsolve_partition(int n, size_t cs)
     return 0;
 }
 
+// The passes of a group: each runs the compile-time plan of its own side
+// length where there is one, so a box of unequal sides uses one per side.
+template <typename T, int N>
+hipError_t launch_x(const PoissonGroup& g, bool inverse, hipStream_t st)
+{
+    static_assert(N == 0 || ct_complete(N), "compile-time sizes must factor into powers of two, 3 and 5");
+    const int most = x_lines_per_block<T, N>(g.nx, g.ny);
+    if (most == 0 || g.lpb > most) return hipErrorInvalidValue;
+    const int lpb = pow2_floor(g.lpb > 0 ? g.lpb : most), lg = __builtin_ctz(lpb);
+    const size_t cs = sizeof(cplx<T>);
+    const size_t sh = (size_t)g.nx * cs + (size_t)(N > 0 ? 1 : 2) * lpb * lds_pitch(N, g.nx) * cs;
+    const dim3 grid(g.max_n * ((g.ny / 2 + lpb - 1) / lpb), g.njobs);
+    const PlanArg<N> pl = plan_arg<N>(g.nx);
+    const cplx<T>* tw = (const cplx<T>*)g.twx;
+    if (inverse)
+        fftx_inv_kernel<T, N><<<grid, 256, sh, st>>>(g.jobs, tw, pl, g.nx, g.ny, lpb, lg, g.split_mean ? 0 : 1);
+    else
+        fftx_fwd_kernel<T, N><<<grid, 256, sh, st>>>(g.jobs, tw, pl, g.nx, g.ny, lpb, lg);
+    return hipSuccess;
+}
+
+template <typename T, int N>
+hipError_t launch_y(const PoissonGroup& g, bool inverse, hipStream_t st)
+{
+    const int most = y_lines_per_block<T, N>(g.ny), nxh = g.nx / 2 + 1;
+    int G = g.ylines > 0 ? g.ylines : most;
+    if (most == 0 || G > most) return hipErrorInvalidValue;
+    if (N == 0) G = pow2_floor(G);
+    const size_t cs = sizeof(cplx<T>);
+    const size_t sh = (size_t)g.ny * cs + (size_t)(N > 0 ? 1 : 2) * G * lds_pitch(N, g.ny) * cs;
+    const dim3 grid((g.max_n * nxh + G - 1) / G, g.njobs);
+    ffty_kernel<T, N><<<grid, 256, sh, st>>>(g.jobs, (const cplx<T>*)g.twy, plan_arg<N>(g.ny), g.ny, nxh, G,
+                                            __builtin_ctz(pow2_floor(G)), inverse ? +1 : -1);
+    return hipSuccess;
+}
+
+// f(constant N) with the compile-time plan's length, 0 for a runtime plan
+template <class F>
+auto with_plan(int n, const F& f)
+{
+    switch (n) {
+    case 48: return f(std::integral_constant<int, 48>{});
+    case 64: return f(std::integral_constant<int, 64>{});
+    case 80: return f(std::integral_constant<int, 80>{});
+    case 96: return f(std::integral_constant<int, 96>{});
+    case 128: return f(std::integral_constant<int, 128>{});
+    case 256: return f(std::integral_constant<int, 256>{});
+    case 512: return f(std::integral_constant<int, 512>{});
+    default: return f(std::integral_constant<int, 0>{});
+    }
+}
+
 // One Poisson solve for every job of a group (same nx, ny, precision; the
 // jobs' plane counts may differ): each kernel runs once over the group, the
 // job index in blockIdx.y.
-template <typename T, int NX, int NY>
-hipError_t poisson_group(const PoissonGroup& g, hipStream_t st)
+template <typename T>
+hipError_t poisson_t(const PoissonGroup& g, hipStream_t st)
 {
     const int nx = g.nx, ny = g.ny, nxh = nx / 2 + 1;
     const int nmax = g.max_n;
-    const FftPlan plx = make_fft_plan(nx), ply = make_fft_plan(ny);
     const size_t cs = sizeof(cplx<T>);
-    const int lpb = g.lpb > 0 ? g.lpb : x_lines_per_block<T, NX>(nx, ny);
-    const int G = g.ylines > 0 ? g.ylines : y_lines_per_block<T, NY>(ny);
-    if (lpb == 0 || G == 0 || (ny / 2) % lpb != 0 || lpb > x_lines_per_block<T, NX>(nx, ny) ||
-        G > y_lines_per_block<T, NY>(ny))
-        return hipErrorInvalidValue;
-    const size_t shx = (size_t)nx * cs + (size_t)(NX > 0 ? 1 : 2) * lpb * lds_pitch(NX, nx) * cs;
-    const size_t shy = (size_t)ny * cs + (size_t)(NY > 0 ? 1 : 2) * G * lds_pitch(NY, ny) * cs;
-    const dim3 gx(nmax * (ny / (2 * lpb)), g.njobs);
-    const dim3 gy((nmax * nxh + G - 1) / G, g.njobs);
-    const cplx<T>* twx = (const cplx<T>*)g.twx;
-    const cplx<T>* twy = (const cplx<T>*)g.twy;
-
+    auto x_pass = [&](bool inverse) {
+        return with_plan(nx, [&](auto n) { return launch_x<T, decltype(n)::value>(g, inverse, st); });
+    };
+    auto y_pass = [&](bool inverse) {
+        return with_plan(ny, [&](auto n) { return launch_y<T, decltype(n)::value>(g, inverse, st); });
+    };
     // debug_sync: each pass synchronised and checked on its own
     auto check = [&](const char* pass) -> hipError_t {
         if (!g.debug_sync) return hipSuccess;
@@ -914,9 +1113,9 @@ hipError_t poisson_group(const PoissonGroup& g, hipStream_t st)
         return e;
     };
     hipError_t ec;
-    fftx_fwd_kernel<T, NX><<<gx, 256, shx, st>>>(g.jobs, twx, plx, nx, ny, lpb);
+    if ((ec = x_pass(false)) != hipSuccess) return ec;
     if ((ec = check("forward x transform")) != hipSuccess) return ec;
-    ffty_kernel<T, NY><<<gy, 256, shy, st>>>(g.jobs, twy, ply, ny, nxh, G, -1);
+    if ((ec = y_pass(false)) != hipSuccess) return ec;
     if ((ec = check("forward y transform")) != hipSuccess) return ec;
 
     const int nmodes = nxh * ny;
@@ -946,9 +1145,9 @@ hipError_t poisson_group(const PoissonGroup& g, hipStream_t st)
     if (ez != hipSuccess) return ez;
     if ((ec = check("z solve")) != hipSuccess) return ec;
 
-    ffty_kernel<T, NY><<<gy, 256, shy, st>>>(g.jobs, twy, ply, ny, nxh, G, +1);
+    if ((ec = y_pass(true)) != hipSuccess) return ec;
     if ((ec = check("inverse y transform")) != hipSuccess) return ec;
-    fftx_inv_kernel<T, NX><<<gx, 256, shx, st>>>(g.jobs, twx, plx, nx, ny, lpb, sm ? 0 : 1);
+    if ((ec = x_pass(true)) != hipSuccess) return ec;
     if ((ec = check("inverse x transform")) != hipSuccess) return ec;
     if (!sm) {
         phi_walls_kernel<<<dim3((nx * ny + 255) / 256, g.njobs), 256, 0, st>>>(g.jobs, nx * ny);
@@ -957,60 +1156,16 @@ hipError_t poisson_group(const PoissonGroup& g, hipStream_t st)
     return hipGetLastError();
 }
 
-// Compile-time FFT sizes for the grids of the configurations; anything else
-// takes the runtime-planned path.
-template <typename T, int NX>
-hipError_t poisson_ny(const PoissonGroup& g, hipStream_t st)
-{
-    static_assert(ct_complete(NX), "compile-time sizes must factor into powers of two, 3 and 5");
-    if (g.ny == NX) return poisson_group<T, NX, NX>(g, st);
-    return poisson_group<T, NX, 0>(g, st);
-}
-
-template <typename T>
-hipError_t poisson_t(const PoissonGroup& g, hipStream_t st)
-{
-    switch (g.nx) {
-    case 48: return poisson_ny<T, 48>(g, st);
-    case 64: return poisson_ny<T, 64>(g, st);
-    case 80: return poisson_ny<T, 80>(g, st);
-    case 96: return poisson_ny<T, 96>(g, st);
-    case 128: return poisson_ny<T, 128>(g, st);
-    case 256: return poisson_ny<T, 256>(g, st);
-    case 512: return poisson_ny<T, 512>(g, st);
-    default: return poisson_group<T, 0, 0>(g, st);
-    }
-}
-
 template <typename T>
 int max_x_lines(int nx, int ny)
 {
-    switch (nx) {
-    case 48: return x_lines_per_block<T, 48>(nx, ny);
-    case 64: return x_lines_per_block<T, 64>(nx, ny);
-    case 80: return x_lines_per_block<T, 80>(nx, ny);
-    case 96: return x_lines_per_block<T, 96>(nx, ny);
-    case 128: return x_lines_per_block<T, 128>(nx, ny);
-    case 256: return x_lines_per_block<T, 256>(nx, ny);
-    case 512: return x_lines_per_block<T, 512>(nx, ny);
-    default: return x_lines_per_block<T, 0>(nx, ny);
-    }
+    return with_plan(nx, [&](auto n) { return x_lines_per_block<T, decltype(n)::value>(nx, ny); });
 }
 
 template <typename T>
-int max_y_lines(int nx, int ny)
+int max_y_lines(int ny)
 {
-    if (ny != nx) return y_lines_per_block<T, 0>(ny);
-    switch (ny) {
-    case 48: return y_lines_per_block<T, 48>(ny);
-    case 64: return y_lines_per_block<T, 64>(ny);
-    case 80: return y_lines_per_block<T, 80>(ny);
-    case 96: return y_lines_per_block<T, 96>(ny);
-    case 128: return y_lines_per_block<T, 128>(ny);
-    case 256: return y_lines_per_block<T, 256>(ny);
-    case 512: return y_lines_per_block<T, 512>(ny);
-    default: return y_lines_per_block<T, 0>(ny);
-    }
+    return with_plan(ny, [&](auto n) { return y_lines_per_block<T, decltype(n)::value>(ny); });
 }
 
 }  // namespace
@@ -1037,7 +1192,7 @@ PoissonShape poisson_shape(Prec prec, int nx, int ny, int nz)
     PoissonShape s{};
     const bool f64 = prec == Prec::F64;
     s.max_x_lines = f64 ? max_x_lines<double>(nx, ny) : max_x_lines<float>(nx, ny);
-    s.max_y_lines = f64 ? max_y_lines<double>(nx, ny) : max_y_lines<float>(nx, ny);
+    s.max_y_lines = f64 ? max_y_lines<double>(ny) : max_y_lines<float>(ny);
     s.zs_partition = zsolve_partition(nz - 2, f64 ? 16 : 8);
     return s;
 }

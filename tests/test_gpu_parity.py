@@ -245,6 +245,16 @@ def test_poisson_vs_oracle(shape, precision):
     assert err < tol
 
 
+# The runtime-planned transforms: each radix (2..5, 7, 9, 11, 13, 16), a prime
+# stage alone, first and second (17, 61, 17 * 19), one side planned at compile
+# time and the other not, a last block of rows that is not full, one row pair.
+@pytest.mark.parametrize("shape", [(122, 122, 9), (34, 4, 6), (646, 2, 5), (64, 34, 7), (90, 154, 6), (18, 26, 11),
+                                   (22, 98, 8), (112, 48, 5), (2, 14, 12), (200, 36, 6)])
+@pytest.mark.parametrize("precision", [E.FP64, E.FP32S])
+def test_poisson_runtime_plans_vs_oracle(shape, precision):
+    test_poisson_vs_oracle(shape, precision)
+
+
 def test_diagnostics_current_vs_oracle():
     ob = oracle_box(16, 12, 10)
     ob.init_equilibrium()
