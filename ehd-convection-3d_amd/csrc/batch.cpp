@@ -51,6 +51,7 @@ struct ehd_batch {
     void* ditems[2] = {nullptr, nullptr};
     unsigned total_tiles = 0;
     unsigned lbm_grid = 0;
+    bool lbm_stream = false;  // streaming population accesses, by the whole batch's size
     unsigned lbm_chunk = 0;   // XCD tile order of the LBM launch (0: linear)
     double lbm_ms = 0.0;
     std::vector<Group> groups;
@@ -74,10 +75,10 @@ int batch_lbm(ehd_batch* bt, int cur, bool first, bool ebuf, bool macro)
 {
     if (bt->prec == Prec::F32S) {
         HIPCHK(launch_lbm_f32s_batch(bt->ditems[cur], (int)bt->boxes.size(), bt->total_tiles, bt->lbm_grid,
-                                     bt->lbm_chunk, first, ebuf, macro, bt->st));
+                                     bt->lbm_chunk, first, ebuf, macro, bt->lbm_stream, bt->st));
     } else {
         for (ehd_box* b : bt->boxes)
-            HIPCHK(launch_lbm_f64(b->lp, pop_bufs_at(b, cur), macro_bufs(b), first, ebuf, macro, bt->st));
+            HIPCHK(launch_lbm_f64(b->lp, pop_bufs_at(b, cur), macro_bufs(b), first, ebuf, macro, bt->lbm_stream, bt->st));
     }
     return EHD_OK;
 }
@@ -132,11 +133,11 @@ int chain_step(ehd_batch* bt, int cur, bool first, bool ebuf, bool macro)
         const hipStream_t s = group_stream(bt, gr);
         if (bt->prec == Prec::F32S) {
             HIPCHK(launch_lbm_f32s_batch(gr.items[cur], (int)gr.members.size(), gr.tiles, 0, gr.chunk, first, ebuf,
-                                         macro, s));
+                                         macro, bt->lbm_stream, s));
         } else {
             for (int m : gr.members) {
                 ehd_box* b = bt->boxes[m];
-                HIPCHK(launch_lbm_f64(b->lp, pop_bufs_at(b, cur), macro_bufs(b), first, ebuf, macro, s));
+                HIPCHK(launch_lbm_f64(b->lp, pop_bufs_at(b, cur), macro_bufs(b), first, ebuf, macro, bt->lbm_stream, s));
             }
         }
         HIPCHK(launch_poisson_group(bt->prec, gr.g, s));
@@ -378,6 +379,15 @@ int ehd_batch_create(const ehd_params* params, int nboxes, int flags, ehd_batch*
         if (rc) return bail(rc);
         bt->boxes.push_back(b);
     }
+    // a batch steps all its boxes before it comes back to one, so its own size
+    // counts; one launch, so the rows that most of its nodes lie in decide
+    {
+        size_t nodes = 0, streamed = 0;
+        for (const ehd_box* b : bt->boxes) nodes += b->S;
+        for (const ehd_box* b : bt->boxes)
+            if (lbm_streams(b->prec, b->nx, nodes)) streamed += b->S;
+        bt->lbm_stream = 2 * streamed > nodes;
+    }
     // Poisson groups by (nx, ny); the z-solve partition follows n, so boxes of
     // one (nx, ny) whose plane counts need different partitions get separate groups
     for (int i = 0; i < nboxes; ++i) {
@@ -597,7 +607,7 @@ int ehd_batch_init_consistent(ehd_batch* bt, const double* const* fields9, int i
         for (int k = 0; k < 2; ++k)
             if (sets[k].n > 0)
                 HIPCHK(launch_lbm_f32s_batch(sets[k].items[cur], sets[k].n, sets[k].tiles, 0, bt->lbm_chunk, direct,
-                                             ebuf, macro, bt->st, k == 1));
+                                             ebuf, macro, bt->lbm_stream, bt->st, k == 1));
         if ((rc = batch_poisson(bt))) return rc;
         cur = 1 - cur;
         direct = false;

@@ -48,6 +48,7 @@ struct ehd_box {
     ehd::PoissonJob pjob_h{};          // host copy (batches build their tables from it)
     void* lbm_items[2] = {nullptr, nullptr};   // FP32S: one-item kernel tables per buffer parity
     unsigned lbm_chunk = 0;              // FP32S LBM XCD tile order (lbm_xcd_chunk)
+    bool lbm_stream = false;             // streaming population accesses (lbm_streams)
     int tune_lpb = 0, tune_ylines = 0;   // Poisson lines per block (0: largest that fits)
     bool debug_sync = false;   // synchronise and check after every launch (ehd_set_debug_sync)
     long long step = 0;

@@ -175,10 +175,11 @@ int run_lbm(ehd_box* b, bool macro, void* const* target_items)
         HIPCHK(hipEventRecord(e0, b->st));
     }
     hipError_t e;
-    if (b->prec == Prec::F64) e = launch_lbm_f64(b->lp, pop_bufs(b), macro_bufs(b), b->direct, b->ebuf, macro, b->st);
+    if (b->prec == Prec::F64) e = launch_lbm_f64(b->lp, pop_bufs(b), macro_bufs(b), b->direct, b->ebuf, macro,
+                                                     b->lbm_stream, b->st);
     else e = launch_lbm_f32s_batch(target_items ? target_items[b->cur] : b->lbm_items[b->cur], 1,
-                                   (unsigned)((b->S + 255) / 256), 0, b->lbm_chunk, b->direct, b->ebuf, macro, b->st,
-                                   target_items != nullptr);
+                                   (unsigned)((b->S + 255) / 256), 0, b->lbm_chunk, b->direct, b->ebuf, macro,
+                                   b->lbm_stream, b->st, target_items != nullptr);
     if (e != hipSuccess) return set_error(EHD_EHIP, "LBM launch failed: %s", hipGetErrorString(e));
     if (b->debug_sync) {
         e = hipStreamSynchronize(b->st);
@@ -474,6 +475,7 @@ int ehd_create(const ehd_params* p, ehd_box** out)
     b->S = b->nxy * p->nz;
     b->esz = (b->prec == Prec::F64) ? 8 : 4;
     fill_lbm_params(b);
+    b->lbm_stream = lbm_streams(b->prec, b->nx, b->S);
 
     auto bail = [&](int code) {
         free_box(b);

@@ -53,7 +53,10 @@ struct MacroBufs {
 };
 
 hipError_t launch_lbm_f64(const LbmParams& P, const PopBufs& pb, const MacroBufs& mb,
-                          bool first, bool ebuf, bool macro, hipStream_t st);
+                          bool first, bool ebuf, bool macro, bool stream, hipStream_t st);
+// Whether the LBM launches of a box, or of a batch of nodes in all, stream
+// the populations past the caches (rows of nx; the first step never does).
+bool lbm_streams(Prec prec, int nx, size_t nodes);
 // FP32S LBM over one box or a batch of boxes: an opaque item per box (lbm_f32s_batch_item writes
 // lbm_f32s_batch_item_size() bytes), items in a device array sorted by tile0,
 // tile0 = number of 256-node tiles of the boxes before it.  grid = 0 launches
@@ -66,7 +69,8 @@ size_t lbm_f32s_batch_item_size();
 void lbm_f32s_batch_item(void* out, const LbmParams& P, const PopBufs& pb, const MacroBufs& mb, unsigned tile0,
                          const double* target = nullptr);
 hipError_t launch_lbm_f32s_batch(const void* items, int nitems, unsigned total_tiles, unsigned grid, unsigned chunk,
-                                 bool first, bool ebuf, bool macro, hipStream_t st, bool target = false);
+                                 bool first, bool ebuf, bool macro, bool stream, hipStream_t st,
+                                 bool target = false);
 // XCD tile-order chunk for boxes of nxy nodes per plane: one plane per
 // superblock when a plane is a whole number of 8-tile groups, else 0.
 unsigned lbm_xcd_chunk(unsigned nxy);

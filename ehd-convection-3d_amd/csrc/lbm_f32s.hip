@@ -78,11 +78,21 @@ __device__ __forceinline__ float pulled(float v, int d, float w, float dup, floa
     return v;
 }
 
-// Every population is read once and written once per step: streaming
-// (non-temporal) loads and stores keep them from displacing the potential
-// and the shift tables in the caches.
-__device__ __forceinline__ float ldnt(cgfloat* p) { return __builtin_nontemporal_load(p); }
-__device__ __forceinline__ void stnt(float v, gfloat* p) { __builtin_nontemporal_store(v, p); }
+// Streaming (nontemporal) loads and stores of the moving populations (NT, see
+// lbm_streams): read once and written once per step, a state beyond the
+// last-level cache displaces the potential and the shift tables for nothing.
+template <bool NT>
+__device__ __forceinline__ float ldnt(cgfloat* p)
+{
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+template <bool NT>
+__device__ __forceinline__ void stnt(float v, gfloat* p)
+{
+    if constexpr (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
 
 // One node s of one box: pull, collide, boundary and injection.
 //
@@ -93,7 +103,7 @@ __device__ __forceinline__ void stnt(float v, gfloat* p) { __builtin_nontemporal
 // target charge, and the target charge is what the Poisson solve sees.
 // Iterated, this builds the non-equilibrium parts of the populations that
 // belong to the target state; the equilibrium start alone lacks them.
-template <bool FIRST, bool EBUF, bool TARGET>
+template <bool FIRST, bool EBUF, bool TARGET, bool NT>
 __device__ __forceinline__ void lbm_f32s_node(const LbmParams& P, const F32Consts& c, const PopBufs& pb,
                                               const MacroBufs& mb, const double* tgp, int macro, unsigned s)
 {
@@ -130,7 +140,7 @@ __device__ __forceinline__ void lbm_f32s_node(const LbmParams& P, const F32Const
     } else {
 #pragma unroll
         for (int d = 1; d < 27; ++d)
-            g[d] = pulled(ldnt(fA + (ZR[1 - CZ[d]] + YR[1 - CY[d]]) * RW + (d - 1) * nx + XS[1 - CX[d]]), d,
+            g[d] = pulled(ldnt<NT>(fA + (ZR[1 - CZ[d]] + YR[1 - CY[d]]) * RW + (d - 1) * nx + XS[1 - CX[d]]), d,
                           c.w[WCLS[d]], dRu, dRd);
         if (z == 0) {
             k[0] = -h0A[s] + c.injk[0];
@@ -140,7 +150,7 @@ __device__ __forceinline__ void lbm_f32s_node(const LbmParams& P, const F32Const
             k[0] = h0A[s];
 #pragma unroll
             for (int d = 1; d < 27; ++d)
-                k[d] = pulled(ldnt(hA + (ZR[1 - CZ[d]] + YR[1 - CY[d]]) * RW + (d - 1) * nx + XS[1 - CX[d]]), d,
+                k[d] = pulled(ldnt<NT>(hA + (ZR[1 - CZ[d]] + YR[1 - CY[d]]) * RW + (d - 1) * nx + XS[1 - CX[d]]), d,
                               c.w[WCLS[d]], dQu, dQd);
         }
     }
@@ -322,14 +332,14 @@ __device__ __forceinline__ void lbm_f32s_node(const LbmParams& P, const F32Const
             od = gd;
             oe = ge;
         }
-        stnt(od, fB + own + (d - 1) * nx);
-        stnt(oe, fB + own + (e - 1) * nx);
+        stnt<NT>(od, fB + own + (d - 1) * nx);
+        stnt<NT>(oe, fB + own + (e - 1) * nx);
         if (z != nz - 1) {
-            stnt(kd, hB + own + (d - 1) * nx);
-            stnt(ke, hB + own + (e - 1) * nx);
+            stnt<NT>(kd, hB + own + (d - 1) * nx);
+            stnt<NT>(ke, hB + own + (e - 1) * nx);
             if (z == nz - 2) {
-                stnt(kd, hB + own + ny * RW + (d - 1) * nx);
-                stnt(ke, hB + own + ny * RW + (e - 1) * nx);
+                stnt<NT>(kd, hB + own + ny * RW + (d - 1) * nx);
+                stnt<NT>(ke, hB + own + ny * RW + (e - 1) * nx);
             }
         }
     }
@@ -359,7 +369,7 @@ struct BatchItem {
     unsigned tile0, ntiles;
 };
 
-template <bool FIRST, bool EBUF, bool TARGET>
+template <bool FIRST, bool EBUF, bool TARGET, bool NT>
 __global__ void __launch_bounds__(256) lbm_f32s_kernel(const BatchItem* __restrict__ items, int nitems,
                                                              unsigned total_tiles, unsigned chunk, int macro)
 {
@@ -379,7 +389,7 @@ __global__ void __launch_bounds__(256) lbm_f32s_kernel(const BatchItem* __restri
         }
         const BatchItem& it = items[lo];
         const unsigned s = (tile - it.tile0) * 256u + threadIdx.x;
-        if (s < it.P.S) lbm_f32s_node<FIRST, EBUF, TARGET>(it.P, it.c, it.pb, it.mb, TARGET ? it.target : nullptr,
+        if (s < it.P.S) lbm_f32s_node<FIRST, EBUF, TARGET, NT>(it.P, it.c, it.pb, it.mb, TARGET ? it.target : nullptr,
                                                            macro, s);
     }
 }
@@ -443,24 +453,25 @@ void lbm_f32s_batch_item(void* out, const LbmParams& P, const PopBufs& pb, const
 
 template <bool TARGET>
 static void launch_variant(const BatchItem* it, int nitems, unsigned total_tiles, unsigned g, unsigned chunk, bool first,
-                    bool ebuf, int m, hipStream_t st)
+                           bool ebuf, int m, bool stream, hipStream_t st)
 {
-    if (first && ebuf) lbm_f32s_kernel<true, true, TARGET><<<g, 256, 0, st>>>(it, nitems, total_tiles, chunk, m);
-    else if (first) lbm_f32s_kernel<true, false, TARGET><<<g, 256, 0, st>>>(it, nitems, total_tiles, chunk, m);
-    else if (ebuf) lbm_f32s_kernel<false, true, TARGET><<<g, 256, 0, st>>>(it, nitems, total_tiles, chunk, m);
-    else lbm_f32s_kernel<false, false, TARGET><<<g, 256, 0, st>>>(it, nitems, total_tiles, chunk, m);
+    if (first && ebuf) lbm_f32s_kernel<true, true, TARGET, false><<<g, 256, 0, st>>>(it, nitems, total_tiles, chunk, m);
+    else if (first) lbm_f32s_kernel<true, false, TARGET, false><<<g, 256, 0, st>>>(it, nitems, total_tiles, chunk, m);
+    else if (ebuf) lbm_f32s_kernel<false, true, TARGET, false><<<g, 256, 0, st>>>(it, nitems, total_tiles, chunk, m);
+    else if (stream) lbm_f32s_kernel<false, false, TARGET, true><<<g, 256, 0, st>>>(it, nitems, total_tiles, chunk, m);
+    else lbm_f32s_kernel<false, false, TARGET, false><<<g, 256, 0, st>>>(it, nitems, total_tiles, chunk, m);
 }
 
 hipError_t launch_lbm_f32s_batch(const void* items, int nitems, unsigned total_tiles, unsigned grid, unsigned chunk,
-                                 bool first, bool ebuf, bool macro, hipStream_t st, bool target)
+                                 bool first, bool ebuf, bool macro, bool stream, hipStream_t st, bool target)
 {
     if (nitems < 1 || total_tiles == 0) return hipErrorInvalidValue;
     const BatchItem* it = (const BatchItem*)items;
     const unsigned g = (grid == 0 || grid > total_tiles) ? total_tiles : grid;
     if (g < total_tiles && g % 8u) return hipErrorInvalidValue;   // the tile order assumes b mod 8 = XCD
     const int m = macro ? 1 : 0;
-    if (target) launch_variant<true>(it, nitems, total_tiles, g, chunk, first, ebuf, m, st);
-    else launch_variant<false>(it, nitems, total_tiles, g, chunk, first, ebuf, m, st);
+    if (target) launch_variant<true>(it, nitems, total_tiles, g, chunk, first, ebuf, m, stream, st);
+    else launch_variant<false>(it, nitems, total_tiles, g, chunk, first, ebuf, m, stream, st);
     return hipGetLastError();
 }
 

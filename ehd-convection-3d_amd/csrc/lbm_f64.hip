@@ -99,11 +99,14 @@ __device__ __forceinline__ double fpop_dir(int d, const double* u, const double*
 }
 
 // TRT relaxation of one node (LBM.cu:519-1089): equilibria, force
-// populations, +/- splits, sources, relaxation.
+// populations, +/- splits, sources, relaxation.  The results leave as they are
+// formed, rest(f, h) and then pair(d, f_d, f_d+1, h_d, h_d+1), so that no set
+// of 27 results is ever held beside the 54 inputs.
+template <class Rest, class Pair>
 __device__ __forceinline__ void relax_f64(const LbmParams& P, const double* ft, const double* ht,
                                           double rho, double charge, double ux, double uy, double uz,
                                           double Ex, double Ey, double Ez, double forcex, double forcey,
-                                          double forcez, double* fo, double* ho)
+                                          double forcez, const Rest& rest, const Pair& pair)
 {
     const double cs_square = P.cs_square, CFL = P.cfl, K = P.K, dt = P.dt;
     const double wr[4] = {P.w[0] * rho, P.w[1] * rho, P.w[2] * rho, P.w[3] * rho};
@@ -138,8 +141,8 @@ __device__ __forceinline__ void relax_f64(const LbmParams& P, const double* ft, 
         const double fpop0 = -coe[0] * (ux * forcex + uy * forcey + uz * forcez);
         const double zero = 0.0;
         const double source0 = sp * fpop0;
-        fo[0] = ft[0] - (tw0rp * (ft[0] - fe0) + tw0rm * (zero - zero)) + dt * source0;
-        ho[0] = ht[0] - (tw0cp * (ht[0] - he0) + tw0cm * (zero - zero));
+        rest(ft[0] - (tw0rp * (ft[0] - fe0) + tw0rm * (zero - zero)) + dt * source0,
+             ht[0] - (tw0cp * (ht[0] - he0) + tw0cm * (zero - zero)));
     }
 #pragma unroll
     for (int d = 1; d < 27; d += 2) {
@@ -167,17 +170,31 @@ __device__ __forceinline__ void relax_f64(const LbmParams& P, const double* ft, 
         const double fm_e = -fm, fem_e = -fem, hm_e = -hm, hem_e = -hem, forcem_e = -forcem;
         const double source_d = sp * forcep + sm * forcem;
         const double source_e = sp * forcep + sm * forcem_e;
-        fo[d] = ft[d] - (tw0rp * (fp - fep) + tw0rm * (fm - fem)) + dt * source_d;
-        ho[d] = ht[d] - (tw0cp * (hp - hep) + tw0cm * (hm - hem));
-        fo[e] = ft[e] - (tw0rp * (fp - fep) + tw0rm * (fm_e - fem_e)) + dt * source_e;
-        ho[e] = ht[e] - (tw0cp * (hp - hep) + tw0cm * (hm_e - hem_e));
+        const double fod = ft[d] - (tw0rp * (fp - fep) + tw0rm * (fm - fem)) + dt * source_d;
+        const double hod = ht[d] - (tw0cp * (hp - hep) + tw0cm * (hm - hem));
+        const double foe = ft[e] - (tw0rp * (fp - fep) + tw0rm * (fm_e - fem_e)) + dt * source_e;
+        const double hoe = ht[e] - (tw0cp * (hp - hep) + tw0cm * (hm_e - hem_e));
+        pair(d, fod, foe, hod, hoe);
     }
 }
 
+// Streaming (nontemporal) stores of the moving populations (NT, see
+// lbm_streams): a state beyond the last-level cache is not read again before
+// it has left it, and whole cache lines need no merging there.
+// 256x256x128: 1390 us plain, 1343 us with streaming stores, 1350 us with
+// streaming loads as well.
+template <bool NT>
+__device__ __forceinline__ void stnt(double v, double* p)
+{
+    if constexpr (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+
 // Two waves per SIMD: left to itself the compiler gives the steady-state
-// variant 256 VGPRs + 4 AGPRs, one wave per SIMD; capped it keeps 256 VGPRs
-// and spills 5 dwords per lane to scratch.
-template <bool FIRST, bool EBUF>
+// variants 256 VGPRs + AGPRs, one wave per SIMD; capped they keep 256 VGPRs
+// and spill 3 to 5 dwords per lane to scratch (three waves would leave 168 VGPRs
+// and spill 84 bytes: 1345 -> 1572 us).
+template <bool FIRST, bool EBUF, bool NT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 lbm_f64_kernel(LbmParams P, PopBufs pb, MacroBufs mb, int macro)
 {
@@ -188,11 +205,11 @@ lbm_f64_kernel(LbmParams P, PopBufs pb, MacroBufs mb, int macro)
     const unsigned xm = (x == 0) ? nx - 1 : x - 1, xp = (x == nx - 1) ? 0 : x + 1;
     const unsigned ym = (y == 0) ? ny - 1 : y - 1, yp = (y == ny - 1) ? 0 : y + 1;
     const unsigned zm = (z == 0) ? nz - 1 : z - 1, zp = (z == nz - 1) ? 0 : z + 1;
-    const unsigned XS[3] = {xm, x, xp};
     // populations in row blocks [z][y][d-1][x]; a pull along c reads row (y - c_y, z - c_z)
     const unsigned RW = 26u * nx;
-    const unsigned YR[3] = {ym, y, yp}, ZR[3] = {zm * ny, z * ny, zp * ny};
+    const unsigned YR[3] = {ym, y, yp}, ZR[3] = {zm * ny, z * ny, zp * ny}, XS[3] = {xm, x, xp};
     const unsigned own = t * RW + x;
+    auto pulled = [&](int d) { return (ZR[1 - CZ[d]] + YR[1 - CY[d]]) * RW + (d - 1) * nx + XS[1 - CX[d]]; };
 
     const double* __restrict__ fA = (const double*)pb.f;
     const double* __restrict__ f0A = (const double*)pb.f0;
@@ -211,7 +228,7 @@ lbm_f64_kernel(LbmParams P, PopBufs pb, MacroBufs mb, int macro)
     } else {
 #pragma unroll
         for (int d = 1; d < 27; ++d)
-            ft[d] = fA[(ZR[1 - CZ[d]] + YR[1 - CY[d]]) * RW + (d - 1) * nx + XS[1 - CX[d]]];
+            ft[d] = fA[pulled(d)];
         if (z == 0) {
             ht[0] = -h0A[s] + P.inj[0];
 #pragma unroll
@@ -220,7 +237,7 @@ lbm_f64_kernel(LbmParams P, PopBufs pb, MacroBufs mb, int macro)
             ht[0] = h0A[s];
 #pragma unroll
             for (int d = 1; d < 27; ++d)
-                ht[d] = hA[(ZR[1 - CZ[d]] + YR[1 - CY[d]]) * RW + (d - 1) * nx + XS[1 - CX[d]]];
+                ht[d] = hA[pulled(d)];
         }
     }
 
@@ -297,39 +314,89 @@ lbm_f64_kernel(LbmParams P, PopBufs pb, MacroBufs mb, int macro)
     }
     ((double*)mb.q)[s] = charge;
 
-    double fo[27], ho[27];
-    relax_f64(P, ft, ht, rho, charge, ux, uy, uz, Ex, Ey, Ez, forcex, forcey, forcez, fo, ho);
-
     double* __restrict__ fB = (double*)pb.fo;
     double* __restrict__ f0B = (double*)pb.f0o;
     double* __restrict__ hB = (double*)pb.ho;
     double* __restrict__ h0B = (double*)pb.h0o;
-    if (z == 0) {
-        f0B[s] = ft[0];
-#pragma unroll
-        for (int d = 1; d < 27; ++d) fB[own + (d - 1) * nx] = ft[opp(d)];
-    } else if (z == nz - 1) {
-        f0B[s] = ft[0];
-#pragma unroll
-        for (int d = 1; d < 27; ++d) {
-            double v = ft[opp(d)];
-            if (TOPSGN[d] > 0) v = v + P.multi[WCLS[d]];
-            else if (TOPSGN[d] < 0) v = v - P.multi[WCLS[d]];
-            fB[own + (d - 1) * nx] = v;
+    const bool bottom = z == 0, top = z == nz - 1, copy = z == nz - 2;
+    auto store_rest = [&](double f, double h) {
+        f0B[s] = bottom || top ? ft[0] : f;
+        if (!top) h0B[s] = h;
+        if (copy) h0B[s + nxy] = h;
+    };
+    auto store_pair = [&](int d, double fd, double fe, double hd, double he) {
+        // walls: the pre-collision values bounced back, the moving top's term added
+        if (bottom || top) {
+            fd = ft[d + 1];
+            fe = ft[d];
+            if (top) {
+                const double m = P.multi[WCLS[d]];
+                if (TOPSGN[d] > 0) fd = fd + m;
+                else if (TOPSGN[d] < 0) fd = fd - m;
+                if (TOPSGN[d + 1] > 0) fe = fe + m;
+                else if (TOPSGN[d + 1] < 0) fe = fe - m;
+            }
         }
+        const unsigned od = own + (d - 1) * nx, oe = od + nx;
+        stnt<NT>(fd, fB + od);
+        stnt<NT>(fe, fB + oe);
+        if (!top) {
+            stnt<NT>(hd, hB + od);
+            stnt<NT>(he, hB + oe);
+        }
+        if (copy) {
+            stnt<NT>(hd, hB + (od + ny * RW));
+            stnt<NT>(he, hB + (oe + ny * RW));
+        }
+    };
+    // A large state leaves pair by pair as it is formed, the stores spread over
+    // the arithmetic.  A small one is bound by the length of a wave, which the
+    // wall tests of every pair add to: all results first, then the stores
+    // (pair by pair / so: 32x32x16 12.9 / 11.3 us, 64x64x32 21.9 / 20.4 us,
+    // equal from 64x64x64 on).
+    if constexpr (NT) {
+        relax_f64(P, ft, ht, rho, charge, ux, uy, uz, Ex, Ey, Ez, forcex, forcey, forcez, store_rest, store_pair);
     } else {
-        f0B[s] = fo[0];
+        double fo[27], ho[27];
+        relax_f64(
+            P, ft, ht, rho, charge, ux, uy, uz, Ex, Ey, Ez, forcex, forcey, forcez,
+            [&](double f, double h) {
+                fo[0] = f;
+                ho[0] = h;
+            },
+            [&](int d, double fd, double fe, double hd, double he) {
+                fo[d] = fd;
+                fo[d + 1] = fe;
+                ho[d] = hd;
+                ho[d + 1] = he;
+            });
+        if (bottom) {
+            f0B[s] = ft[0];
 #pragma unroll
-        for (int d = 1; d < 27; ++d) fB[own + (d - 1) * nx] = fo[d];
-    }
-    if (z != nz - 1) {
-        h0B[s] = ho[0];
+            for (int d = 1; d < 27; ++d) fB[own + (d - 1) * nx] = ft[opp(d)];
+        } else if (top) {
+            f0B[s] = ft[0];
 #pragma unroll
-        for (int d = 1; d < 27; ++d) hB[own + (d - 1) * nx] = ho[d];
-        if (z == nz - 2) {
-            h0B[s + nxy] = ho[0];
+            for (int d = 1; d < 27; ++d) {
+                double v = ft[opp(d)];
+                if (TOPSGN[d] > 0) v = v + P.multi[WCLS[d]];
+                else if (TOPSGN[d] < 0) v = v - P.multi[WCLS[d]];
+                fB[own + (d - 1) * nx] = v;
+            }
+        } else {
+            f0B[s] = fo[0];
 #pragma unroll
-            for (int d = 1; d < 27; ++d) hB[own + ny * RW + (d - 1) * nx] = ho[d];
+            for (int d = 1; d < 27; ++d) fB[own + (d - 1) * nx] = fo[d];
+        }
+        if (!top) {
+            h0B[s] = ho[0];
+#pragma unroll
+            for (int d = 1; d < 27; ++d) hB[own + (d - 1) * nx] = ho[d];
+            if (copy) {
+                h0B[s + nxy] = ho[0];
+#pragma unroll
+                for (int d = 1; d < 27; ++d) hB[own + ny * RW + (d - 1) * nx] = ho[d];
+            }
         }
     }
 }
@@ -446,15 +513,32 @@ inline dim3 grid_for(unsigned n) { return dim3((n + 255) / 256); }
 }  // namespace
 
 hipError_t launch_lbm_f64(const LbmParams& P, const PopBufs& pb, const MacroBufs& mb, bool first,
-                          bool ebuf, bool macro, hipStream_t st)
+                          bool ebuf, bool macro, bool stream, hipStream_t st)
 {
     dim3 g = grid_for(P.S), b(256);
     int m = macro ? 1 : 0;
-    if (first && ebuf) lbm_f64_kernel<true, true><<<g, b, 0, st>>>(P, pb, mb, m);
-    else if (first) lbm_f64_kernel<true, false><<<g, b, 0, st>>>(P, pb, mb, m);
-    else if (ebuf) lbm_f64_kernel<false, true><<<g, b, 0, st>>>(P, pb, mb, m);
-    else lbm_f64_kernel<false, false><<<g, b, 0, st>>>(P, pb, mb, m);
+    if (first && ebuf) lbm_f64_kernel<true, true, false><<<g, b, 0, st>>>(P, pb, mb, m);
+    else if (first) lbm_f64_kernel<true, false, false><<<g, b, 0, st>>>(P, pb, mb, m);
+    else if (ebuf) lbm_f64_kernel<false, true, false><<<g, b, 0, st>>>(P, pb, mb, m);
+    else if (stream) lbm_f64_kernel<false, false, true><<<g, b, 0, st>>>(P, pb, mb, m);
+    else lbm_f64_kernel<false, false, false><<<g, b, 0, st>>>(P, pb, mb, m);
     return hipGetLastError();
+}
+
+// Streaming pays where a step's two population buffers are beyond the
+// last-level cache (256 MB) and a row of the lattice is whole cache lines;
+// a streamed part of a line reaches memory on its own.  Measured, us per
+// launch, streaming / plain:
+//   rows of whole lines: FP32S 64x64x64 (226 MB) 23.5 / 21.9, 96x96x64 (255 MB) 52 / 52,
+//     128x128x64 82 / 92, 192x192x32 93 / 104, 256x256x128 629 / 692;
+//     FP64 64x64x64 (226 MB) 46 / 39, 128x128x64 168 / 176, 256x256x128 1345 / 1390
+//   other rows: FP32S 90x154x45 94 / 61, 122x122x101 212 / 160, 250x250x64 547 / 431;
+//     halves of a line (nx = 112, 144, 240) equal;
+//     FP64 122x122x101 320 / 295, 250x250x64 839 / 788, 120x120x64 156 / 166
+bool lbm_streams(Prec prec, int nx, size_t nodes)
+{
+    const size_t es = prec == Prec::F64 ? 8 : 4, row = (size_t)nx * es;
+    return 2 * 54 * es * nodes > ((size_t)256 << 20) && row % (prec == Prec::F64 ? 64 : 128) == 0;
 }
 
 hipError_t launch_init_equilibrium(Prec prec, const LbmParams& P, const double* rho, const double* q,
