@@ -13,6 +13,7 @@
 
 #include "box.h"
 #include "fft_plan.h"
+#include "host_copy.h"
 
 using namespace ehd;
 
@@ -144,6 +145,7 @@ void free_box(ehd_box* b)
     for (auto& pr : b->step_pairs) { (void)hipEventDestroy(pr.first); (void)hipEventDestroy(pr.second); }
     for (hipEvent_t e : b->ev_pool) (void)hipEventDestroy(e);
     if (b->st) (void)hipStreamDestroy(b->st);
+    staging_release();
 }
 
 }  // namespace
@@ -467,6 +469,7 @@ int ehd_create(const ehd_params* p, ehd_box** out)
     if (rc) return rc;
     ehd_box* b = new (std::nothrow) ehd_box();
     if (!b) return set_error(EHD_ENOMEM, "host allocation failed");
+    staging_retain();
     b->prm = *p;
     ehd_derive(p, &b->der);
     b->prec = (p->precision == EHD_FP64) ? Prec::F64 : Prec::F32S;
@@ -756,36 +759,24 @@ int ehd_read_fields(ehd_box* b, double* rho, double* q, double* phi, double* ux,
     if (!b) return set_error(EHD_EINVAL, "null box");
     if (!b->initialised) return set_error(EHD_ESTATE, "box not initialised");
     const size_t S = b->S;
-    double* tmp = nullptr;
-    int rc = alloc((void**)&tmp, S * sizeof(double));
-    if (rc) return rc;
-    struct Guard {
-        double* p;
-        ~Guard() { if (p) (void)hipFree(p); }
-    } guard{tmp};
-    struct Item {
-        double* host;
-        void* dev;
-    } items[] = {{rho, b->rho}, {q, b->q}, {ux, b->ux}, {uy, b->uy}, {uz, b->uz}};
-    for (auto& it : items) {
-        if (!it.host) continue;
-        HIPCHK(launch_to_double(b->prec, it.dev, tmp, S, b->st));
-        HIPCHK(hipMemcpyAsync(it.host, tmp, S * 8, hipMemcpyDeviceToHost, b->st));
-        HIPCHK(hipStreamSynchronize(b->st));
-    }
-    if (phi) {
-        HIPCHK(launch_phi_full(b->prec, b->lp, b->phi, b->phibar, tmp, b->st));
-        HIPCHK(hipMemcpyAsync(phi, tmp, S * 8, hipMemcpyDeviceToHost, b->st));
-        HIPCHK(hipStreamSynchronize(b->st));
-    }
-    if (ex || ey || ez) {
-        if (!b->ebuf) HIPCHK(launch_efield(b->prec, b->lp, b->phi, b->phibar, b->ex, b->ey, b->ez, b->st));
-        if (ex) HIPCHK(hipMemcpyAsync(ex, b->ex, S * 8, hipMemcpyDeviceToHost, b->st));
-        if (ey) HIPCHK(hipMemcpyAsync(ey, b->ey, S * 8, hipMemcpyDeviceToHost, b->st));
-        if (ez) HIPCHK(hipMemcpyAsync(ez, b->ez, S * 8, hipMemcpyDeviceToHost, b->st));
-        HIPCHK(hipStreamSynchronize(b->st));
-    }
-    return EHD_OK;
+    const bool f32 = b->prec == Prec::F32S;
+    HostCopy c[9];
+    int n = 0;
+    auto field = [&](double* host, const void* dev) {
+        if (host) c[n++] = HostCopy{f32 ? HostCopy::kWiden : HostCopy::kDouble, host, dev, S};
+    };
+    field(rho, b->rho);
+    field(q, b->q);
+    field(ux, b->ux);
+    field(uy, b->uy);
+    field(uz, b->uz);
+    if (phi && f32) c[n++] = HostCopy{HostCopy::kWidenAddMean, phi, b->phi, S, b->phibar, (size_t)b->nz, b->nxy};
+    else field(phi, b->phi);
+    if ((ex || ey || ez) && !b->ebuf)
+        HIPCHK(launch_efield(b->prec, b->lp, b->phi, b->phibar, b->ex, b->ey, b->ez, b->st));
+    for (const auto& e : {std::make_pair(ex, b->ex), std::make_pair(ey, b->ey), std::make_pair(ez, b->ez)})
+        if (e.first) c[n++] = HostCopy{HostCopy::kDouble, e.first, e.second, S};
+    return n > 0 ? download(c, n, b->st) : EHD_OK;
 }
 
 int ehd_write_phi(ehd_box* b, const double* phi)

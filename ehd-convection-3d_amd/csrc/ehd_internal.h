@@ -96,10 +96,7 @@ hipError_t launch_efield(Prec prec, const LbmParams& P, const void* phi, const d
                          double* ex, double* ey, double* ez, hipStream_t st);
 
 // Macroscopic field conversion helpers.
-hipError_t launch_to_double(Prec prec, const void* src, double* dst, size_t n, hipStream_t st);
 hipError_t launch_from_double(Prec prec, const double* src, void* dst, size_t n, hipStream_t st);
-hipError_t launch_phi_full(Prec prec, const LbmParams& P, const void* phi, const double* phibar,
-                           double* out, hipStream_t st);
 hipError_t launch_phi_split(Prec prec, const LbmParams& P, const double* phi, void* phio,
                             double* phibar, hipStream_t st);
 

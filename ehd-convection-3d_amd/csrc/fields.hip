@@ -124,24 +124,10 @@ __global__ void __launch_bounds__(256) efield_kernel(LbmParams P, const T* phi, 
     }
 }
 
-__global__ void __launch_bounds__(256) f2d_kernel(const float* src, double* dst, size_t n)
-{
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = (double)src[i];
-}
 __global__ void __launch_bounds__(256) d2f_kernel(const double* src, float* dst, size_t n)
 {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) dst[i] = (float)src[i];
-}
-
-__global__ void __launch_bounds__(256) phi_full_kernel(LbmParams P, const float* phi, const double* phibar,
-                                                       double* out)
-{
-    const unsigned s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= P.S) return;
-    const unsigned z = s / P.nxy;
-    out[s] = (double)phi[s] + phibar[z];
 }
 
 // per-plane mean (one block per plane, fixed reduction order) and fluctuation
@@ -273,25 +259,10 @@ hipError_t launch_efield(Prec prec, const LbmParams& P, const void* phi, const d
     return hipGetLastError();
 }
 
-hipError_t launch_to_double(Prec prec, const void* src, double* dst, size_t n, hipStream_t st)
-{
-    if (prec == Prec::F64) return hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToDevice, st);
-    f2d_kernel<<<grid_for(n), 256, 0, st>>>((const float*)src, dst, n);
-    return hipGetLastError();
-}
-
 hipError_t launch_from_double(Prec prec, const double* src, void* dst, size_t n, hipStream_t st)
 {
     if (prec == Prec::F64) return hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToDevice, st);
     d2f_kernel<<<grid_for(n), 256, 0, st>>>(src, (float*)dst, n);
-    return hipGetLastError();
-}
-
-hipError_t launch_phi_full(Prec prec, const LbmParams& P, const void* phi, const double* phibar, double* out,
-                           hipStream_t st)
-{
-    if (prec == Prec::F64) return hipMemcpyAsync(out, phi, (size_t)P.S * sizeof(double), hipMemcpyDeviceToDevice, st);
-    phi_full_kernel<<<grid_for(P.S), 256, 0, st>>>(P, (const float*)phi, phibar, out);
     return hipGetLastError();
 }
 

@@ -21,6 +21,7 @@
 #include "../../include/ehd_fno.h"
 #include "box.h"
 #include "fno_internal.h"
+#include "host_copy.h"
 
 using namespace ehd;
 
@@ -202,9 +203,10 @@ void free_fno(ehd_fno* f)
     f->allocs.clear();
     f->alloc_bytes.clear();
     if (f->st) (void)hipStreamDestroy(f->st);
+    staging_release();
 }
 
-int upload(const std::vector<float>& h, float* d)
+int put_table(const std::vector<float>& h, float* d)
 {
     HIPCHK(hipMemcpy(d, h.data(), h.size() * sizeof(float), hipMemcpyHostToDevice));
     return EHD_OK;
@@ -225,8 +227,8 @@ int make_dft(ehd_fno* f)
     const double tp = 2.0 * 3.14159265358979323846;
     std::vector<float> r, im;
     auto put = [&](Cbuf& b) -> int {
-        int rc = upload(r, b.r);
-        return rc ? rc : upload(im, b.i);
+        int rc = put_table(r, b.r);
+        return rc ? rc : put_table(im, b.i);
     };
     int rc;
     // AzT[k][z] = exp(-2 pi i k z / Z)
@@ -574,6 +576,12 @@ int loss_and_grad(ehd_fno* f, int B, const float* in, const float* target, doubl
     return EHD_OK;
 }
 
+int download_floats(ehd_fno* f, float* host, const float* dev, size_t n)
+{
+    const HostCopy c{HostCopy::kFloat, host, dev, n};
+    return download(&c, 1, f->st);
+}
+
 int check_batch(const ehd_fno* f, int B)
 {
     if (B < 1 || B > f->c.max_batch) return set_error(EHD_EINVAL, "batch %d outside 1..%d", B, f->c.max_batch);
@@ -596,6 +604,7 @@ int ehd_fno_create(const ehd_fno_config* cfg, ehd_fno** out)
         return set_error(EHD_EINVAL, "modes must lie in 1..X/2, 1..Y/2, 1..Z/2");
     ehd_fno* f = new (std::nothrow) ehd_fno();
     if (!f) return set_error(EHD_ENOMEM, "host allocation failed");
+    staging_retain();
     auto bail = [&](int code) {
         free_fno(f);
         delete f;
@@ -700,8 +709,7 @@ int ehd_fno_set_params(ehd_fno* f, const float* params)
 int ehd_fno_get_params(ehd_fno* f, float* params)
 {
     if (!f || !params) return set_error(EHD_EINVAL, "null argument");
-    HIPCHK(hipMemcpy(params, f->p, f->nparam * sizeof(float), hipMemcpyDeviceToHost));
-    return EHD_OK;
+    return download_floats(f, params, f->p, (size_t)f->nparam);
 }
 
 int ehd_fno_forward(ehd_fno* f, int batch, const float* in, float* out)
@@ -712,9 +720,7 @@ int ehd_fno_forward(ehd_fno* f, int batch, const float* in, float* out)
     HIPCHK(hipMemcpyAsync(f->in, in, (size_t)batch * f->c.d_in * f->ZP * sizeof(float), hipMemcpyHostToDevice, f->st));
     f->resident = 0;   // the inputs no longer match the resident targets
     if ((rc = forward(f, batch))) return rc;
-    HIPCHK(hipMemcpyAsync(out, f->out, (size_t)batch * f->c.d_out * f->ZP * sizeof(float), hipMemcpyDeviceToHost, f->st));
-    HIPCHK(hipStreamSynchronize(f->st));
-    return EHD_OK;
+    return download_floats(f, out, f->out, (size_t)batch * f->c.d_out * f->ZP);
 }
 
 int ehd_fno_gradients(ehd_fno* f, int batch, const float* in, const float* target, double* loss, float* grad)
@@ -723,8 +729,7 @@ int ehd_fno_gradients(ehd_fno* f, int batch, const float* in, const float* targe
     int rc = check_batch(f, batch);
     if (rc) return rc;
     if ((rc = loss_and_grad(f, batch, in, target, loss))) return rc;
-    if (grad) HIPCHK(hipMemcpy(grad, f->g, f->nparam * sizeof(float), hipMemcpyDeviceToHost));
-    return EHD_OK;
+    return grad ? download_floats(f, grad, f->g, (size_t)f->nparam) : EHD_OK;
 }
 
 int ehd_fno_train_step(ehd_fno* f, int batch, const float* in, const float* target, float lr, double* loss)

@@ -278,6 +278,28 @@ def test_diagnostics_current_vs_oracle():
         assert d.step == 3
 
 
+# Field reads below and above one megabyte (with and without worker threads), with
+# a last piece that is not full, and with more pieces than staging slots.
+@pytest.mark.parametrize("shape", [(16, 12, 10), (64, 64, 33), (122, 62, 40), (256, 256, 44)])
+@pytest.mark.parametrize("precision", [E.FP64, E.FP32S])
+def test_field_reads_are_exact(shape, precision):
+    nx, ny, nz = shape
+    rng = np.random.default_rng(5)
+    q, phi = rng.standard_normal((2, nz, ny, nx))
+    with E.Box(E.make_params(nx, ny, nz, T=200.0, precision=precision)) as b:
+        b.init()
+        b.step(2)
+        b.write_charge(q)
+        b.write_phi(phi)
+        every = b.read_fields()
+        alone = {k: b.read_fields((k,))[k] for k in every}
+    for k, v in every.items():
+        assert np.array_equal(v, alone[k]), k
+    assert np.array_equal(every["q"], q if precision == E.FP64 else q.astype(np.float32).astype(np.float64))
+    # FP32S keeps phi as a float beside its plane's mean: rounded once
+    assert np.max(np.abs(every["phi"] - phi)) <= (0.0 if precision == E.FP64 else 2.0**-23 * np.max(np.abs(phi)))
+
+
 def test_profile_sampling_counts_launches():
     """ehd_profile_enable(b, n) brackets the LBM launch and the Poisson chain
     of the steps whose index is a multiple of n, and every ehd_step call; the
