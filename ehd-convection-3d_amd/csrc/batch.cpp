@@ -385,7 +385,7 @@ int ehd_batch_create(const ehd_params* params, int nboxes, int flags, ehd_batch*
         size_t nodes = 0, streamed = 0;
         for (const ehd_box* b : bt->boxes) nodes += b->S;
         for (const ehd_box* b : bt->boxes)
-            if (lbm_streams(b->prec, b->nx, nodes)) streamed += b->S;
+            if (lbm_streams(b->prec, (int)b->lp.px, nodes)) streamed += b->S;
         bt->lbm_stream = 2 * streamed > nodes;
     }
     // Poisson groups by (nx, ny); the z-solve partition follows n, so boxes of
@@ -461,7 +461,7 @@ int ehd_batch_create(const ehd_params* params, int nboxes, int flags, ehd_batch*
             for (int i = 0; i < nboxes; ++i) {
                 ehd_box* b = bt->boxes[i];
                 lbm_f32s_batch_item(h.data() + i * isz, b->lp, pop_bufs_at(b, cur), macro_bufs(b), tile0);
-                tile0 += (unsigned)((b->S + 255) / 256);
+                tile0 += lbm_tiles(b->lp);
             }
             bt->total_tiles = tile0;
             if (hipMalloc(&bt->ditems[cur], h.size()) != hipSuccess)
@@ -482,7 +482,7 @@ int ehd_batch_create(const ehd_params* params, int nboxes, int flags, ehd_batch*
                     for (size_t j = 0; j < gr.members.size(); ++j) {
                         ehd_box* b = bt->boxes[gr.members[j]];
                         lbm_f32s_batch_item(h.data() + j * isz, b->lp, pop_bufs_at(b, cur), macro_bufs(b), tile0);
-                        tile0 += (unsigned)((b->S + 255) / 256);
+                        tile0 += lbm_tiles(b->lp);
                     }
                     gr.tiles = tile0;
                     if (hipMalloc(&gr.items[cur], h.size()) != hipSuccess)
@@ -585,7 +585,7 @@ int ehd_batch_init_consistent(ehd_batch* bt, const double* const* fields9, int i
                 ehd_box* b = bt->boxes[i];
                 h.resize(isz * (m + 1));
                 lbm_f32s_batch_item(h.data() + m * isz, b->lp, pop_bufs_at(b, cur), macro_bufs(b), tile0, tg[i]);
-                tile0 += (unsigned)((b->S + 255) / 256);
+                tile0 += lbm_tiles(b->lp);
                 ++m;
             }
             sets[k].n = m;

@@ -94,6 +94,8 @@ void fill_lbm_params(ehd_box* b)
     L.nx = p.nx; L.ny = p.ny; L.nz = p.nz;
     L.nxy = (unsigned)(p.nx * p.ny);
     L.S = (unsigned)((size_t)p.nx * p.ny * p.nz);
+    L.px = lbm_row_pitch(b->prec, p.nx, p.ny, p.nz);
+    L.SP = (unsigned)((size_t)L.px * p.ny * p.nz);
     L.dt = d.dt; L.cfl = p.cfl; L.cs_square = d.cs_square; L.K = d.K; L.exf = p.exf;
     L.charge0 = d.charge0; L.rho0 = p.rho0;
     L.w[0] = 8.0 / 27.0; L.w[1] = 2.0 / 27.0; L.w[2] = 1.0 / 54.0; L.w[3] = 1.0 / 216.0;
@@ -180,7 +182,7 @@ int run_lbm(ehd_box* b, bool macro, void* const* target_items)
     if (b->prec == Prec::F64) e = launch_lbm_f64(b->lp, pop_bufs(b), macro_bufs(b), b->direct, b->ebuf, macro,
                                                      b->lbm_stream, b->st);
     else e = launch_lbm_f32s_batch(target_items ? target_items[b->cur] : b->lbm_items[b->cur], 1,
-                                   (unsigned)((b->S + 255) / 256), 0, b->lbm_chunk, b->direct, b->ebuf, macro,
+                                   lbm_tiles(b->lp), 0, b->lbm_chunk, b->direct, b->ebuf, macro,
                                    b->lbm_stream, b->st, target_items != nullptr);
     if (e != hipSuccess) return set_error(EHD_EHIP, "LBM launch failed: %s", hipGetErrorString(e));
     if (b->debug_sync) {
@@ -384,15 +386,22 @@ int ckpt_io(ehd_box* b, FILE* f, bool save)
         {b->phibar, (size_t)b->nz * sizeof(double)},
         {b->ex, S * sizeof(double)}, {b->ey, S * sizeof(double)}, {b->ez, S * sizeof(double)},
     };
+    // the file holds the populations' rows without their padding
+    const size_t row = b->nx * es, pitch = b->lp.px * es;
     std::vector<unsigned char> buf;
     for (auto& it : items) {
         buf.resize(it.bytes);
+        const bool padded = (it.dev == b->f[A] || it.dev == b->h[A]) && pitch != row;
         if (save) {
-            HIPCHK(hipMemcpy(buf.data(), it.dev, it.bytes, hipMemcpyDeviceToHost));
+            if (padded)
+                HIPCHK(hipMemcpy2D(buf.data(), row, it.dev, pitch, row, it.bytes / row, hipMemcpyDeviceToHost));
+            else HIPCHK(hipMemcpy(buf.data(), it.dev, it.bytes, hipMemcpyDeviceToHost));
             if (std::fwrite(buf.data(), 1, it.bytes, f) != it.bytes) return set_error(EHD_EINVAL, "checkpoint write failed");
         } else {
             if (std::fread(buf.data(), 1, it.bytes, f) != it.bytes) return set_error(EHD_EINVAL, "checkpoint truncated");
-            HIPCHK(hipMemcpy(it.dev, buf.data(), it.bytes, hipMemcpyHostToDevice));
+            if (padded)
+                HIPCHK(hipMemcpy2D(it.dev, pitch, buf.data(), row, row, it.bytes / row, hipMemcpyHostToDevice));
+            else HIPCHK(hipMemcpy(it.dev, buf.data(), it.bytes, hipMemcpyHostToDevice));
         }
     }
     return EHD_OK;
@@ -478,7 +487,7 @@ int ehd_create(const ehd_params* p, ehd_box** out)
     b->S = b->nxy * p->nz;
     b->esz = (b->prec == Prec::F64) ? 8 : 4;
     fill_lbm_params(b);
-    b->lbm_stream = lbm_streams(b->prec, b->nx, b->S);
+    b->lbm_stream = lbm_streams(b->prec, (int)b->lp.px, b->S);
 
     auto bail = [&](int code) {
         free_box(b);
@@ -487,10 +496,10 @@ int ehd_create(const ehd_params* p, ehd_box** out)
     };
     if (hipStreamCreateWithFlags(&b->st, hipStreamNonBlocking) != hipSuccess)
         return bail(set_error(EHD_EHIP, "hipStreamCreate failed: %s", hipGetErrorString(hipGetLastError())));
-    const size_t S = b->S, es = b->esz;
+    const size_t S = b->S, es = b->esz, pops = 26 * (size_t)b->lp.SP * es;
     for (int i = 0; i < 2; ++i) {
-        if ((rc = alloc(&b->f[i], 26 * S * es)) || (rc = alloc(&b->f0[i], S * es)) ||
-            (rc = alloc(&b->h[i], 26 * S * es)) || (rc = alloc(&b->h0[i], S * es)))
+        if ((rc = alloc(&b->f[i], pops)) || (rc = alloc(&b->f0[i], S * es)) ||
+            (rc = alloc(&b->h[i], pops)) || (rc = alloc(&b->h0[i], S * es)))
             return bail(rc);
     }
     if ((rc = alloc(&b->rho, S * es)) || (rc = alloc(&b->ux, S * es)) || (rc = alloc(&b->uy, S * es)) ||
@@ -594,7 +603,7 @@ int ehd_create(const ehd_params* p, ehd_box** out)
             if (hipMemcpy(b->lbm_items[c], item.data(), isz, hipMemcpyHostToDevice) != hipSuccess)
                 return bail(set_error(EHD_EHIP, "LBM item upload failed"));
         }
-        b->lbm_chunk = lbm_xcd_chunk((unsigned)(p->nx * p->ny));
+        b->lbm_chunk = lbm_xcd_chunk(b->lp.px * (unsigned)p->ny);
     }
     *out = b;
     return EHD_OK;

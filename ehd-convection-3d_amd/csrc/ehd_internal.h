@@ -14,6 +14,9 @@ namespace ehd {
 struct LbmParams {
     int nx, ny, nz;
     unsigned nxy, S;             // nx*ny, nx*ny*nz
+    // pitch of the populations' rows (lbm_row_pitch) and the padded node count
+    // px*ny*nz, which the LBM launches' threads run over
+    unsigned px, SP;
     double dt, cfl, cs_square, K, exf, charge0, rho0;
     double w[4];                 // w0, ws, wa, wd (LBM.h:73-76)
     double omega_plus, omega_minus, omega_c_plus, omega_c_minus;  // LBM.cu:298-302
@@ -55,15 +58,18 @@ struct MacroBufs {
 hipError_t launch_lbm_f64(const LbmParams& P, const PopBufs& pb, const MacroBufs& mb,
                           bool first, bool ebuf, bool macro, bool stream, hipStream_t st);
 // Whether the LBM launches of a box, or of a batch of nodes in all, stream
-// the populations past the caches (rows of nx; the first step never does).
-bool lbm_streams(Prec prec, int nx, size_t nodes);
+// the populations past the caches (rows of pitch px; the first step never does).
+bool lbm_streams(Prec prec, int px, size_t nodes);
+// Pitch of the rows of a box's populations, nx or a whole number of cache lines.
+unsigned lbm_row_pitch(Prec prec, int nx, int ny, int nz);
 // FP32S LBM over one box or a batch of boxes: an opaque item per box (lbm_f32s_batch_item writes
 // lbm_f32s_batch_item_size() bytes), items in a device array sorted by tile0,
-// tile0 = number of 256-node tiles of the boxes before it.  grid = 0 launches
+// tile0 = number of 256-node tiles (lbm_tiles) of the boxes before it.  grid = 0 launches
 // one workgroup per tile; a smaller grid (a multiple of 8) makes the
 // workgroups persistent.  chunk: XCD tile order (0 = linear), see
 // lbm_xcd_chunk.
 size_t lbm_f32s_batch_item_size();
+inline unsigned lbm_tiles(const LbmParams& P) { return (P.SP + 255) / 256; }
 // target: consistent-start target fields [ux, uy, uz, q] (4 S doubles) of the
 // box, used only by launches with target = true (null: the box steps normally).
 void lbm_f32s_batch_item(void* out, const LbmParams& P, const PopBufs& pb, const MacroBufs& mb, unsigned tile0,
@@ -71,7 +77,7 @@ void lbm_f32s_batch_item(void* out, const LbmParams& P, const PopBufs& pb, const
 hipError_t launch_lbm_f32s_batch(const void* items, int nitems, unsigned total_tiles, unsigned grid, unsigned chunk,
                                  bool first, bool ebuf, bool macro, bool stream, hipStream_t st,
                                  bool target = false);
-// XCD tile-order chunk for boxes of nxy nodes per plane: one plane per
+// XCD tile-order chunk for boxes of nxy (padded) nodes per plane: one plane per
 // superblock when a plane is a whole number of 8-tile groups, else 0.
 unsigned lbm_xcd_chunk(unsigned nxy);
 

@@ -94,7 +94,8 @@ __device__ __forceinline__ void stnt(float v, gfloat* p)
     else *p = v;
 }
 
-// One node s of one box: pull, collide, boundary and injection.
+// One node of one box, number sp in its padded rows: pull, collide, boundary
+// and injection.
 //
 // TARGET (consistent start, after Mei et al., J. Comput. Phys. 2006): when
 // the box carries target fields tg = [ux, uy, uz, q] (4 S doubles), every
@@ -105,17 +106,19 @@ __device__ __forceinline__ void stnt(float v, gfloat* p)
 // belong to the target state; the equilibrium start alone lacks them.
 template <bool FIRST, bool EBUF, bool TARGET, bool NT>
 __device__ __forceinline__ void lbm_f32s_node(const LbmParams& P, const F32Consts& c, const PopBufs& pb,
-                                              const MacroBufs& mb, const double* tgp, int macro, unsigned s)
+                                              const MacroBufs& mb, const double* tgp, int macro, unsigned sp)
 {
-    const unsigned nx = P.nx, ny = P.ny, nz = P.nz, nxy = P.nxy, S = P.S;
-    const unsigned x = s % nx, t = s / nx, y = t % ny, z = t / ny;
+    const unsigned nx = P.nx, ny = P.ny, nz = P.nz, nxy = P.nxy, S = P.S, px = P.px;
+    const unsigned x = sp % px, t = sp / px, y = t % ny, z = t / ny;
+    if (x >= nx) return;
+    const unsigned s = t * nx + x;
     const unsigned xm = (x == 0) ? nx - 1 : x - 1, xp = (x == nx - 1) ? 0 : x + 1;
     const unsigned ym = (y == 0) ? ny - 1 : y - 1, yp = (y == ny - 1) ? 0 : y + 1;
     const unsigned zm = (z == 0) ? nz - 1 : z - 1, zp = (z == nz - 1) ? 0 : z + 1;
     const unsigned XS[3] = {xm, x, xp};
-    // populations: row blocks [z][y][d-1][x] (26 x nx floats per row); the
+    // populations: row blocks [z][y][d-1][px] (26 x px floats per row); the
     // source row of a pull along c is (y - c_y, z - c_z)
-    const unsigned RW = 26u * nx;
+    const unsigned RW = 26u * px;
     const unsigned YR[3] = {ym, y, yp}, ZR[3] = {zm * ny, z * ny, zp * ny};
     const unsigned own = t * RW + x;
 
@@ -134,23 +137,23 @@ __device__ __forceinline__ void lbm_f32s_node(const LbmParams& P, const F32Const
         k[0] = h0A[s];
 #pragma unroll
         for (int d = 1; d < 27; ++d) {
-            g[d] = fA[own + (d - 1) * nx];
-            k[d] = hA[own + (d - 1) * nx];
+            g[d] = fA[own + (d - 1) * px];
+            k[d] = hA[own + (d - 1) * px];
         }
     } else {
 #pragma unroll
         for (int d = 1; d < 27; ++d)
-            g[d] = pulled(ldnt<NT>(fA + (ZR[1 - CZ[d]] + YR[1 - CY[d]]) * RW + (d - 1) * nx + XS[1 - CX[d]]), d,
+            g[d] = pulled(ldnt<NT>(fA + (ZR[1 - CZ[d]] + YR[1 - CY[d]]) * RW + (d - 1) * px + XS[1 - CX[d]]), d,
                           c.w[WCLS[d]], dRu, dRd);
         if (z == 0) {
             k[0] = -h0A[s] + c.injk[0];
 #pragma unroll
-            for (int d = 1; d < 27; ++d) k[d] = -hA[own + (opp(d) - 1) * nx] + c.injk[WCLS[d]];
+            for (int d = 1; d < 27; ++d) k[d] = -hA[own + (opp(d) - 1) * px] + c.injk[WCLS[d]];
         } else {
             k[0] = h0A[s];
 #pragma unroll
             for (int d = 1; d < 27; ++d)
-                k[d] = pulled(ldnt<NT>(hA + (ZR[1 - CZ[d]] + YR[1 - CY[d]]) * RW + (d - 1) * nx + XS[1 - CX[d]]), d,
+                k[d] = pulled(ldnt<NT>(hA + (ZR[1 - CZ[d]] + YR[1 - CY[d]]) * RW + (d - 1) * px + XS[1 - CX[d]]), d,
                               c.w[WCLS[d]], dQu, dQd);
         }
     }
@@ -216,15 +219,15 @@ __device__ __forceinline__ void lbm_f32s_node(const LbmParams& P, const F32Const
             const unsigned own1 = own + ny * RW;
 #pragma unroll
             for (int d = 1; d < 27; ++d) {
-                gm[d] = fA[own1 + (d - 1) * nx];
-                dqm += hA[own1 + (d - 1) * nx];
+                gm[d] = fA[own1 + (d - 1) * px];
+                dqm += hA[own1 + (d - 1) * px];
             }
         } else {
             const float dRu1 = sh[nz + 1], dRd1 = sh[2 * nz + 1], dQu1 = sh[4 * nz + 1], dQd1 = sh[5 * nz + 1];
 #pragma unroll
             for (int d = 1; d < 27; ++d) {
                 // node (x, y, 1) pulls from row (y - c_y, 1 - c_z)
-                const unsigned src = ((unsigned)(1 - CZ[d]) * ny + YR[1 - CY[d]]) * RW + (d - 1) * nx + XS[1 - CX[d]];
+                const unsigned src = ((unsigned)(1 - CZ[d]) * ny + YR[1 - CY[d]]) * RW + (d - 1) * px + XS[1 - CX[d]];
                 gm[d] = pulled(fA[src], d, c.w[WCLS[d]], dRu1, dRd1);
                 dqm += pulled(hA[src], d, c.w[WCLS[d]], dQu1, dQd1);
             }
@@ -332,20 +335,20 @@ __device__ __forceinline__ void lbm_f32s_node(const LbmParams& P, const F32Const
             od = gd;
             oe = ge;
         }
-        stnt<NT>(od, fB + own + (d - 1) * nx);
-        stnt<NT>(oe, fB + own + (e - 1) * nx);
+        stnt<NT>(od, fB + own + (d - 1) * px);
+        stnt<NT>(oe, fB + own + (e - 1) * px);
         if (z != nz - 1) {
-            stnt<NT>(kd, hB + own + (d - 1) * nx);
-            stnt<NT>(ke, hB + own + (e - 1) * nx);
+            stnt<NT>(kd, hB + own + (d - 1) * px);
+            stnt<NT>(ke, hB + own + (e - 1) * px);
             if (z == nz - 2) {
-                stnt<NT>(kd, hB + own + ny * RW + (d - 1) * nx);
-                stnt<NT>(ke, hB + own + ny * RW + (e - 1) * nx);
+                stnt<NT>(kd, hB + own + ny * RW + (d - 1) * px);
+                stnt<NT>(ke, hB + own + ny * RW + (e - 1) * px);
             }
         }
     }
 }
 
-// One launch over one box or a batch of boxes: the boxes' node ranges are
+// One launch over one box or a batch of boxes: the boxes' (padded) node ranges are
 // cut into 256-node tiles numbered across the batch (box i owns tiles
 // tile0[i] .. tile0[i+1]-1) and the workgroups stride over all tiles (one
 // tile each when the grid covers them, persistent otherwise).  A single box
@@ -389,7 +392,7 @@ __global__ void __launch_bounds__(256) lbm_f32s_kernel(const BatchItem* __restri
         }
         const BatchItem& it = items[lo];
         const unsigned s = (tile - it.tile0) * 256u + threadIdx.x;
-        if (s < it.P.S) lbm_f32s_node<FIRST, EBUF, TARGET, NT>(it.P, it.c, it.pb, it.mb, TARGET ? it.target : nullptr,
+        if (s < it.P.SP) lbm_f32s_node<FIRST, EBUF, TARGET, NT>(it.P, it.c, it.pb, it.mb, TARGET ? it.target : nullptr,
                                                            macro, s);
     }
 }
@@ -447,7 +450,7 @@ void lbm_f32s_batch_item(void* out, const LbmParams& P, const PopBufs& pb, const
     it.mb = mb;
     it.target = target;
     it.tile0 = tile0;
-    it.ntiles = (P.S + 255) / 256;
+    it.ntiles = lbm_tiles(P);
     std::memcpy(out, &it, sizeof(it));
 }
 

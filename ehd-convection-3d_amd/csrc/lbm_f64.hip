@@ -198,18 +198,20 @@ template <bool FIRST, bool EBUF, bool NT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 lbm_f64_kernel(LbmParams P, PopBufs pb, MacroBufs mb, int macro)
 {
-    const unsigned s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= P.S) return;
-    const unsigned nx = P.nx, ny = P.ny, nz = P.nz, nxy = P.nxy;
-    const unsigned x = s % nx, t = s / nx, y = t % ny, z = t / ny;
+    // threads run over the padded rows, so that a wave's accesses to the populations are whole lines
+    const unsigned sp = blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned nx = P.nx, ny = P.ny, nz = P.nz, nxy = P.nxy, px = P.px;
+    const unsigned x = sp % px, t = sp / px, y = t % ny, z = t / ny;
+    if (sp >= P.SP || x >= nx) return;
+    const unsigned s = t * nx + x;
     const unsigned xm = (x == 0) ? nx - 1 : x - 1, xp = (x == nx - 1) ? 0 : x + 1;
     const unsigned ym = (y == 0) ? ny - 1 : y - 1, yp = (y == ny - 1) ? 0 : y + 1;
     const unsigned zm = (z == 0) ? nz - 1 : z - 1, zp = (z == nz - 1) ? 0 : z + 1;
-    // populations in row blocks [z][y][d-1][x]; a pull along c reads row (y - c_y, z - c_z)
-    const unsigned RW = 26u * nx;
+    // populations in row blocks [z][y][d-1][px]; a pull along c reads row (y - c_y, z - c_z)
+    const unsigned RW = 26u * px;
     const unsigned YR[3] = {ym, y, yp}, ZR[3] = {zm * ny, z * ny, zp * ny}, XS[3] = {xm, x, xp};
     const unsigned own = t * RW + x;
-    auto pulled = [&](int d) { return (ZR[1 - CZ[d]] + YR[1 - CY[d]]) * RW + (d - 1) * nx + XS[1 - CX[d]]; };
+    auto pulled = [&](int d) { return (ZR[1 - CZ[d]] + YR[1 - CY[d]]) * RW + (d - 1) * px + XS[1 - CX[d]]; };
 
     const double* __restrict__ fA = (const double*)pb.f;
     const double* __restrict__ f0A = (const double*)pb.f0;
@@ -222,8 +224,8 @@ lbm_f64_kernel(LbmParams P, PopBufs pb, MacroBufs mb, int macro)
         ht[0] = h0A[s];
 #pragma unroll
         for (int d = 1; d < 27; ++d) {
-            ft[d] = fA[own + (d - 1) * nx];
-            ht[d] = hA[own + (d - 1) * nx];
+            ft[d] = fA[own + (d - 1) * px];
+            ht[d] = hA[own + (d - 1) * px];
         }
     } else {
 #pragma unroll
@@ -232,7 +234,7 @@ lbm_f64_kernel(LbmParams P, PopBufs pb, MacroBufs mb, int macro)
         if (z == 0) {
             ht[0] = -h0A[s] + P.inj[0];
 #pragma unroll
-            for (int d = 1; d < 27; ++d) ht[d] = -hA[own + (opp(d) - 1) * nx] + P.inj[WCLS[d]];
+            for (int d = 1; d < 27; ++d) ht[d] = -hA[own + (opp(d) - 1) * px] + P.inj[WCLS[d]];
         } else {
             ht[0] = h0A[s];
 #pragma unroll
@@ -275,14 +277,14 @@ lbm_f64_kernel(LbmParams P, PopBufs pb, MacroBufs mb, int macro)
             const unsigned own1 = own + ny * RW;
 #pragma unroll
             for (int d = 1; d < 27; ++d) {
-                ftm[d] = fA[own1 + (d - 1) * nx];
-                htm[d] = hA[own1 + (d - 1) * nx];
+                ftm[d] = fA[own1 + (d - 1) * px];
+                htm[d] = hA[own1 + (d - 1) * px];
             }
         } else {
 #pragma unroll
             for (int d = 1; d < 27; ++d) {
                 // node (x, y, 1) pulls from row (y - c_y, 1 - c_z)
-                const unsigned src = ((unsigned)(1 - CZ[d]) * ny + YR[1 - CY[d]]) * RW + (d - 1) * nx + XS[1 - CX[d]];
+                const unsigned src = ((unsigned)(1 - CZ[d]) * ny + YR[1 - CY[d]]) * RW + (d - 1) * px + XS[1 - CX[d]];
                 ftm[d] = fA[src];
                 htm[d] = hA[src];
             }
@@ -337,7 +339,7 @@ lbm_f64_kernel(LbmParams P, PopBufs pb, MacroBufs mb, int macro)
                 else if (TOPSGN[d + 1] < 0) fe = fe - m;
             }
         }
-        const unsigned od = own + (d - 1) * nx, oe = od + nx;
+        const unsigned od = own + (d - 1) * px, oe = od + px;
         stnt<NT>(fd, fB + od);
         stnt<NT>(fe, fB + oe);
         if (!top) {
@@ -373,7 +375,7 @@ lbm_f64_kernel(LbmParams P, PopBufs pb, MacroBufs mb, int macro)
         if (bottom) {
             f0B[s] = ft[0];
 #pragma unroll
-            for (int d = 1; d < 27; ++d) fB[own + (d - 1) * nx] = ft[opp(d)];
+            for (int d = 1; d < 27; ++d) fB[own + (d - 1) * px] = ft[opp(d)];
         } else if (top) {
             f0B[s] = ft[0];
 #pragma unroll
@@ -381,31 +383,31 @@ lbm_f64_kernel(LbmParams P, PopBufs pb, MacroBufs mb, int macro)
                 double v = ft[opp(d)];
                 if (TOPSGN[d] > 0) v = v + P.multi[WCLS[d]];
                 else if (TOPSGN[d] < 0) v = v - P.multi[WCLS[d]];
-                fB[own + (d - 1) * nx] = v;
+                fB[own + (d - 1) * px] = v;
             }
         } else {
             f0B[s] = fo[0];
 #pragma unroll
-            for (int d = 1; d < 27; ++d) fB[own + (d - 1) * nx] = fo[d];
+            for (int d = 1; d < 27; ++d) fB[own + (d - 1) * px] = fo[d];
         }
         if (!top) {
             h0B[s] = ho[0];
 #pragma unroll
-            for (int d = 1; d < 27; ++d) hB[own + (d - 1) * nx] = ho[d];
+            for (int d = 1; d < 27; ++d) hB[own + (d - 1) * px] = ho[d];
             if (copy) {
                 h0B[s + nxy] = ho[0];
 #pragma unroll
-                for (int d = 1; d < 27; ++d) hB[own + ny * RW + (d - 1) * nx] = ho[d];
+                for (int d = 1; d < 27; ++d) hB[own + ny * RW + (d - 1) * px] = ho[d];
             }
         }
     }
 }
 
 // Index of moving population d (1..26) of node `node` in the box's row-block
-// layout [z][y][d-1][x].
-__device__ __forceinline__ size_t pop_at(int d, unsigned node, unsigned nx)
+// layout [z][y][d-1][px].
+__device__ __forceinline__ size_t pop_at(int d, unsigned node, const LbmParams& P)
 {
-    return (size_t)(node / nx) * 26u * nx + (size_t)(d - 1) * nx + node % nx;
+    return (size_t)(node / P.nx) * 26u * P.px + (size_t)(d - 1) * P.px + node % P.nx;
 }
 
 // Equilibrium populations (gpu_init_equilibrium, LBM.cu:114-276) in FP64,
@@ -446,8 +448,8 @@ __global__ void __launch_bounds__(256) init_eq_kernel(LbmParams P, const double*
         const double cc = cdot<true>(d, tc);
         const double fe = wr[c] * (omusq + cu * (1.0 + 0.5 * cu));
         const double he = wc[c] * (omusq_c + cc * (1.0 + 0.5 * cc));
-        f[pop_at(d, s, P.nx)] = (T)(fe - P.w[c] * rs);
-        h[pop_at(d, s, P.nx)] = (T)(he - P.w[c] * qs);
+        f[pop_at(d, s, P)] = (T)(fe - P.w[c] * rs);
+        h[pop_at(d, s, P)] = (T)(he - P.w[c] * qs);
     }
 }
 
@@ -480,11 +482,11 @@ __global__ void __launch_bounds__(256) read_pre_kernel(LbmParams P, int direct, 
         const double wf = P.w[WCLS[d]];
         const unsigned src = direct ? s : (XS[1 - CX[d]] + YS[1 - CY[d]] + ZS[1 - CZ[d]]);
         const unsigned zs = direct ? z : ZP[1 - CZ[d]];
-        f1o[(d - 1) * S + s] = (double)f[pop_at(d, src, nx)] + wf * rsh(zs);
+        f1o[(d - 1) * S + s] = (double)f[pop_at(d, src, P)] + wf * rsh(zs);
         if (!direct && z == 0)
-            h1o[(d - 1) * S + s] = -((double)h[pop_at(opp(d), s, nx)] + wf * qsh(0)) + P.inj[WCLS[d]];
+            h1o[(d - 1) * S + s] = -((double)h[pop_at(opp(d), s, P)] + wf * qsh(0)) + P.inj[WCLS[d]];
         else
-            h1o[(d - 1) * S + s] = (double)h[pop_at(d, src, nx)] + wf * qsh(zs);
+            h1o[(d - 1) * S + s] = (double)h[pop_at(d, src, P)] + wf * qsh(zs);
     }
 }
 
@@ -503,8 +505,8 @@ __global__ void __launch_bounds__(256) write_pre_kernel(LbmParams P, const doubl
 #pragma unroll
     for (int d = 1; d < 27; ++d) {
         const double wf = P.w[WCLS[d]];
-        f[pop_at(d, s, P.nx)] = (T)(f1[(d - 1) * S + s] - wf * rs);
-        h[pop_at(d, s, P.nx)] = (T)(h1[(d - 1) * S + s] - wf * qs);
+        f[pop_at(d, s, P)] = (T)(f1[(d - 1) * S + s] - wf * rs);
+        h[pop_at(d, s, P)] = (T)(h1[(d - 1) * S + s] - wf * qs);
     }
 }
 
@@ -515,7 +517,7 @@ inline dim3 grid_for(unsigned n) { return dim3((n + 255) / 256); }
 hipError_t launch_lbm_f64(const LbmParams& P, const PopBufs& pb, const MacroBufs& mb, bool first,
                           bool ebuf, bool macro, bool stream, hipStream_t st)
 {
-    dim3 g = grid_for(P.S), b(256);
+    dim3 g = grid_for(P.SP), b(256);
     int m = macro ? 1 : 0;
     if (first && ebuf) lbm_f64_kernel<true, true, false><<<g, b, 0, st>>>(P, pb, mb, m);
     else if (first) lbm_f64_kernel<true, false, false><<<g, b, 0, st>>>(P, pb, mb, m);
@@ -525,20 +527,39 @@ hipError_t launch_lbm_f64(const LbmParams& P, const PopBufs& pb, const MacroBufs
     return hipGetLastError();
 }
 
-// Streaming pays where a step's two population buffers are beyond the
-// last-level cache (256 MB) and a row of the lattice is whole cache lines;
-// a streamed part of a line reaches memory on its own.  Measured, us per
-// launch, streaming / plain:
+// Streaming pays where a step's two population buffers are well beyond the
+// last-level cache (256 MB) and a row of the lattice is whole cache lines; a
+// streamed part of a line reaches memory on its own.  Measured, us per launch,
+// streaming / plain:
 //   rows of whole lines: FP32S 64x64x64 (226 MB) 23.5 / 21.9, 96x96x64 (255 MB) 52 / 52,
-//     128x128x64 82 / 92, 192x192x32 93 / 104, 256x256x128 629 / 692;
-//     FP64 64x64x64 (226 MB) 46 / 39, 128x128x64 168 / 176, 256x256x128 1345 / 1390
-//   other rows: FP32S 90x154x45 94 / 61, 122x122x101 212 / 160, 250x250x64 547 / 431;
-//     halves of a line (nx = 112, 144, 240) equal;
-//     FP64 122x122x101 320 / 295, 250x250x64 839 / 788, 120x120x64 156 / 166
-bool lbm_streams(Prec prec, int nx, size_t nodes)
+//     112x112x64 (347 MB) 76 / 76, 128x128x64 (453 MB) 82 / 92, 256x256x128 629 / 692;
+//     FP64 64x64x64 (226 MB) 46 / 39, 72x72x64 (287 MB) 66 / 62,
+//     128x128x32 (453 MB) 86 / 91, 256x256x128 1343 / 1390
+//   other rows: FP32S 122x122x101 212 / 160, 250x250x64 547 / 431; FP64
+//     122x122x101 320 / 297, 250x250x64 839 / 788; halves of a line: FP32S
+//     equal (nx = 112, 144, 240), FP64 156 / 166 (120x120x64)
+constexpr size_t kStreamed = (size_t)384 << 20;
+
+bool lbm_streams(Prec prec, int px, size_t nodes)
 {
-    const size_t es = prec == Prec::F64 ? 8 : 4, row = (size_t)nx * es;
-    return 2 * 54 * es * nodes > ((size_t)256 << 20) && row % (prec == Prec::F64 ? 64 : 128) == 0;
+    const size_t es = prec == Prec::F64 ? 8 : 4, row = (size_t)px * es;
+    return 2 * 54 * es * nodes > kStreamed && row % (prec == Prec::F64 ? 64 : 128) == 0;
+}
+
+// Rows of whole cache lines for a state that streams, where they cost at most
+// an eighth more memory (the padding is never read or written): every line is
+// then written whole by one wave, which an unpadded row's first and last are
+// not.  Dense (plain) / padded (streaming): FP32S 122x122x101 158 / 140 us,
+// 200x200x64 252 / 222, 250x250x64 432 / 328; FP64 122x122x101 297 / 270,
+// 250x250x64 800 / 660; a state that mostly stays in the cache loses (FP32S
+// 90x154x45, 269 MB, 62 / 68).
+unsigned lbm_row_pitch(Prec prec, int nx, int ny, int nz)
+{
+    const size_t es = prec == Prec::F64 ? 8 : 4, line = 128 / es;
+    const size_t px = ((size_t)nx + line - 1) / line * line, rows = (size_t)ny * nz;
+    if (2 * 54 * es * nx * rows <= kStreamed || 8 * px > 9 * (size_t)nx || 26 * px * rows >= ((size_t)1 << 32))
+        return (unsigned)nx;
+    return (unsigned)px;
 }
 
 hipError_t launch_init_equilibrium(Prec prec, const LbmParams& P, const double* rho, const double* q,
