@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <initializer_list>
 #include <new>
 #include <vector>
 
@@ -178,6 +179,29 @@ hipError_t cgemm(ehd_fno* f, const Geo& g, const float* Ar, const float* Ai, con
                  float* Cr, float* Ci, int sa, int sb, float beta, hipStream_t st)
 {
     return xgemm(f, g, Ar, Ai, Br, Bi, Cr, Ci, sa, sb, 1.f, beta, st);
+}
+
+// the mixing kernels' operands, checked like the GEMMs'
+bool mix_operands(const ehd_fno* f, int B, std::initializer_list<const float*> spectra,
+                  std::initializer_list<const float*> weights)
+{
+    const long long w = f->c.width;
+    for (const float* p : spectra)
+        if (!in_range(f, p, B * w * f->NM - 1)) return false;
+    for (const float* p : weights)
+        if (!in_range(f, p, f->NM * w * w - 1)) return false;
+    return true;
+}
+
+// n complex products of B x w by w x w per mode in one launch: each weight
+// plane read (and for the second product written) once, the spectra read and
+// one of them written
+void mix_work(ehd_fno* f, int B, int n)
+{
+    const double w = f->c.width, spec = 2.0 * B * w * f->NM, weights = 2.0 * w * w * f->NM;
+    f->work.flops += 8.0 * B * w * w * f->NM * n;
+    f->work.bytes += 4.0 * (n * weights + (n + 1) * spec);
+    f->work.launches += 1;
 }
 
 int calloc_c(ehd_fno* f, Cbuf* b, long long n)
@@ -371,7 +395,12 @@ int spectral_fwd(ehd_fno* f, int l, int B, const float* v, float* out, float bet
         g.cm = KX; g.cn = 1;
         FCHK(cgemm(f, g, f->Vy.r, f->Vy.i, f->Cx.r, f->Cx.i, S.r, S.i, 1, 1, 0.f, f->st));
     }
-    {   // 4. Ym[b][o][md] = sum_c S[b][c][md] R[md][c][o]
+    // 4. Ym[b][o][md] = sum_c S[b][c][md] R[md][c][o]
+    if (mix_fits(w, B)) {
+        if (!mix_operands(f, B, {S.r, S.i, f->Ym.r, f->Ym.i}, {Rr, Ri})) return set_error(EHD_EINVAL, "mixing operands");
+        mix_work(f, B, 1);
+        FCHK(mix_forward(w, B, NM, S.r, S.i, Rr, Ri, f->Ym.r, f->Ym.i, f->st));
+    } else {
         Geo g;
         g.M = B; g.N = w; g.K = w;
         g.am = (long long)w * NM; g.ak = NM; g.a1 = 1;
@@ -446,7 +475,14 @@ int spectral_bwd(ehd_fno* f, int l, int B, const float* du, float* dv, float bet
         g.cm = KX; g.cn = 1;
         FCHK(cgemm(f, g, f->Wx.r, f->Wx.i, f->Cxi.r, f->Cxi.i, f->Ym.r, f->Ym.i, 1, -1, 0.f, f->st));
     }
-    {   // 4b. G_R[md][c][o] = sum_b conj(S[b][c][md]) G_Ym[b][o][md]
+    // 4b. G_R[md][c][o] = sum_b conj(S[b][c][md]) G_Ym[b][o][md], and
+    // 4b'. G_S[b][c][md] = sum_o G_Ym[b][o][md] conj(R[md][c][o])  (into S: the spectrum is no longer needed)
+    if (mix_fits(w, B)) {
+        if (!mix_operands(f, B, {S.r, S.i, f->Ym.r, f->Ym.i}, {Rr, Ri, dRr, dRi}))
+            return set_error(EHD_EINVAL, "mixing operands");
+        mix_work(f, B, 2);
+        FCHK(mix_backward(w, B, NM, S.r, S.i, f->Ym.r, f->Ym.i, Rr, Ri, dRr, dRi, f->st));
+    } else {
         Geo g;
         g.M = w; g.N = w; g.K = B;
         g.am = NM; g.ak = (long long)w * NM; g.a1 = 1;
@@ -454,9 +490,7 @@ int spectral_bwd(ehd_fno* f, int l, int B, const float* du, float* dv, float bet
         g.cm = w; g.cn = 1; g.c1 = (long long)w * w;
         g.nb1 = NM;
         FCHK(cgemm(f, g, S.r, S.i, f->Ym.r, f->Ym.i, dRr, dRi, -1, 1, 0.f, f->st));
-    }
-    {   // 4b'. G_S[b][c][md] = sum_o G_Ym[b][o][md] conj(R[md][c][o])  (into S: the spectrum is no longer needed)
-        Geo g;
+        g = Geo{};
         g.M = B; g.N = w; g.K = w;
         g.am = (long long)w * NM; g.ak = NM; g.a1 = 1;
         g.bk = 1; g.bn = w; g.b1 = (long long)w * w;

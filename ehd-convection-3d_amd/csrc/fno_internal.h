@@ -45,6 +45,16 @@ struct CGemmArgs {
     float sa, sb;
 };
 hipError_t cgemm_bf16(const CGemmArgs& x, hipStream_t st);
+// The per-mode mixing of a spectral layer (fno_mix.hip), bit-identical to the
+// batched complex GEMMs: spectra [b][c][md], weights [md][c][o], md < NM
+// (a multiple of 4); shapes for which mix_fits holds.
+//   forward:  Y[b][o] = sum_c S[b][c] R[c][o]
+//   backward: dR[c][o] = sum_b conj(S[b][c]) G[b][o], then S[b][c] = sum_o G[b][o] conj(R[c][o])
+bool mix_fits(int w, int B);
+hipError_t mix_forward(int w, int B, int NM, const float* Sr, const float* Si, const float* Rr, const float* Ri,
+                       float* Yr, float* Yi, hipStream_t st);
+hipError_t mix_backward(int w, int B, int NM, float* Sr, float* Si, const float* Gr, const float* Gi, const float* Rr,
+                        const float* Ri, float* dRr, float* dRi, hipStream_t st);
 // staging layout gemm_bf16 picks for A and B: 0 k unit-stride, 1 m (n) unit-stride
 // (16-byte loads), 2 element loads
 int gemm_layout_a(const GemmArgs& g);

@@ -14,30 +14,11 @@
 
 #include <cstdint>
 
+#include "fno_device.h"
 #include "fno_internal.h"
 
 namespace ehd {
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ uint32_t to_bf16(float f)
-{
-    uint32_t u = __float_as_uint(f);
-    u += 0x7FFFu + ((u >> 16) & 1u);   // round to nearest even (finite inputs)
-    return u >> 16;
-}
-
-__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) { return to_bf16(lo) | (to_bf16(hi) << 16); }
-
-// GELU with the exact (erf) form, and its derivative
-__device__ __forceinline__ float gelu(float v) { return 0.5f * v * (1.0f + erff(v * 0.70710678118654752f)); }
-
-__device__ __forceinline__ float gelu_grad(float x)
-{
-    return 0.5f * (1.0f + erff(x * 0.70710678118654752f)) + x * expf(-0.5f * x * x) * 0.3989422804014327f;
-}
 
 // Tile 64 x 64 x 32; 256 threads = 4 waves, each owning a 32 x 32 block of C
 // (2 x 2 MFMA blocks of 16 x 16).  Both operands sit in LDS as bf16 rows of

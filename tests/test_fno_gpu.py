@@ -237,6 +237,50 @@ def test_gradients_with_split_k_slices_match_oracle():
     assert max(errs.values()) < 5e-2, errs
 
 
+def _small_net(width, modes, batch, seed, grid=(12, 8, 6), layers=2):
+    cfg = F.FNOConfig(X=grid[0], Y=grid[1], Z=grid[2], width=width, modes=modes, layers=layers, d_in=6, d_hidden=24,
+                      d_out=5)
+    rng = np.random.default_rng(seed)
+    p = F.init_params(cfg, seed=seed)
+    for k in p:
+        if k in ("Pb", "Q1b", "Q2b") or k.startswith("b"):
+            p[k] = 0.1 * rng.standard_normal(p[k].shape)
+        if k.startswith("R"):
+            p[k] = p[k] * width * width * 0.3
+    net = G.FNO(cfg.X, cfg.Y, cfg.Z, width=width, modes=modes, layers=layers, d_in=cfg.d_in, d_hidden=cfg.d_hidden,
+                d_out=cfg.d_out, max_batch=batch)
+    net.set_params(p)
+    a = rng.standard_normal((batch, cfg.d_in, cfg.Z, cfg.Y, cfg.X)).astype(np.float32)
+    t = rng.standard_normal((batch, cfg.d_out, cfg.Z, cfg.Y, cfg.X)).astype(np.float32)
+    return cfg, p, net, a, t
+
+
+# Widths 16 and 32 take kernels of their own up to 16 samples: 17 samples go through
+# the batched GEMMs, and every sample alone or in a smaller batch has to come out
+# the same bit for bit (mode counts that are and are not whole groups of 16).
+@pytest.mark.parametrize("width", [16, 32])
+@pytest.mark.parametrize("modes", [(3, 3, 1), (4, 2, 3)])
+def test_small_batches_match_the_batched_gemms_bitwise(width, modes):
+    _, _, net, a, _ = _small_net(width, modes, 17, seed=3)
+    every = net.forward(a)
+    assert np.all(np.isfinite(every))
+    for i, n in ((0, 1), (1, 3), (4, 8), (1, 16)):
+        assert np.array_equal(net.forward(a[i:i + n]), every[i:i + n]), (i, n)
+
+
+@pytest.mark.parametrize("width,batch", [(16, 2), (32, 8), (32, 9), (16, 16), (32, 17)])
+def test_gradients_of_every_width_and_batch_path_match_oracle(width, batch):
+    cfg, p, net, a, t = _small_net(width, (3, 3, 2), batch, seed=11)
+    out, cache = F.forward(cfg, p, a.astype(np.float64))
+    loss_ref, dout = F.mse(out, t)
+    gref = F.backward(cfg, p, cache, dout)
+    loss, g = net.gradients(a, t)
+    gg = G.unflatten(net.cfg, g)
+    assert abs(loss / loss_ref - 1) < 1e-2, (loss, loss_ref)
+    errs = {k: _rel(gg[k], gref[k]) for k in gref}
+    assert max(errs.values()) < 5e-2, errs
+
+
 def test_adam_steps_reduce_loss():
     p, a, t, net = _setup(seed=2)
     losses = [net.train_step(a, t, 3e-3) for _ in range(30)]
