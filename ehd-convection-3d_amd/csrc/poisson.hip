@@ -884,6 +884,20 @@ __global__ void __launch_bounds__(NT) zsolve_kernel(const PoissonJob* __restrict
     }
 }
 
+// Dirichlet values of the potential on the walls (odd_extract,
+// poisson.cu:158-165) for the rows first .. first + count of a plane, beside the
+// first and the last interior plane (FP64; FP32S keeps them in the plane means)
+template <typename T>
+__device__ __forceinline__ void wall_rows(EHD_GLOBAL T* phi, int zi, int n, int nx, int ny, int first, int count,
+                                          double voltage)
+{
+    for (int w = 0; w < 2; ++w) {
+        if (zi != (w ? n - 1 : 0)) continue;
+        EHD_GLOBAL T* p = phi + (size_t)(w ? n + 1 : 0) * nx * ny + (size_t)first * nx;
+        for (int i = threadIdx.x; i < count * nx; i += blockDim.x) p[i] = w ? (T)0 : (T)voltage;
+    }
+}
+
 // (3b) C2R along x, two real rows per complex line, scaled by 1/(nx*ny), plus
 // the wall potential (F64) or nothing (FP32S fluctuation).  A block takes up
 // to 2*lpb consecutive rows y0.. of one plane; the transposed spectrum is read
@@ -951,6 +965,7 @@ __global__ void __launch_bounds__(256) fftx_inv_kernel(const PoissonJob* __restr
     const double inv = 1.0 / ((double)nx * (double)ny);
     const double lin = add_linear ? voltage * (1.0 - (double)z / (double)(nz - 1)) : 0.0;
     EHD_GLOBAL T* row0 = phi + (size_t)z * nx * ny + (size_t)y0 * nx;
+    if (add_linear) wall_rows(phi, zi, J.n, nx, ny, y0, 2 * nl, voltage);
     if constexpr (N > 0) {
         auto ld = [&](int l, int i) -> cplx<T> { return A[l * ldl + padi(i)]; };
         auto sf = [&](int l, int i, cplx<T> v) {
@@ -970,15 +985,152 @@ __global__ void __launch_bounds__(256) fftx_inv_kernel(const PoissonJob* __restr
     }
 }
 
-// Dirichlet values of the potential on the walls (odd_extract, poisson.cu:158-165).
-__global__ void __launch_bounds__(256) phi_walls_kernel(const PoissonJob* __restrict__ jobs, int nxy)
+// (1) and (3) for a small plane in one launch each: a block holds a whole
+// plane, transforms its row pairs, turns them into the nx/2+1 lines along y in
+// LDS and transforms those, or the other way round.  The same line programs
+// as the separate passes, so the same numbers bit for bit.  Two launches and
+// a spectrum round trip less per direction: the whole solve takes, five launches
+// / three, FP32S 32x32x16 22.5 / 19.0 us, 64x64x64 24.1 / 18.2; FP64 64x64x32
+// 28.1 / 22.2 us.
+constexpr int kPlaneThreads = 512;
+constexpr int plane_pitch(int N, int n) { return N > 0 ? (padi(N - 1) + 1) | 1 : n | 1; }
+
+// lines and elements of the two LDS buffers of a plane
+template <int N>
+struct PlaneBufs {
+    int ldx, ldy, size;      // pitches, elements per buffer
+    __host__ __device__ PlaneBufs(int nx, int ny)
+        : ldx(plane_pitch(N, nx)), ldy(plane_pitch(N, ny)),
+          size((ny / 2) * ldx > (nx / 2 + 1) * ldy ? (ny / 2) * ldx : (nx / 2 + 1) * ldy)
+    {
+    }
+};
+
+template <typename T, int N>
+__global__ void __launch_bounds__(kPlaneThreads) plane_fwd_kernel(const PoissonJob* __restrict__ jobs,
+                                                                  const cplx<T>* __restrict__ twx,
+                                                                  const cplx<T>* __restrict__ twy, PlanArg<N> plx,
+                                                                  PlanArg<N> ply, int nx_rt, int ny_rt, int lgx,
+                                                                  int lgy)
 {
     const PoissonJob& J = jobs[blockIdx.y];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nxy) return;
-    EHD_GLOBAL double* phi = gptr((double*)J.phi);
-    phi[i] = J.voltage;
-    phi[(size_t)(J.n + 1) * nxy + i] = 0.0;
+    const int zi = blockIdx.x;
+    if (zi >= J.n) return;                           // a shorter box of the batch
+    const int nx = N > 0 ? N : nx_rt, ny = N > 0 ? N : ny_rt, nxh = nx / 2 + 1, nl = ny / 2;
+    const PlaneBufs<N> pb(nx, ny);
+    extern __shared__ unsigned char smem_raw[];
+    cplx<T>* tx = reinterpret_cast<cplx<T>*>(smem_raw);
+    cplx<T>* ty = tx + nx;
+    cplx<T>* A = ty + ny;
+    cplx<T>* B = A + pb.size;
+    EHD_GLOBAL const T* qp = gptr((const T*)J.q) + (size_t)(zi + 1) * nx * ny;
+    EHD_GLOBAL cplx<T>* out = gptr((cplx<T>*)J.spec) + (size_t)zi * nxh * ny;
+    const double neps = -1.0 / J.eps;
+    for (int i = threadIdx.x; i < nx; i += blockDim.x) tx[i] = twx[i];
+    for (int i = threadIdx.x; i < ny; i += blockDim.x) ty[i] = twy[i];
+    auto row_pair = [&](int l, int i) -> cplx<T> {
+        return {(T)((double)qp[(size_t)(2 * l) * nx + i] * neps), (T)((double)qp[(size_t)(2 * l + 1) * nx + i] * neps)};
+    };
+    cplx<T>* res = A;
+    if constexpr (N > 0) {
+        __syncthreads();
+        auto sf = [](int, int, cplx<T>) {};
+        ct_run<T, N, 0, 1, false, false>(row_pair, sf, A, nl, pb.ldx, tx, -1);
+    } else {
+        rows_copy<4, cplx<T>>(nl * nx, nx, plx.mn, row_pair,
+                              [&](int l, int i, cplx<T> v) { A[l * pb.ldx + i] = v; });
+        __syncthreads();
+        res = rt_fft<T>(A, B, plx, nl, lgx, pb.ldx, tx, -1);
+    }
+    // the lines along y: as fftx_fwd_kernel writes them, into the other buffer
+    cplx<T>* lines = res == A ? B : A;
+    const int lanes = 1 << lgx;
+    for (int w = threadIdx.x; w < nxh * lanes; w += blockDim.x) {
+        const int k = w >> lgx, l = w & (lanes - 1);
+        if (l >= nl) continue;
+        const int kn = k == 0 ? 0 : nx - k;
+        const cplx<T> zk = res[l * pb.ldx + (N > 0 ? padi(k) : k)], zn = res[l * pb.ldx + (N > 0 ? padi(kn) : kn)];
+        cplx<T>* p = lines + k * pb.ldy;
+        p[N > 0 ? padi(2 * l) : 2 * l] = {(T)0.5 * (zk.x + zn.x), (T)0.5 * (zk.y - zn.y)};
+        p[N > 0 ? padi(2 * l + 1) : 2 * l + 1] = {(T)0.5 * (zk.y + zn.y), (T)-0.5 * (zk.x - zn.x)};
+    }
+    __syncthreads();
+    if constexpr (N > 0) {
+        auto ld = [&](int l, int i) -> cplx<T> { return lines[l * pb.ldy + padi(i)]; };
+        auto sf = [&](int l, int i, cplx<T> v) { stc(out + (size_t)l * N + i, v); };
+        ct_run<T, N, 0, 1, true, true>(ld, sf, lines, nxh, pb.ldy, ty, -1);
+    } else {
+        const cplx<T>* r = rt_fft<T>(lines, res, ply, nxh, lgy, pb.ldy, ty, -1);
+        rows_copy<4, cplx<T>>(
+            nxh * ny, ny, ply.mn, [&](int l, int i) { return r[l * pb.ldy + i]; },
+            [&](int l, int i, cplx<T> v) { stc(out + (size_t)l * ny + i, v); });
+    }
+}
+
+template <typename T, int N>
+__global__ void __launch_bounds__(kPlaneThreads) plane_inv_kernel(const PoissonJob* __restrict__ jobs,
+                                                                  const cplx<T>* __restrict__ twx,
+                                                                  const cplx<T>* __restrict__ twy, PlanArg<N> plx,
+                                                                  PlanArg<N> ply, int nx_rt, int ny_rt, int lgx,
+                                                                  int lgy, int add_linear)
+{
+    const PoissonJob& J = jobs[blockIdx.y];
+    const int zi = blockIdx.x;
+    if (zi >= J.n) return;                           // a shorter box of the batch
+    const int nx = N > 0 ? N : nx_rt, ny = N > 0 ? N : ny_rt, nxh = nx / 2 + 1, nl = ny / 2;
+    const PlaneBufs<N> pb(nx, ny);
+    extern __shared__ unsigned char smem_raw[];
+    cplx<T>* tx = reinterpret_cast<cplx<T>*>(smem_raw);
+    cplx<T>* ty = tx + nx;
+    cplx<T>* A = ty + ny;
+    cplx<T>* B = A + pb.size;
+    EHD_GLOBAL const cplx<T>* in = gptr((const cplx<T>*)J.spec) + (size_t)zi * nxh * ny;
+    EHD_GLOBAL T* phi = gptr((T*)J.phi);
+    for (int i = threadIdx.x; i < nx; i += blockDim.x) tx[i] = twx[i];
+    for (int i = threadIdx.x; i < ny; i += blockDim.x) ty[i] = twy[i];
+    auto line = [&](int l, int i) -> cplx<T> { return ldc(in + (size_t)l * ny + i); };
+    cplx<T>* res = A;
+    if constexpr (N > 0) {
+        __syncthreads();
+        auto sf = [](int, int, cplx<T>) {};
+        ct_run<T, N, 0, 1, false, false>(line, sf, A, nxh, pb.ldy, ty, +1);
+    } else {
+        rows_copy<4, cplx<T>>(nxh * ny, ny, ply.mn, line, [&](int l, int i, cplx<T> v) { A[l * pb.ldy + i] = v; });
+        __syncthreads();
+        res = rt_fft<T>(A, B, ply, nxh, lgy, pb.ldy, ty, +1);
+    }
+    // the row pairs: as fftx_inv_kernel builds them, into the other buffer
+    cplx<T>* rows = res == A ? B : A;
+    const int lanes = 1 << lgx;
+    for (int w = threadIdx.x; w < nxh * lanes; w += blockDim.x) {
+        const int k = w >> lgx, l = w & (lanes - 1);
+        if (l >= nl) continue;
+        const cplx<T>* p = res + k * pb.ldy;
+        cplx<T> a = p[N > 0 ? padi(2 * l) : 2 * l], b = p[N > 0 ? padi(2 * l + 1) : 2 * l + 1];
+        if (k == 0 || 2 * k == nx) {
+            a.y = (T)0;
+            b.y = (T)0;
+        }
+        cplx<T>* z = rows + l * pb.ldx;
+        z[N > 0 ? padi(k) : k] = {a.x - b.y, a.y + b.x};
+        if (k > 0 && 2 * k < nx) z[N > 0 ? padi(nx - k) : nx - k] = {a.x + b.y, b.x - a.y};
+    }
+    __syncthreads();
+    const double inv = 1.0 / ((double)nx * (double)ny);
+    const double lin = add_linear ? J.voltage * (1.0 - (double)(zi + 1) / (double)(J.n + 1)) : 0.0;
+    EHD_GLOBAL T* row0 = phi + (size_t)(zi + 1) * nx * ny;
+    if (add_linear) wall_rows(phi, zi, J.n, nx, ny, 0, ny, J.voltage);
+    auto put = [&](int l, int i, cplx<T> v) {
+        row0[(size_t)(2 * l) * nx + i] = (T)((double)v.x * inv + lin);
+        row0[(size_t)(2 * l + 1) * nx + i] = (T)((double)v.y * inv + lin);
+    };
+    if constexpr (N > 0) {
+        auto ld = [&](int l, int i) -> cplx<T> { return rows[l * pb.ldx + padi(i)]; };
+        ct_run<T, N, 0, 1, true, true>(ld, put, rows, nl, pb.ldx, tx, +1);
+    } else {
+        const cplx<T>* r = rt_fft<T>(rows, res, plx, nl, lgx, pb.ldx, tx, +1);
+        rows_copy<4, cplx<T>>(nl * nx, nx, plx.mn, [&](int l, int i) { return r[l * pb.ldx + i]; }, put);
+    }
 }
 
 constexpr size_t kMaxLds = 65536;
@@ -1073,11 +1225,68 @@ hipError_t launch_y(const PoissonGroup& g, bool inverse, hipStream_t st)
     return hipSuccess;
 }
 
+int log2_ceil(int v)
+{
+    int lg = 0;
+    while ((1 << lg) < v) ++lg;
+    return lg;
+}
+
+// Planes of up to 64 x 64 points take the one-launch transforms where their two
+// buffers fit.  Larger ones keep too few blocks busy for too long, five launches /
+// three: FP32S 96x96x64 26.3 / 39 us, 100x80x64 29.6 / 35.5, 128x128x64 33 / 47
+// (62x64x40, the slowest kind of plan within the line, 28.9 / 28.1).
+template <typename T, int N>
+size_t plane_lds(int nx, int ny)
+{
+    return ((size_t)nx + ny + 2 * (size_t)PlaneBufs<N>(nx, ny).size) * sizeof(cplx<T>);
+}
+constexpr int kPlaneMost = 4096;
+constexpr size_t kPlaneLds = 80 << 10;   // two blocks per compute unit
+
+template <typename T, int N>
+bool plane_fits(int nx, int ny)
+{
+    if (N > 0 && (nx != ny || (nx / 2 + 1) * ct_max_nb(N > 0 ? N : 1) > kPlaneThreads)) return false;
+    return nx * ny <= kPlaneMost && plane_lds<T, N>(nx, ny) <= kPlaneLds;
+}
+
+template <typename T, int N>
+hipError_t launch_plane(const PoissonGroup& g, bool inverse, hipStream_t st)
+{
+    const dim3 grid(g.max_n, g.njobs);
+    const size_t sh = plane_lds<T, N>(g.nx, g.ny);
+    const cplx<T>*twx = (const cplx<T>*)g.twx, *twy = (const cplx<T>*)g.twy;
+    const int lgx = log2_ceil(g.ny / 2), lgy = log2_ceil(g.nx / 2 + 1);
+    const PlanArg<N> plx = plan_arg<N>(g.nx), ply = plan_arg<N>(g.ny);
+    if (inverse)
+        plane_inv_kernel<T, N><<<grid, kPlaneThreads, sh, st>>>(g.jobs, twx, twy, plx, ply, g.nx, g.ny, lgx, lgy,
+                                                                g.split_mean ? 0 : 1);
+    else
+        plane_fwd_kernel<T, N><<<grid, kPlaneThreads, sh, st>>>(g.jobs, twx, twy, plx, ply, g.nx, g.ny, lgx, lgy);
+    return hipGetLastError();
+}
+
+// The plane kernels' plan: a compile-time one where both sides have it and a
+// line's butterflies fit the block (f(constant N) of 32, 48 or 64), else the
+// runtime plan, else none
+template <typename T, class F>
+bool with_plane(int nx, int ny, const F& f)
+{
+    if (nx == 32 && plane_fits<T, 32>(nx, ny)) f(std::integral_constant<int, 32>{});
+    else if (nx == 48 && plane_fits<T, 48>(nx, ny)) f(std::integral_constant<int, 48>{});
+    else if (nx == 64 && plane_fits<T, 64>(nx, ny)) f(std::integral_constant<int, 64>{});
+    else if (plane_fits<T, 0>(nx, ny)) f(std::integral_constant<int, 0>{});
+    else return false;
+    return true;
+}
+
 // f(constant N) with the compile-time plan's length, 0 for a runtime plan
 template <class F>
 auto with_plan(int n, const F& f)
 {
     switch (n) {
+    case 32: return f(std::integral_constant<int, 32>{});
     case 48: return f(std::integral_constant<int, 48>{});
     case 64: return f(std::integral_constant<int, 64>{});
     case 80: return f(std::integral_constant<int, 80>{});
@@ -1112,11 +1321,18 @@ hipError_t poisson_t(const PoissonGroup& g, hipStream_t st)
         if (e != hipSuccess) g_failed_pass = pass;
         return e;
     };
-    hipError_t ec;
-    if ((ec = x_pass(false)) != hipSuccess) return ec;
-    if ((ec = check("forward x transform")) != hipSuccess) return ec;
-    if ((ec = y_pass(false)) != hipSuccess) return ec;
-    if ((ec = check("forward y transform")) != hipSuccess) return ec;
+    hipError_t ec = hipSuccess;
+    auto plane_pass = [&](bool inverse) {
+        return with_plane<T>(nx, ny, [&](auto n) { ec = launch_plane<T, decltype(n)::value>(g, inverse, st); });
+    };
+    if (plane_pass(false)) {
+        if (ec != hipSuccess || (ec = check("forward x and y transforms")) != hipSuccess) return ec;
+    } else {
+        if ((ec = x_pass(false)) != hipSuccess) return ec;
+        if ((ec = check("forward x transform")) != hipSuccess) return ec;
+        if ((ec = y_pass(false)) != hipSuccess) return ec;
+        if ((ec = check("forward y transform")) != hipSuccess) return ec;
+    }
 
     const int nmodes = nxh * ny;
     const int Pz = zsolve_partition(nmax, cs);
@@ -1145,13 +1361,13 @@ hipError_t poisson_t(const PoissonGroup& g, hipStream_t st)
     if (ez != hipSuccess) return ez;
     if ((ec = check("z solve")) != hipSuccess) return ec;
 
-    if ((ec = y_pass(true)) != hipSuccess) return ec;
-    if ((ec = check("inverse y transform")) != hipSuccess) return ec;
-    if ((ec = x_pass(true)) != hipSuccess) return ec;
-    if ((ec = check("inverse x transform")) != hipSuccess) return ec;
-    if (!sm) {
-        phi_walls_kernel<<<dim3((nx * ny + 255) / 256, g.njobs), 256, 0, st>>>(g.jobs, nx * ny);
-        if ((ec = check("wall potential")) != hipSuccess) return ec;
+    if (plane_pass(true)) {
+        if (ec != hipSuccess || (ec = check("inverse y and x transforms")) != hipSuccess) return ec;
+    } else {
+        if ((ec = y_pass(true)) != hipSuccess) return ec;
+        if ((ec = check("inverse y transform")) != hipSuccess) return ec;
+        if ((ec = x_pass(true)) != hipSuccess) return ec;
+        if ((ec = check("inverse x transform")) != hipSuccess) return ec;
     }
     return hipGetLastError();
 }

@@ -288,7 +288,9 @@ def test_poisson_vs_oracle(shape, precision):
 # stage alone, first and second (17, 61, 17 * 19), one side planned at compile
 # time and the other not, a last block of rows that is not full, one row pair.
 @pytest.mark.parametrize("shape", [(122, 122, 9), (34, 4, 6), (646, 2, 5), (64, 34, 7), (90, 154, 6), (18, 26, 11),
-                                   (22, 98, 8), (112, 48, 5), (2, 14, 12), (200, 36, 6)])
+                                   (22, 98, 8), (112, 48, 5), (2, 14, 12), (200, 36, 6),
+                                   # planes on both sides of the one-launch transforms' limit, and their plans
+                                   (62, 66, 6), (64, 66, 6), (32, 32, 9), (32, 128, 5), (32, 130, 5)])
 @pytest.mark.parametrize("precision", [E.FP64, E.FP32S])
 def test_poisson_runtime_plans_vs_oracle(shape, precision):
     test_poisson_vs_oracle(shape, precision)
