@@ -12,19 +12,9 @@
 #include <vector>
 
 #include "box.h"
-#include "fft_plan.h"
 #include "host_copy.h"
 
 using namespace ehd;
-
-namespace {
-
-
-
-constexpr double kPi = 3.14159265358979323846;
-
-}  // namespace
-
 
 namespace {
 
@@ -112,17 +102,6 @@ void fill_lbm_params(ehd_box* b)
     }
     L.dx = d.dx; L.dy = d.dy; L.dz = d.dz;
     L.rs = nullptr; L.qs = nullptr; L.shf = nullptr; L.qs0 = 0.0;
-}
-
-template <typename T>
-void make_twiddles(int n, std::vector<T>& out)
-{
-    out.resize(2 * (size_t)n);
-    for (int j = 0; j < n; ++j) {
-        const double a = 2.0 * kPi * (double)j / (double)n;
-        out[2 * j] = (T)std::cos(a);
-        out[2 * j + 1] = (T)(-std::sin(a));
-    }
 }
 
 int alloc(void** p, size_t bytes)
@@ -564,21 +543,6 @@ int ehd_create(const ehd_params* p, ehd_box** out)
         b->lp.shf = b->shift_f;
         b->lp.qs0 = qs[0];
     }
-    if (b->prec == Prec::F64) {
-        std::vector<double> tx, ty;
-        make_twiddles(b->nx, tx);
-        make_twiddles(b->ny, ty);
-        if (hipMemcpy(b->twx, tx.data(), tx.size() * 8, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(b->twy, ty.data(), ty.size() * 8, hipMemcpyHostToDevice) != hipSuccess)
-            return bail(set_error(EHD_EHIP, "twiddle upload failed"));
-    } else {
-        std::vector<float> tx, ty;
-        make_twiddles(b->nx, tx);
-        make_twiddles(b->ny, ty);
-        if (hipMemcpy(b->twx, tx.data(), tx.size() * 4, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(b->twy, ty.data(), ty.size() * 4, hipMemcpyHostToDevice) != hipSuccess)
-            return bail(set_error(EHD_EHIP, "twiddle upload failed"));
-    }
     {
         const PoissonShape ps = poisson_shape(b->prec, b->nx, b->ny, b->nz);
         if (ps.max_x_lines == 0 || ps.max_y_lines == 0 || ps.zs_partition == 0)
@@ -588,8 +552,9 @@ int ehd_create(const ehd_params* p, ehd_box** out)
         const PoissonJob job = make_poisson_job(b->lp, pb, b->q, b->phi, p->voltage, p->eps);
         if ((rc = alloc((void**)&b->pjob, sizeof(PoissonJob)))) return bail(rc);
         b->pjob_h = job;
-        if (hipMemcpy(b->pjob, &job, sizeof(job), hipMemcpyHostToDevice) != hipSuccess)
-            return bail(set_error(EHD_EHIP, "Poisson job upload failed"));
+        if (launch_poisson_setup(b->prec, job, b->pjob, b->twx, b->nx, b->twy, b->ny, b->st) != hipSuccess ||
+            hipStreamSynchronize(b->st) != hipSuccess)   // a batch reads the tables on streams of its own
+            return bail(set_error(EHD_EHIP, "Poisson tables failed"));
     }
     if (b->prec == Prec::F32S) {
         // one-item tables of the FP32S kernel, one per buffer parity

@@ -142,6 +142,9 @@ struct PoissonShape {
 PoissonJob make_poisson_job(const LbmParams& P, const PoissonBufs& pb, const void* q, void* phi, double voltage,
                             double eps);
 PoissonShape poisson_shape(Prec prec, int nx, int ny, int nz);
+// writes the job table *dst and the twiddle tables of nx and ny (path type) on the device
+hipError_t launch_poisson_setup(Prec prec, const PoissonJob& job, PoissonJob* dst, void* twx, int nx, void* twy, int ny,
+                                hipStream_t st);
 hipError_t launch_poisson_group(Prec prec, const PoissonGroup& g, hipStream_t st);
 
 // --- diagnostics (diag.hip) --------------------------------------------------

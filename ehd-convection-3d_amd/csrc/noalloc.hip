@@ -13,10 +13,7 @@
 // returns after its stream has finished the solve.
 #include <hip/hip_runtime.h>
 
-#include <cmath>
-#include <cstring>
 #include <mutex>
-#include <vector>
 
 #include "box.h"
 
@@ -78,27 +75,15 @@ extern "C" int ehd_poisson_noalloc(const ehd_params* p, const double* q, double*
     unsigned char* s = (unsigned char*)base;
     hipStream_t st = (hipStream_t)stream;
 
-    // twiddles and the job, as ehd_create builds them for a box
-    std::vector<double> tw(2 * (size_t)(nx > ny ? nx : ny));
-    auto twiddles = [&](int n) {
-        for (int j = 0; j < n; ++j) {
-            const double a = 2.0 * 3.14159265358979323846 * (double)j / (double)n;
-            tw[2 * j] = std::cos(a);
-            tw[2 * j + 1] = -std::sin(a);
-        }
-    };
     ehd::LbmParams L{};
     L.dx = d.dx;
     L.dy = d.dy;
     L.dz = d.dz;
     const ehd::PoissonBufs pb{nx, ny, nz, nxh, s + o_spec, s + o_twx, s + o_twy, nullptr};
     const ehd::PoissonJob job = ehd::make_poisson_job(L, pb, q, phi, p->voltage, p->eps);
-    HIPCHK(hipMemcpyAsync(s + o_job, &job, sizeof(job), hipMemcpyHostToDevice, st));
-    twiddles(nx);
-    HIPCHK(hipMemcpyAsync(s + o_twx, tw.data(), 16 * (size_t)nx, hipMemcpyHostToDevice, st));
-    HIPCHK(hipStreamSynchronize(st));   // the host tables are reused below
-    twiddles(ny);
-    HIPCHK(hipMemcpyAsync(s + o_twy, tw.data(), 16 * (size_t)ny, hipMemcpyHostToDevice, st));
+    // the job and the twiddles, as ehd_create makes them for a box
+    HIPCHK(ehd::launch_poisson_setup(ehd::Prec::F64, job, (ehd::PoissonJob*)(s + o_job), s + o_twx, nx, s + o_twy, ny,
+                                     st));
 
     ehd::PoissonGroup g{};
     g.nx = nx;
