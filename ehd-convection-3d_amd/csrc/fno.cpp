@@ -68,6 +68,9 @@ struct ehd_fno {
     Cbuf Vz, Vy, Ym, Wx, Wy;      // spectral temporaries (reused by the backward pass)
     float *dv0 = nullptr, *dv1 = nullptr, *dh = nullptr;
     double* part = nullptr;
+    bool head = false;            // the projection's own kernels (head_fits): no h and dh
+    float* quads = nullptr;       // sums of four points of the hidden gradient
+    float* wscr2 = nullptr;       // split-K partial sums of the projection's second weight gradient
     float* wscr = nullptr;        // split-K partial sums of the weight gradients
     float* red = nullptr;         // partial sums of sum_slices and channel_sum
     long long wscr_n = 0;
@@ -201,6 +204,30 @@ void mix_work(ehd_fno* f, int B, int n)
     const double w = f->c.width, spec = 2.0 * B * w * f->NM, weights = 2.0 * w * w * f->NM;
     f->work.flops += 8.0 * B * w * w * f->NM * n;
     f->work.bytes += 4.0 * (n * weights + (n + 1) * spec);
+    f->work.launches += 1;
+}
+
+// the projection's operands, checked like the GEMMs'
+bool head_operands(const ehd_fno* f, int B, std::initializer_list<const float*> inputs,
+                   std::initializer_list<const float*> outputs)
+{
+    const long long w = f->c.width, H = f->c.d_hidden, O = f->c.d_out;
+    for (const float* p : inputs)
+        if (!in_range(f, p, B * w * f->ZP - 1)) return false;
+    for (const float* p : outputs)
+        if (!in_range(f, p, B * O * f->ZP - 1)) return false;
+    return in_range(f, f->z1, B * H * f->ZP - 1) && in_range(f, f->p + f->oQ1w, w * H - 1) &&
+           in_range(f, f->p + f->oQ1b, H - 1) && in_range(f, f->p + f->oQ2w, H * O - 1) &&
+           in_range(f, f->p + f->oQ2b, O - 1);
+}
+
+// n products with each of the projection's two weights in one launch; rows
+// floats per point read and written
+void head_work(ehd_fno* f, int B, int n, int rows)
+{
+    const double w = f->c.width, H = f->c.d_hidden, O = f->c.d_out, points = (double)B * f->ZP;
+    f->work.flops += 2.0 * H * (w + O) * points * n;
+    f->work.bytes += 4.0 * (rows * points + n * H * (w + O));
     f->work.launches += 1;
 }
 
@@ -527,9 +554,10 @@ int spectral_bwd(ehd_fno* f, int l, int B, const float* du, float* dv, float bet
     return EHD_OK;
 }
 
-int forward(ehd_fno* f, int B)
+// keep: the values the backward pass needs are kept
+int forward(ehd_fno* f, int B, bool keep)
 {
-    const int w = f->c.width, L = f->c.layers;
+    const int w = f->c.width, L = f->c.layers, H = f->c.d_hidden, O = f->c.d_out;
     int rc;
     // each layer's bias and GELU run in the epilogue of the GEMM that completes its sum
     Epi ep;
@@ -545,14 +573,21 @@ int forward(ehd_fno* f, int B)
         }
         if ((rc = pointwise(f, B, w, w, f->p + f->oW[l], f->v[l], f->v[l + 1], 1.f, el))) return rc;
     }
+    if (f->head) {
+        if (!head_operands(f, B, {f->v[L]}, {f->out})) return set_error(EHD_EINVAL, "projection operands");
+        head_work(f, B, 1, w + O + (keep ? H : 0));
+        FCHK(head_forward(w, B, O, f->ZP, f->v[L], f->p + f->oQ1w, f->p + f->oQ1b, f->p + f->oQ2w, f->p + f->oQ2b,
+                          keep ? f->z1 : nullptr, f->out, f->st));
+        return EHD_OK;
+    }
     Epi eq1;
     eq1.bias = f->p + f->oQ1b;
     eq1.act = kActGelu;
     eq1.pre = f->z1;
-    if ((rc = pointwise(f, B, w, f->c.d_hidden, f->p + f->oQ1w, f->v[L], f->h, 0.f, eq1))) return rc;
+    if ((rc = pointwise(f, B, w, H, f->p + f->oQ1w, f->v[L], f->h, 0.f, eq1))) return rc;
     Epi eq2;
     eq2.bias = f->p + f->oQ2b;
-    if ((rc = pointwise(f, B, f->c.d_hidden, f->c.d_out, f->p + f->oQ2w, f->h, f->out, 0.f, eq2))) return rc;
+    if ((rc = pointwise(f, B, H, O, f->p + f->oQ2w, f->h, f->out, 0.f, eq2))) return rc;
     return EHD_OK;
 }
 
@@ -562,14 +597,28 @@ int backward(ehd_fno* f, int B)
     const int w = f->c.width, L = f->c.layers, H = f->c.d_hidden, O = f->c.d_out;
     const long long ZP = f->ZP;
     int rc;
-    if ((rc = pointwise_dw(f, B, H, O, f->h, f->dout, f->g + f->oQ2w))) return rc;
-    FCHK(channel_sum(f->dout, f->g + f->oQ2b, B, O, ZP, false, f->red, f->st));
-    if ((rc = pointwise_dx(f, B, H, O, f->p + f->oQ2w, f->dout, f->dh, 0.f, f->z1))) return rc;
-    if ((rc = pointwise_dw(f, B, w, H, f->v[L], f->dh, f->g + f->oQ1w))) return rc;
-    FCHK(channel_sum(f->dh, f->g + f->oQ1b, B, H, ZP, false, f->red, f->st));
     float* dv = f->dv0;
     float* dn = f->dv1;
-    if ((rc = pointwise_dx(f, B, w, H, f->p + f->oQ1w, f->dh, dv, 0.f))) return rc;
+    FCHK(channel_sum(f->dout, f->g + f->oQ2b, B, O, ZP, false, f->red, f->st));
+    if (f->head) {
+        const long long ns = (long long)B * f->nsplit, n1 = (long long)w * H, n2 = (long long)H * O;
+        if (!head_operands(f, B, {f->v[L], dv}, {f->dout}) || f->nsplit != head_slices(ZP) ||
+            !in_range(f, f->wscr, ns * n1 - 1) || !in_range(f, f->wscr2, ns * n2 - 1) ||
+            !in_range(f, f->quads, B * H * (ZP / 4) - 1))
+            return set_error(EHD_EINVAL, "projection operands");
+        head_work(f, B, 2, 2 * w + 2 * O + H + H / 4);
+        FCHK(head_backward(w, B, O, ZP, f->v[L], f->z1, f->dout, f->p + f->oQ1w, f->p + f->oQ2w, dv, f->wscr, f->wscr2,
+                           f->quads, f->st));
+        FCHK(sum_slices(f->wscr, f->g + f->oQ1w, n1, (int)ns, 0.f, f->red, f->st));
+        FCHK(sum_slices(f->wscr2, f->g + f->oQ2w, n2, (int)ns, 0.f, f->red, f->st));
+        FCHK(channel_sum_quads(f->quads, f->g + f->oQ1b, B, H, ZP, f->red, f->st));
+    } else {
+        if ((rc = pointwise_dw(f, B, H, O, f->h, f->dout, f->g + f->oQ2w))) return rc;
+        if ((rc = pointwise_dx(f, B, H, O, f->p + f->oQ2w, f->dout, f->dh, 0.f, f->z1))) return rc;
+        if ((rc = pointwise_dw(f, B, w, H, f->v[L], f->dh, f->g + f->oQ1w))) return rc;
+        FCHK(channel_sum(f->dh, f->g + f->oQ1b, B, H, ZP, false, f->red, f->st));
+        if ((rc = pointwise_dx(f, B, w, H, f->p + f->oQ1w, f->dh, dv, 0.f))) return rc;
+    }
     // dv enters iteration l as the gradient of layer l's pre-activation: the
     // input gradient of layer l + 1 leaves its GEMM times gelu'(u[l])
     for (int l = L - 1; l >= 0; --l) {
@@ -597,7 +646,7 @@ int loss_and_grad(ehd_fno* f, int B, const float* in, const float* target, doubl
     } else if (B > f->resident) {
         return set_error(EHD_EINVAL, "no resident batch of %d samples (last loaded: %d)", B, f->resident);
     }
-    int rc = forward(f, B);
+    int rc = forward(f, B, true);
     if (rc) return rc;
     FCHK(mse(f->out, f->tgt, f->dout, f->part, nout, f->st));
     if ((rc = backward(f, B))) return rc;
@@ -674,10 +723,13 @@ int ehd_fno_create(const ehd_fno_config* cfg, ehd_fno** out)
     const long long sp_z = B * w * f->KZ * f->P, sp_y = B * w * f->KZ * f->KY * c.X, sp_m = B * w * f->NM;
     if ((rc = falloc(f, &f->p, o)) || (rc = falloc(f, &f->g, o)) || (rc = falloc(f, &f->m1, o)) ||
         (rc = falloc(f, &f->m2, o)) || (rc = falloc(f, &f->in, B * c.d_in * f->ZP)) ||
-        (rc = falloc(f, &f->z1, B * c.d_hidden * f->ZP)) || (rc = falloc(f, &f->h, B * c.d_hidden * f->ZP)) ||
-        (rc = falloc(f, &f->dh, B * c.d_hidden * f->ZP)) || (rc = falloc(f, &f->out, B * c.d_out * f->ZP)) ||
+        (rc = falloc(f, &f->z1, B * c.d_hidden * f->ZP)) || (rc = falloc(f, &f->out, B * c.d_out * f->ZP)) ||
         (rc = falloc(f, &f->tgt, B * c.d_out * f->ZP)) || (rc = falloc(f, &f->dout, B * c.d_out * f->ZP)) ||
         (rc = falloc(f, &f->dv0, act)) || (rc = falloc(f, &f->dv1, act)))
+        return bail(rc);
+    f->head = head_fits(c.width, c.d_hidden, c.d_out, f->ZP);
+    if (f->head ? (rc = falloc(f, &f->quads, B * c.d_hidden * (f->ZP / 4)))
+                : (rc = falloc(f, &f->h, B * c.d_hidden * f->ZP)) || (rc = falloc(f, &f->dh, B * c.d_hidden * f->ZP)))
         return bail(rc);
     f->v.assign(c.layers + 1, nullptr);
     for (auto& p : f->v)
@@ -701,6 +753,7 @@ int ehd_fno_create(const ehd_fno_config* cfg, ehd_fno** out)
                                                     (long long)c.d_hidden * c.d_out});
         f->wscr_n = B * f->nsplit * wmax;
         if ((rc = falloc(f, &f->wscr, f->wscr_n))) return bail(rc);
+        if (f->head && (rc = falloc(f, &f->wscr2, B * f->nsplit * c.d_hidden * c.d_out))) return bail(rc);
         const int cmax = std::max({c.width, c.d_hidden, c.d_out});
         const long long nred = std::max(sum_slices_part_floats(wmax), channel_sum_part_floats((int)B, cmax, f->ZP));
         if ((rc = falloc(f, &f->red, nred))) return bail(rc);
@@ -753,7 +806,7 @@ int ehd_fno_forward(ehd_fno* f, int batch, const float* in, float* out)
     if (rc) return rc;
     HIPCHK(hipMemcpyAsync(f->in, in, (size_t)batch * f->c.d_in * f->ZP * sizeof(float), hipMemcpyHostToDevice, f->st));
     f->resident = 0;   // the inputs no longer match the resident targets
-    if ((rc = forward(f, batch))) return rc;
+    if ((rc = forward(f, batch, false))) return rc;
     return download_floats(f, out, f->out, (size_t)batch * f->c.d_out * f->ZP);
 }
 

@@ -55,6 +55,20 @@ hipError_t mix_forward(int w, int B, int NM, const float* Sr, const float* Si, c
                        float* Yr, float* Yi, hipStream_t st);
 hipError_t mix_backward(int w, int B, int NM, float* Sr, float* Si, const float* Gr, const float* Gi, const float* Rr,
                         const float* Ri, float* dRr, float* dRi, hipStream_t st);
+// The projection width -> hidden -> d_out of a prediction and its backward
+// pass (fno_head.hip), bit-identical to the pointwise GEMMs: shapes for which
+// head_fits holds, S points a sample, weights [c][h] and [h][o], biases b1, b2.
+//   forward:  z1[b][h] = b1 + W1 v (stored unless z1 is null), out = b2 + W2 gelu(z1)
+//   backward: dv[b][c], the partial sums dW1[slice][c][h] and dW2[slice][h][o] of
+//             B head_slices(S) slices, and quads[b][h][S/4], the sums of four
+//             consecutive points of the hidden layer's gradient
+bool head_fits(int w, int hidden, int O, long long S);
+int head_slices(long long S);
+hipError_t head_forward(int w, int B, int O, long long S, const float* v, const float* W1, const float* b1,
+                        const float* W2, const float* b2, float* z1, float* out, hipStream_t st);
+hipError_t head_backward(int w, int B, int O, long long S, const float* v, const float* z1, const float* dout,
+                         const float* W1, const float* W2, float* dv, float* dW1, float* dW2, float* quads,
+                         hipStream_t st);
 // staging layout gemm_bf16 picks for A and B: 0 k unit-stride, 1 m (n) unit-stride
 // (16-byte loads), 2 element loads
 int gemm_layout_a(const GemmArgs& g);
@@ -70,6 +84,8 @@ hipError_t sum_slices(const float* src, float* dst, long long n, int nslices, fl
 long long channel_sum_part_floats(int B, int C, long long S);
 hipError_t channel_sum(const float* g, float* db, int B, int C, long long S, bool accumulate, float* part,
                        hipStream_t st);
+// the same sums of g from the sums of its quads, quads[b][c][S/4] (S a multiple of 4), to the last bit
+hipError_t channel_sum_quads(const float* quads, float* db, int B, int C, long long S, float* part, hipStream_t st);
 // grad = 2 (out - tgt) / n, part[mse_blocks()] = partial sums of (out - tgt)^2
 int mse_blocks();
 hipError_t mse(const float* out, const float* tgt, float* grad, double* part, long long n, hipStream_t st);

@@ -438,17 +438,21 @@ __device__ __forceinline__ float block_sum_256(float s, float* red)
     return red[0];
 }
 
-// part[row][chunk] = sum of g[row][chunk*kRowChunk ...) for the rows (b, c)
-template <bool VEC>
+// part[row][chunk] = sum of g[row][chunk*kRowChunk ...) for the rows (b, c): element loads, quads
+// where the rows allow it (the sum of a quad first), or those quads' sums as given
+constexpr int kElements = 0, kQuads = 1, kQuadSums = 2;
+template <int FROM>
 __global__ void __launch_bounds__(256) row_chunk_sum_kernel(const float* __restrict__ g, float* __restrict__ part,
                                                             long long S, int nchunk)
 {
     __shared__ float red[256];
     const long long row = blockIdx.y;
-    const float* __restrict__ p = g + row * S;
+    const float* __restrict__ p = g + row * (FROM == kQuadSums ? S / 4 : S);
     const long long s0 = (long long)blockIdx.x * kRowChunk, s1 = min(S, s0 + kRowChunk);
     float s = 0.f;
-    if constexpr (VEC) {
+    if constexpr (FROM == kQuadSums) {
+        for (long long i = s0 / 4 + threadIdx.x; i < s1 / 4; i += 256) s += p[i];
+    } else if constexpr (FROM == kQuads) {
         for (long long i = s0 + 4 * threadIdx.x; i < s1; i += 1024) {
             const float4 v = *(const float4*)(p + i);
             s += (v.x + v.y) + (v.z + v.w);
@@ -645,10 +649,20 @@ hipError_t channel_sum(const float* g, float* db, int B, int C, long long S, boo
     const int nchunk = (int)((S + kRowChunk - 1) / kRowChunk);
     const dim3 grid((unsigned)nchunk, (unsigned)rows);
     if (S % 4 == 0 && (uintptr_t)g % 16 == 0)
-        row_chunk_sum_kernel<true><<<grid, 256, 0, st>>>(g, part, S, nchunk);
+        row_chunk_sum_kernel<kQuads><<<grid, 256, 0, st>>>(g, part, S, nchunk);
     else
-        row_chunk_sum_kernel<false><<<grid, 256, 0, st>>>(g, part, S, nchunk);
+        row_chunk_sum_kernel<kElements><<<grid, 256, 0, st>>>(g, part, S, nchunk);
     channel_total_kernel<<<C, 256, 0, st>>>(part, db, B, C, nchunk, accumulate ? 1 : 0);
+    return hipGetLastError();
+}
+
+hipError_t channel_sum_quads(const float* quads, float* db, int B, int C, long long S, float* part, hipStream_t st)
+{
+    const long long rows = (long long)B * C;
+    if (rows <= 0 || rows > 65535 || S <= 0 || S % 4 != 0) return hipErrorInvalidValue;
+    const int nchunk = (int)((S + kRowChunk - 1) / kRowChunk);
+    row_chunk_sum_kernel<kQuadSums><<<dim3((unsigned)nchunk, (unsigned)rows), 256, 0, st>>>(quads, part, S, nchunk);
+    channel_total_kernel<<<C, 256, 0, st>>>(part, db, B, C, nchunk, 0);
     return hipGetLastError();
 }
 

@@ -281,6 +281,40 @@ def test_gradients_of_every_width_and_batch_path_match_oracle(width, batch):
     assert max(errs.values()) < 5e-2, errs
 
 
+# A projection of 128 hidden channels takes kernels of its own; with 32 more channels
+# whose weights are zero it goes through the pointwise GEMMs, and adds only zeros: outputs,
+# loss and every gradient are the same bit for bit.  Points: 20 beyond the last
+# whole tile of 32; two slices of 2048, the second part full; ragged in both.
+@pytest.mark.parametrize("grid", [(6, 6, 5), (16, 16, 10), (18, 14, 9)])
+@pytest.mark.parametrize("width,d_out", [(16, 1), (32, 2), (16, 8), (32, 5)])
+def test_projection_matches_the_pointwise_gemms_bitwise(grid, width, d_out):
+    cfg = F.FNOConfig(X=grid[0], Y=grid[1], Z=grid[2], width=width, modes=(2, 3, 2), layers=2, d_in=3, d_hidden=128,
+                      d_out=d_out)
+    rng = np.random.default_rng(17)
+    p = F.init_params(cfg, seed=17)
+    for k in ("Q1b", "Q2b"):
+        p[k] = 0.3 * rng.standard_normal(p[k].shape)
+    wide = dict(p)
+    wide["Q1w"] = np.concatenate([p["Q1w"], np.zeros((width, 32))], axis=1)
+    wide["Q1b"] = np.concatenate([p["Q1b"], np.zeros(32)])
+    wide["Q2w"] = np.concatenate([p["Q2w"], np.zeros((32, d_out))], axis=0)
+    a = rng.standard_normal((3, 3, cfg.Z, cfg.Y, cfg.X)).astype(np.float32)
+    t = rng.standard_normal((3, d_out, cfg.Z, cfg.Y, cfg.X)).astype(np.float32)
+    res = []
+    for hidden, q in ((128, p), (160, wide)):
+        net = G.FNO(cfg.X, cfg.Y, cfg.Z, width=width, modes=cfg.modes, layers=2, d_in=3, d_hidden=hidden, d_out=d_out,
+                    max_batch=3)
+        net.set_params(q)
+        loss, g = net.gradients(a, t)
+        res.append((net.forward(a), loss, G.unflatten(net.cfg, g)))
+        net.close()
+    (out, loss, g), (out_w, loss_w, g_w) = res
+    assert np.array_equal(out, out_w) and loss == loss_w
+    g_w["Q1w"], g_w["Q1b"], g_w["Q2w"] = g_w["Q1w"][:, :128], g_w["Q1b"][:128], g_w["Q2w"][:128]
+    for k in g:
+        assert np.all(np.isfinite(g[k])) and np.array_equal(g[k], g_w[k]), k
+
+
 def test_adam_steps_reduce_loss():
     p, a, t, net = _setup(seed=2)
     losses = [net.train_step(a, t, 3e-3) for _ in range(30)]
