@@ -8,17 +8,20 @@
 namespace ehd {
 namespace {
 
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ uint32_t to_bf16(float f)
+// rounded to nearest even, two to a conversion instruction
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi)
 {
-    uint32_t u = __float_as_uint(f);
-    u += 0x7FFFu + ((u >> 16) & 1u);   // round to nearest even (finite inputs)
-    return u >> 16;
+    const bf16x2 v = {(__bf16)lo, (__bf16)hi};
+    uint32_t u;
+    __builtin_memcpy(&u, &v, 4);
+    return u;
 }
 
-__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) { return to_bf16(lo) | (to_bf16(hi) << 16); }
+__device__ __forceinline__ uint32_t to_bf16(float f) { return pack_bf16(f, 0.f) & 0xFFFFu; }
 
 // GELU with the exact (erf) form, and its derivative
 __device__ __forceinline__ float gelu(float v) { return 0.5f * v * (1.0f + erff(v * 0.70710678118654752f)); }
