@@ -216,7 +216,7 @@ bool head_operands(const ehd_fno* f, int B, std::initializer_list<const float*> 
         if (!in_range(f, p, B * w * f->ZP - 1)) return false;
     for (const float* p : outputs)
         if (!in_range(f, p, B * O * f->ZP - 1)) return false;
-    return in_range(f, f->z1, B * H * f->ZP - 1) && in_range(f, f->p + f->oQ1w, w * H - 1) &&
+    return in_range(f, f->z1, B * H * head_points(f->ZP) - 1) && in_range(f, f->p + f->oQ1w, w * H - 1) &&
            in_range(f, f->p + f->oQ1b, H - 1) && in_range(f, f->p + f->oQ2w, H * O - 1) &&
            in_range(f, f->p + f->oQ2b, O - 1);
 }
@@ -604,7 +604,7 @@ int backward(ehd_fno* f, int B)
         const long long ns = (long long)B * f->nsplit, n1 = (long long)w * H, n2 = (long long)H * O;
         if (!head_operands(f, B, {f->v[L], dv}, {f->dout}) || f->nsplit != head_slices(ZP) ||
             !in_range(f, f->wscr, ns * n1 - 1) || !in_range(f, f->wscr2, ns * n2 - 1) ||
-            !in_range(f, f->quads, B * H * (ZP / 4) - 1))
+            !in_range(f, f->quads, B * H * (head_points(ZP) / 4) - 1))
             return set_error(EHD_EINVAL, "projection operands");
         head_work(f, B, 2, 2 * w + 2 * O + H + H / 4);
         FCHK(head_backward(w, B, O, ZP, f->v[L], f->z1, f->dout, f->p + f->oQ1w, f->p + f->oQ2w, dv, f->wscr, f->wscr2,
@@ -723,12 +723,12 @@ int ehd_fno_create(const ehd_fno_config* cfg, ehd_fno** out)
     const long long sp_z = B * w * f->KZ * f->P, sp_y = B * w * f->KZ * f->KY * c.X, sp_m = B * w * f->NM;
     if ((rc = falloc(f, &f->p, o)) || (rc = falloc(f, &f->g, o)) || (rc = falloc(f, &f->m1, o)) ||
         (rc = falloc(f, &f->m2, o)) || (rc = falloc(f, &f->in, B * c.d_in * f->ZP)) ||
-        (rc = falloc(f, &f->z1, B * c.d_hidden * f->ZP)) || (rc = falloc(f, &f->out, B * c.d_out * f->ZP)) ||
+        (rc = falloc(f, &f->z1, B * c.d_hidden * head_points(f->ZP))) || (rc = falloc(f, &f->out, B * c.d_out * f->ZP)) ||
         (rc = falloc(f, &f->tgt, B * c.d_out * f->ZP)) || (rc = falloc(f, &f->dout, B * c.d_out * f->ZP)) ||
         (rc = falloc(f, &f->dv0, act)) || (rc = falloc(f, &f->dv1, act)))
         return bail(rc);
     f->head = head_fits(c.width, c.d_hidden, c.d_out, f->ZP);
-    if (f->head ? (rc = falloc(f, &f->quads, B * c.d_hidden * (f->ZP / 4)))
+    if (f->head ? (rc = falloc(f, &f->quads, B * c.d_hidden * (head_points(f->ZP) / 4)))
                 : (rc = falloc(f, &f->h, B * c.d_hidden * f->ZP)) || (rc = falloc(f, &f->dh, B * c.d_hidden * f->ZP)))
         return bail(rc);
     f->v.assign(c.layers + 1, nullptr);

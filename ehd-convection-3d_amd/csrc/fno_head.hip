@@ -16,8 +16,10 @@
 // input channels; 128 hidden in four steps; d_out; 32 consecutive points of a
 // slice of 2048), operands rounded to bf16 where the GEMMs staged them, FP32
 // epilogues.  At 8 samples of 64x64x64 points, width 32, 2.0 ms of GEMMs and
-// sums became 0.37 ms forward and 1.07 backward (0.08 for a prediction of 4).
+// sums became 0.28 ms forward and 0.57 backward (0.08 for a prediction of 4).
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "fno_device.h"
 #include "fno_internal.h"
@@ -48,10 +50,10 @@ __device__ __forceinline__ bf16x8 operand(const unsigned short* p)
 
 // the sum of a quad as a sum over stored values forms it: no product of its
 // terms is fused into the additions
-__device__ __forceinline__ float quad_total(float4 d)
+__device__ __forceinline__ float quad_total(const float* d)
 {
 #pragma clang fp contract(off)
-    return (d.x + d.y) + (d.z + d.w);
+    return (d[0] + d[1]) + (d[2] + d[3]);
 }
 
 // operand of row (column) m of M[m][k] at m*sm + k*sk, k = k0 .. k0 + 7: zero beyond rows x cols
@@ -67,7 +69,12 @@ __device__ __forceinline__ bf16x8 weights(const float* __restrict__ M, int m, in
 // A wave takes tiles of PT points in turn, points as rows and channels as
 // columns of the products, so that a lane holds four consecutive points of a
 // channel; the hidden channels turn around in the wave's piece of LDS.
-// KEEP: z1 is stored.
+// Row i of half ct of a tile is point 8 (i/4) + 4 ct + i%4: the four rows of a
+// lane in both halves are eight consecutive points.  KEEP: z1 is stored, tile
+// by tile in the order in which the lanes hold it, [tile][t][ct][lane][4].
+// (By channel, z1 was a page per channel for every 128 bytes: 0.35 against
+// 0.28 ms here and 1.04 against 0.87 in the backward kernel at 8 samples of
+// 64x64x64, width 32.)
 template <int WT, bool KEEP>
 __global__ void __launch_bounds__(256) head_fwd_kernel(const float* __restrict__ v, const float* __restrict__ W1,
                                                        const float* __restrict__ b1, const float* __restrict__ W2,
@@ -95,8 +102,8 @@ __global__ void __launch_bounds__(256) head_fwd_kernel(const float* __restrict__
         bf16x8 x[2];
 #pragma unroll
         for (int ct = 0; ct < 2; ++ct) {
-            // a row beyond the last point repeats it and is not stored
-            const long long p = p0 + ct * 16 + lj < S ? p0 + ct * 16 + lj : S - 1;
+            // a row beyond the last point repeats it; its output is not stored
+            const long long pr = p0 + 8 * (lj >> 2) + 4 * ct + (lj & 3), p = pr < S ? pr : S - 1;
             const float* row = v + ((long long)b * w + (8 * lg < w ? 8 * lg : 0)) * S + p;
             float f[8];
 #pragma unroll
@@ -112,14 +119,13 @@ __global__ void __launch_bounds__(256) head_fwd_kernel(const float* __restrict__
 #pragma unroll
             for (int ct = 0; ct < 2; ++ct) {
                 const f32x4 acc = mfma(x[ct], a1[t], f32x4{0.f, 0.f, 0.f, 0.f});
-                const long long p = p0 + ct * 16 + 4 * lg;
                 float4 z;
                 z.x = acc[0] + bias[t];
                 z.y = acc[1] + bias[t];
                 z.z = acc[2] + bias[t];
                 z.w = acc[3] + bias[t];
-                if (KEEP && p < S) *(float4*)(z1 + ((long long)b * H + t * 16 + lj) * S + p) = z;
-                unsigned short* q = Hw + (ct * 16 + 4 * lg) * HP + t * 16 + lj;
+                if (KEEP) *(float4*)(z1 + tile * (H * PT) + ((t * 2 + ct) * 64 + lane) * 4) = z;
+                unsigned short* q = Hw + (8 * lg + 4 * ct) * HP + t * 16 + lj;
                 q[0] = (unsigned short)to_bf16(gelu(z.x));
                 q[HP] = (unsigned short)to_bf16(gelu(z.y));
                 q[2 * HP] = (unsigned short)to_bf16(gelu(z.z));
@@ -144,10 +150,12 @@ __global__ void __launch_bounds__(256) head_fwd_kernel(const float* __restrict__
 //   dh[h][p] = (sum_o W2[h][o] dout[o][p]) gelu'(z1[h][p]),
 //   dv[c][p] = sum_h W1[c][h] dh[h][p],
 //   dW1[c][h] = sum_p v[c][p] dh[h][p], dW2[h][o] = sum_p gelu(z1[h][p]) dout[o][p] over the slice,
-//   quads[h][p/4] = the sums of four consecutive dh, for the bias gradient.
+//   quads[tile][h][PT/4] = the sums of four consecutive dh, for the bias gradient.
 // A wave has 32 hidden channels, their weights and gradients in registers,
 // and one of the tile's 16x16 pieces of dv, for which the waves exchange dh
-// (two buffers, one barrier a tile).
+// (two buffers, one barrier a tile).  With the forward kernel's order of the
+// points, dh and the activation lie in the lanes as the weight gradients'
+// products take them.
 template <int WT>
 __global__ void __launch_bounds__(256, 4)
 head_bwd_kernel(const float* __restrict__ v, const float* __restrict__ z1, const float* __restrict__ dout,
@@ -157,25 +165,26 @@ head_bwd_kernel(const float* __restrict__ v, const float* __restrict__ z1, const
 {
     constexpr int w = WT * 16;
     __shared__ __align__(16) unsigned short Ds[2][PT * HP];   // dh [point][hidden]
-    __shared__ __align__(16) unsigned short Ks[4][2 * 32 * QP];   // [wave][dh, activation][its hidden channel][point]
+    __shared__ __align__(16) unsigned short Ws[w * HP];       // W1 [c][hidden]
+    __shared__ __align__(16) unsigned short Xs[4][PT * 8];    // dout [wave][row of the products][channel]
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lj = lane & 15, lg = lane >> 4;
     const int h0 = wave * 32, dp = wave & 1, dc = wave >> 1;   // this wave's channels; its half and channel tile of dv
-    unsigned short* Kw = Ks[wave];
+    unsigned short* Xw = Xs[wave];
     const int b = blockIdx.x / nsplit;
     const int q0 = (blockIdx.x - b * nsplit) * SLICE;
     const int q1 = q0 + SLICE < S ? q0 + SLICE : S;   // a multiple of 4
     const float* vb = v + (long long)b * w * S;
     const float* ob = dout + (long long)b * O * S;
-    const float* zb = z1 + ((long long)b * H + h0) * S;
-    float* qb = quads + ((long long)b * H + h0) * (S / 4);
     float* db = dv + ((long long)b * w + dc * 16) * S;
     const unsigned row = (unsigned)lj * S;   // this lane's channel, in a tile of 16: 32 bits as S < 2^26
-    bf16x8 a2[2], a1[H / 32];
+    const unsigned rowo = lj < O ? row : 0;
+    for (int i = threadIdx.x; i < w * H / 2; i += 256) {
+        const float2 x = *(const float2*)(W1 + 2 * i);
+        *(uint32_t*)&Ws[(i / (H / 2)) * HP + 2 * (i % (H / 2))] = pack_bf16(x.x, x.y);
+    }
+    bf16x8 a2[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) a2[t] = weights(W2, h0 + t * 16 + lj, H, O, 8 * lg, O, 1);
-    if (dc < WT)
-#pragma unroll
-        for (int s = 0; s < H / 32; ++s) a1[s] = weights(W1, dc * 16 + lj, w, H, 32 * s + 8 * lg, H, 1);
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     f32x4 g1[WT][2], g2[2];
 #pragma unroll
@@ -184,86 +193,94 @@ head_bwd_kernel(const float* __restrict__ v, const float* __restrict__ z1, const
 #pragma unroll
         for (int c = 0; c < WT; ++c) g1[c][t] = zero;
     }
+    float4 z[2][2], xr[WT + 1][2];
+    const float* zt = z1 + ((long long)b * ((S + PT - 1) / PT) + q0 / PT) * (H * PT) + h0 * PT + lane * 4;
+    float* qt = quads + ((long long)b * ((S + PT - 1) / PT) + q0 / PT) * (H * PT / 4) + h0 * (PT / 4) +
+                lj * (PT / 4) + 2 * lg;
+    auto load_z = [&](int t) {
+        z[t][0] = *(const float4*)(zt + t * 512);
+        z[t][1] = *(const float4*)(zt + t * 512 + 256);
+    };
+    auto load_x = [&](int p0) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int q = p0 + 8 * lg + 4 * k, p = q < q1 ? q : q1 - 4;
+#pragma unroll
+            for (int c = 0; c < WT; ++c) xr[c][k] = *(const float4*)(vb + (long long)c * 16 * S + (row + p));
+            xr[WT][k] = *(const float4*)(ob + (rowo + p));
+        }
+    };
     int buf = 0;
     for (int p0 = q0; p0 < q1; p0 += PT, buf ^= 1) {
-        // rows of points: dout's channels of a point
-        bf16x8 xo[2];
-#pragma unroll
-        for (int ct = 0; ct < 2; ++ct) {
-            const int p = p0 + ct * 16 + lj;
-            const unsigned at = p < q1 ? p : q0;
-            float f[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                f[e] = 0.f;
-                if (e < O) f[e] = (ob + (long long)e * S)[at];
-                if (lg != 0 || p >= q1) f[e] = 0.f;
-            }
-            xo[ct] = to_bf16x8(f);
-        }
-        // eight consecutive points of a channel
-        auto points = [&](const float* x0, unsigned r, bool on) {
-            float f[8];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int p = p0 + 8 * lg + 4 * h;
-                const float4 x = (on && p < q1) ? *(const float4*)(x0 + (r + p)) : make_float4(0.f, 0.f, 0.f, 0.f);
-                f[4 * h] = x.x;
-                f[4 * h + 1] = x.y;
-                f[4 * h + 2] = x.z;
-                f[4 * h + 3] = x.w;
-            }
-            return to_bf16x8(f);
-        };
-        bf16x8 xv[WT];
-#pragma unroll
-        for (int c = 0; c < WT; ++c) xv[c] = points(vb + (long long)c * 16 * S, row, true);
-        const bf16x8 xk = points(ob, lj < O ? row : 0, lj < O);
+        load_x(p0);
+        load_z(0);
+        load_z(1);
         unsigned short* D = Ds[buf];
-        wave_exchange();   // the last tile's reads of Kw are done
-        // piece s: channel tile s/2, half s%2 of the points; rolled, so that
-        // one piece's error functions at a time take registers
-        auto zload = [&](int s) {
-            const int p = p0 + (s & 1) * 16 + 4 * lg;
-            return p < q1 ? *(const float4*)(zb + (long long)(s >> 1) * 16 * S + (row + p)) : make_float4(0.f, 0.f, 0.f, 0.f);
-        };
-        float4 zn = zload(0);
-#pragma unroll 1
-        for (int s = 0; s < 4; ++s) {
-            const float4 z = zn;
-            if (s < 3) zn = zload(s + 1);
-            const f32x4 acc = mfma((s & 1) ? xo[1] : xo[0], (s >> 1) ? a2[1] : a2[0], zero);
-            const int p = p0 + (s & 1) * 16 + 4 * lg;
-            float4 d;
-            d.x = acc[0] * gelu_grad(z.x);
-            d.y = acc[1] * gelu_grad(z.y);
-            d.z = acc[2] * gelu_grad(z.z);
-            d.w = acc[3] * gelu_grad(z.w);
-            if (p < q1) (qb + (long long)(s >> 1) * 16 * (S / 4))[(row + p) / 4] = quad_total(d);
-            else d = make_float4(0.f, 0.f, 0.f, 0.f);
-            const uint2 k = make_uint2(pack_bf16(d.x, d.y), pack_bf16(d.z, d.w));
-            const int ko = ((s >> 1) * 16 + lj) * QP + (s & 1) * 16 + 4 * lg;
-            *(uint2*)&Kw[ko] = k;
-            // beyond the slice z = 0 and so is gelu(z)
-            *(uint2*)&Kw[32 * QP + ko] = make_uint2(pack_bf16(gelu(z.x), gelu(z.y)), pack_bf16(gelu(z.z), gelu(z.w)));
-            unsigned short* q = D + ((s & 1) * 16 + 4 * lg) * HP + h0 + (s >> 1) * 16 + lj;
-            q[0] = (unsigned short)k.x;
-            q[HP] = (unsigned short)(k.x >> 16);
-            q[2 * HP] = (unsigned short)k.y;
-            q[3 * HP] = (unsigned short)(k.y >> 16);
+        if (p0 + PT > q1)   // points beyond the slice count as zeros
+#pragma unroll
+            for (int c = 0; c <= WT; ++c)
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+                    if (p0 + 8 * lg + 4 * k >= q1) xr[c][k] = make_float4(0.f, 0.f, 0.f, 0.f);
+        bf16x8 x[WT + 1];
+#pragma unroll
+        for (int c = 0; c <= WT; ++c) {
+            const float f[8] = {xr[c][0].x, xr[c][0].y, xr[c][0].z, xr[c][0].w,
+                                xr[c][1].x, xr[c][1].y, xr[c][1].z, xr[c][1].w};
+            x[c] = to_bf16x8(f);
         }
-        __syncthreads();
+        if (lj >= O) x[WT] = bf16x8{};
+        // dout turns from points to channels through LDS (loaded a second time by
+        // channel, 16 loads of a quarter of a wave: 0.87 against 0.57 ms): point 8 lg + 4 ct + i is row 16 ct + 4 lg + i of the products
+        wave_exchange();
+        if (lj < 8) {
+            unsigned short q[8];
+            __builtin_memcpy(q, &x[WT], 16);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) Xw[(16 * (e >> 2) + 4 * lg + (e & 3)) * 8 + lj] = q[e];
+        }
+        wave_exchange();
+        bf16x8 xo[2] = {};
+        if (lg == 0) {
+            xo[0] = operand(&Xw[lj * 8]);
+            xo[1] = operand(&Xw[(16 + lj) * 8]);
+        }
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            const bf16x8 x = operand(&Kw[(t * 16 + lj) * QP + 8 * lg]);
+            float d[8], h[8];
 #pragma unroll
-            for (int c = 0; c < WT; ++c) g1[c][t] = mfma(xv[c], x, g1[c][t]);
-            g2[t] = mfma(operand(&Kw[(32 + t * 16 + lj) * QP + 8 * lg]), xk, g2[t]);
+            for (int ct = 0; ct < 2; ++ct) {
+                const f32x4 acc = mfma(xo[ct], a2[t], zero);
+                const float zs[4] = {z[t][ct].x, z[t][ct].y, z[t][ct].z, z[t][ct].w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    d[4 * ct + e] = acc[e] * gelu_grad(zs[e]);
+                    h[4 * ct + e] = gelu(zs[e]);
+                }
+            }
+            if (p0 + PT > q1)
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (p0 + 8 * lg + (e & 4) >= q1) d[e] = h[e] = 0.f;
+            *(float2*)(qt + t * (16 * PT / 4)) = make_float2(quad_total(d), quad_total(d + 4));
+            const bf16x8 xd = to_bf16x8(d);
+            unsigned short q[8];
+            __builtin_memcpy(q, &xd, 16);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) D[(8 * lg + e) * HP + h0 + t * 16 + lj] = q[e];
+#pragma unroll
+            for (int c = 0; c < WT; ++c) g1[c][t] = mfma(x[c], xd, g1[c][t]);
+            g2[t] = mfma(to_bf16x8(h), x[WT], g2[t]);
         }
+        zt += H * PT;
+        qt += H * PT / 4;
+        __syncthreads();
         if (dc < WT) {
             f32x4 acc = zero;
 #pragma unroll
-            for (int s = 0; s < H / 32; ++s) acc = mfma(operand(&D[(dp * 16 + lj) * HP + 32 * s + 8 * lg]), a1[s], acc);
+            for (int s = 0; s < H / 32; ++s)
+                acc = mfma(operand(&D[(dp * 16 + lj) * HP + 32 * s + 8 * lg]),
+                           operand(&Ws[(dc * 16 + lj) * HP + 32 * s + 8 * lg]), acc);
             const int p = p0 + dp * 16 + 4 * lg;
             if (p < q1) *(float4*)(db + (row + p)) = make_float4(acc[0], acc[1], acc[2], acc[3]);
         }
@@ -299,6 +316,8 @@ hipError_t head_forward(int w, int B, int O, long long S, const float* v, const 
     kernel<<<grid, 256, 0, st>>>(v, W1, b1, W2, b2, z1, out, B, O, S);
     return hipGetLastError();
 }
+
+long long head_points(long long S) { return (S + PT - 1) / PT * PT; }
 
 int head_slices(long long S) { return (int)((S + SLICE - 1) / SLICE); }
 

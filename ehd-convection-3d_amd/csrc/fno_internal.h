@@ -58,11 +58,13 @@ hipError_t mix_backward(int w, int B, int NM, float* Sr, float* Si, const float*
 // The projection width -> hidden -> d_out of a prediction and its backward
 // pass (fno_head.hip), bit-identical to the pointwise GEMMs: shapes for which
 // head_fits holds, S points a sample, weights [c][h] and [h][o], biases b1, b2.
-//   forward:  z1[b][h] = b1 + W1 v (stored unless z1 is null), out = b2 + W2 gelu(z1)
+//   forward:  z1 = b1 + W1 v (B hidden head_points(S) floats in an order of its own,
+//             stored unless z1 is null), out = b2 + W2 gelu(z1)
 //   backward: dv[b][c], the partial sums dW1[slice][c][h] and dW2[slice][h][o] of
-//             B head_slices(S) slices, and quads[b][h][S/4], the sums of four
-//             consecutive points of the hidden layer's gradient
+//             B head_slices(S) slices, and the sums of four consecutive points of
+//             the hidden layer's gradient, quads[b][tile of 32 points][h][8]
 bool head_fits(int w, int hidden, int O, long long S);
+long long head_points(long long S);   // in whole tiles
 int head_slices(long long S);
 hipError_t head_forward(int w, int B, int O, long long S, const float* v, const float* W1, const float* b1,
                         const float* W2, const float* b2, float* z1, float* out, hipStream_t st);
@@ -84,7 +86,8 @@ hipError_t sum_slices(const float* src, float* dst, long long n, int nslices, fl
 long long channel_sum_part_floats(int B, int C, long long S);
 hipError_t channel_sum(const float* g, float* db, int B, int C, long long S, bool accumulate, float* part,
                        hipStream_t st);
-// the same sums of g from the sums of its quads, quads[b][c][S/4] (S a multiple of 4), to the last bit
+// the same sums of g, to the last bit, from the sums of its quads, quads[b][tile of 32 points][c][8]
+// (S a multiple of 4, C of 8)
 hipError_t channel_sum_quads(const float* quads, float* db, int B, int C, long long S, float* part, hipStream_t st);
 // grad = 2 (out - tgt) / n, part[mse_blocks()] = partial sums of (out - tgt)^2
 int mse_blocks();

@@ -438,21 +438,17 @@ __device__ __forceinline__ float block_sum_256(float s, float* red)
     return red[0];
 }
 
-// part[row][chunk] = sum of g[row][chunk*kRowChunk ...) for the rows (b, c): element loads, quads
-// where the rows allow it (the sum of a quad first), or those quads' sums as given
-constexpr int kElements = 0, kQuads = 1, kQuadSums = 2;
-template <int FROM>
+// part[row][chunk] = sum of g[row][chunk*kRowChunk ...) for the rows (b, c)
+template <bool VEC>
 __global__ void __launch_bounds__(256) row_chunk_sum_kernel(const float* __restrict__ g, float* __restrict__ part,
                                                             long long S, int nchunk)
 {
     __shared__ float red[256];
     const long long row = blockIdx.y;
-    const float* __restrict__ p = g + row * (FROM == kQuadSums ? S / 4 : S);
+    const float* __restrict__ p = g + row * S;
     const long long s0 = (long long)blockIdx.x * kRowChunk, s1 = min(S, s0 + kRowChunk);
     float s = 0.f;
-    if constexpr (FROM == kQuadSums) {
-        for (long long i = s0 / 4 + threadIdx.x; i < s1 / 4; i += 256) s += p[i];
-    } else if constexpr (FROM == kQuads) {
+    if constexpr (VEC) {
         for (long long i = s0 + 4 * threadIdx.x; i < s1; i += 1024) {
             const float4 v = *(const float4*)(p + i);
             s += (v.x + v.y) + (v.z + v.w);
@@ -462,6 +458,29 @@ __global__ void __launch_bounds__(256) row_chunk_sum_kernel(const float* __restr
     }
     const float t = block_sum_256(s, red);
     if (threadIdx.x == 0) part[row * nchunk + blockIdx.x] = t;
+}
+
+// The same part from the quads' sums, eight channels (whole cache lines of a
+// tile) a workgroup: a thread adds the quads that it would have formed.
+__global__ void __launch_bounds__(256) quad_chunk_sum_kernel(const float* __restrict__ quads, float* __restrict__ part,
+                                                             int C, long long S, int nchunk)
+{
+    __shared__ float red[256];
+    const int c0 = blockIdx.y * 8, b = blockIdx.z;
+    const long long i0 = (long long)blockIdx.x * (kRowChunk / 4), i1 = min(S / 4, i0 + kRowChunk / 4);
+    const long long tiles = (S + 31) / 32;
+    float s[8] = {};
+    for (long long i = i0 + threadIdx.x; i < i1; i += 256) {
+        const float* p = quads + ((b * tiles + i / 8) * C + c0) * 8 + (i & 7);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) s[c] += p[8 * c];
+    }
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const float t = block_sum_256(s[c], red);
+        if (threadIdx.x == 0) part[((long long)b * C + c0 + c) * nchunk + blockIdx.x] = t;
+        __syncthreads();
+    }
 }
 
 // db[c] (+)= sum over b and chunks of part[(b C + c) nchunk + chunk]: one workgroup per channel
@@ -649,9 +668,9 @@ hipError_t channel_sum(const float* g, float* db, int B, int C, long long S, boo
     const int nchunk = (int)((S + kRowChunk - 1) / kRowChunk);
     const dim3 grid((unsigned)nchunk, (unsigned)rows);
     if (S % 4 == 0 && (uintptr_t)g % 16 == 0)
-        row_chunk_sum_kernel<kQuads><<<grid, 256, 0, st>>>(g, part, S, nchunk);
+        row_chunk_sum_kernel<true><<<grid, 256, 0, st>>>(g, part, S, nchunk);
     else
-        row_chunk_sum_kernel<kElements><<<grid, 256, 0, st>>>(g, part, S, nchunk);
+        row_chunk_sum_kernel<false><<<grid, 256, 0, st>>>(g, part, S, nchunk);
     channel_total_kernel<<<C, 256, 0, st>>>(part, db, B, C, nchunk, accumulate ? 1 : 0);
     return hipGetLastError();
 }
@@ -659,9 +678,10 @@ hipError_t channel_sum(const float* g, float* db, int B, int C, long long S, boo
 hipError_t channel_sum_quads(const float* quads, float* db, int B, int C, long long S, float* part, hipStream_t st)
 {
     const long long rows = (long long)B * C;
-    if (rows <= 0 || rows > 65535 || S <= 0 || S % 4 != 0) return hipErrorInvalidValue;
+    if (rows <= 0 || rows > 65535 || S <= 0 || S % 4 != 0 || C % 8 != 0) return hipErrorInvalidValue;
     const int nchunk = (int)((S + kRowChunk - 1) / kRowChunk);
-    row_chunk_sum_kernel<kQuadSums><<<dim3((unsigned)nchunk, (unsigned)rows), 256, 0, st>>>(quads, part, S, nchunk);
+    quad_chunk_sum_kernel<<<dim3((unsigned)nchunk, (unsigned)(C / 8), (unsigned)B), 256, 0, st>>>(quads, part, C, S,
+                                                                                                nchunk);
     channel_total_kernel<<<C, 256, 0, st>>>(part, db, B, C, nchunk, 0);
     return hipGetLastError();
 }
