@@ -69,6 +69,7 @@ struct ehd_fno {
     float *dv0 = nullptr, *dv1 = nullptr, *dh = nullptr;
     double* part = nullptr;
     bool head = false;            // the projection's own kernels (head_fits): no h and dh
+    bool layer = false;           // the layers' last step in one kernel (layer_fits)
     float* quads = nullptr;       // sums of four points of the hidden gradient
     float* wscr2 = nullptr;       // split-K partial sums of the projection's second weight gradient
     float* wscr = nullptr;        // split-K partial sums of the weight gradients
@@ -387,7 +388,36 @@ int pointwise_dw(ehd_fno* f, int B, int cin, int cout, const float* X, const flo
     return EHD_OK;
 }
 
-// out[b][o] (+)= K_l(v)  (the spectral convolution of layer l); keeps the spectrum in S[l]
+// The last step of layer l (a.mode kLayerBias or kLayerGelu) or of its adjoint:
+// the transform along z of S added to the pointwise product with x, operands
+// checked like the GEMMs'
+int layer_end(ehd_fno* f, int l, int B, const Cbuf& A, int sa, const Cbuf& S, const float* x, float* out, bool adjoint,
+              LayerOut a)
+{
+    const long long w = f->c.width, KZ = f->KZ, Z = f->c.Z, P = f->P, act = B * w * Z * P;
+    a.w = f->c.width; a.B = B; a.KZ = f->KZ; a.Z = f->c.Z; a.P = (int)P;
+    a.x = x;
+    a.W = f->p + f->oW[l];   // [c][o]: the product sums over c, its adjoint over o
+    a.sm = adjoint ? a.w : 1;
+    a.sk = adjoint ? 1 : a.w;
+    a.Ar = A.r; a.Ai = A.i; a.sa = (float)sa;
+    a.Sr = S.r; a.Si = S.i;
+    a.out = out;
+    for (const float* p : {a.x, (const float*)a.out, (const float*)a.pre, a.dact})
+        if (p && !in_range(f, p, act - 1)) return set_error(EHD_EINVAL, "layer operands");
+    if (!in_range(f, a.Sr, B * w * KZ * P - 1) || !in_range(f, a.Si, B * w * KZ * P - 1) ||
+        !in_range(f, a.Ar, KZ * Z - 1) || !in_range(f, a.Ai, KZ * Z - 1) || !in_range(f, a.W, w * w - 1) ||
+        (a.bias && !in_range(f, a.bias, w - 1)))
+        return set_error(EHD_EINVAL, "layer operands");
+    f->work.flops += 2.0 * act * (w + 2.0 * KZ);
+    f->work.bytes += 4.0 * ((double)act * (2 + (a.pre ? 1 : 0) + (a.dact ? 1 : 0)) + 2.0 * (B * w * P + Z) * KZ + w * w);
+    f->work.launches += 1;
+    FCHK(layer_out(a, f->st));
+    return EHD_OK;
+}
+
+// out[b][o] (+)= K_l(v)  (the spectral convolution of layer l) up to the
+// spectrum along z in f->Wy where layer_end ends it; keeps the spectrum in S[l]
 int spectral_fwd(ehd_fno* f, int l, int B, const float* v, float* out, float beta)
 {
     const int w = f->c.width, X = f->c.X, Y = f->c.Y, Z = f->c.Z;
@@ -453,7 +483,7 @@ int spectral_fwd(ehd_fno* f, int l, int B, const float* v, float* out, float bet
         g.nb1 = (int)(BC * KZ);
         FCHK(cgemm(f, g, f->Byi.r, f->Byi.i, f->Wx.r, f->Wx.i, f->Wy.r, f->Wy.i, 1, 1, 0.f, f->st));
     }
-    {   // 7. out = Re(Azi^T Wy) along z
+    if (!f->layer) {   // 7. out = Re(Azi^T Wy) along z
         Geo g;
         g.M = Z; g.N = (int)P; g.K = KZ;
         g.am = 1; g.ak = Z;
@@ -465,7 +495,7 @@ int spectral_fwd(ehd_fno* f, int l, int B, const float* v, float* out, float bet
     return EHD_OK;
 }
 
-// dv (+)= K_l^T(du); dRr, dRi = gradient of the mixing weights
+// dv (+)= K_l^T(du), up to the spectrum along z in f->Vz where layer_end ends it; dRr, dRi = gradient of the mixing weights
 int spectral_bwd(ehd_fno* f, int l, int B, const float* du, float* dv, float beta)
 {
     const int w = f->c.width, X = f->c.X, Y = f->c.Y, Z = f->c.Z;
@@ -542,7 +572,7 @@ int spectral_bwd(ehd_fno* f, int l, int B, const float* du, float* dv, float bet
         g.nb1 = (int)(BC * KZ);
         FCHK(cgemm(f, g, f->ByT.r, f->ByT.i, f->Vy.r, f->Vy.i, f->Vz.r, f->Vz.i, -1, 1, 0.f, f->st));
     }
-    {   // 1b. dv (+)= Re(AzT^H G_Vz) = AzT_r^T G_r + AzT_i^T G_i
+    if (!f->layer) {   // 1b. dv (+)= Re(AzT^H G_Vz) = AzT_r^T G_r + AzT_i^T G_i
         Geo g;
         g.M = Z; g.N = (int)P; g.K = KZ;
         g.am = 1; g.ak = Z;
@@ -565,6 +595,14 @@ int forward(ehd_fno* f, int B, bool keep)
     if ((rc = pointwise(f, B, f->c.d_in, w, f->p + f->oPw, f->in, f->v[0], 0.f, ep))) return rc;
     for (int l = 0; l < L; ++l) {
         if ((rc = spectral_fwd(f, l, B, f->v[l], f->v[l + 1], 0.f))) return rc;
+        if (f->layer) {
+            LayerOut a{};
+            a.mode = l < L - 1 ? kLayerGelu : kLayerBias;
+            a.bias = f->p + f->ob[l];
+            a.pre = l < L - 1 && keep ? f->u[l] : nullptr;
+            if ((rc = layer_end(f, l, B, f->Azi, 1, f->Wy, f->v[l], f->v[l + 1], false, a))) return rc;
+            continue;
+        }
         Epi el;
         el.bias = f->p + f->ob[l];
         if (l < L - 1) {
@@ -625,7 +663,14 @@ int backward(ehd_fno* f, int B)
         if ((rc = pointwise_dw(f, B, w, w, f->v[l], dv, f->g + f->oW[l]))) return rc;
         FCHK(channel_sum(dv, f->g + f->ob[l], B, w, ZP, false, f->red, f->st));
         if ((rc = spectral_bwd(f, l, B, dv, dn, 0.f))) return rc;
-        if ((rc = pointwise_dx(f, B, w, w, f->p + f->oW[l], dv, dn, 1.f, l >= 1 ? f->u[l - 1] : nullptr))) return rc;
+        if (f->layer) {
+            LayerOut a{};
+            a.mode = l >= 1 ? kLayerGrad : kLayerNone;
+            a.dact = l >= 1 ? f->u[l - 1] : nullptr;
+            if ((rc = layer_end(f, l, B, f->AzT, -1, f->Vz, dv, dn, true, a))) return rc;
+        } else if ((rc = pointwise_dx(f, B, w, w, f->p + f->oW[l], dv, dn, 1.f, l >= 1 ? f->u[l - 1] : nullptr))) {
+            return rc;
+        }
         float* t = dv;
         dv = dn;
         dn = t;
@@ -727,6 +772,7 @@ int ehd_fno_create(const ehd_fno_config* cfg, ehd_fno** out)
         (rc = falloc(f, &f->tgt, B * c.d_out * f->ZP)) || (rc = falloc(f, &f->dout, B * c.d_out * f->ZP)) ||
         (rc = falloc(f, &f->dv0, act)) || (rc = falloc(f, &f->dv1, act)))
         return bail(rc);
+    f->layer = layer_fits(c.width, f->KZ, c.Z, f->P);
     f->head = head_fits(c.width, c.d_hidden, c.d_out, f->ZP);
     if (f->head ? (rc = falloc(f, &f->quads, B * c.d_hidden * (head_points(f->ZP) / 4)))
                 : (rc = falloc(f, &f->h, B * c.d_hidden * f->ZP)) || (rc = falloc(f, &f->dh, B * c.d_hidden * f->ZP)))

@@ -83,7 +83,7 @@ __global__ void __launch_bounds__(256) head_fwd_kernel(const float* __restrict__
 {
     constexpr int w = WT * 16;
     __shared__ __align__(16) unsigned short Hs[4][PT * HP];   // [wave][point][hidden]
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lj = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, lj = lane & 15, lg = lane >> 4;
     unsigned short* Hw = Hs[wave];
     bf16x8 a1[HT], a2[H / 32];
     float bias[HT];
@@ -167,7 +167,7 @@ head_bwd_kernel(const float* __restrict__ v, const float* __restrict__ z1, const
     __shared__ __align__(16) unsigned short Ds[2][PT * HP];   // dh [point][hidden]
     __shared__ __align__(16) unsigned short Ws[w * HP];       // W1 [c][hidden]
     __shared__ __align__(16) unsigned short Xs[4][PT * 8];    // dout [wave][row of the products][channel]
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lj = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, lj = lane & 15, lg = lane >> 4;
     const int h0 = wave * 32, dp = wave & 1, dc = wave >> 1;   // this wave's channels; its half and channel tile of dv
     unsigned short* Xw = Xs[wave];
     const int b = blockIdx.x / nsplit;

@@ -55,6 +55,28 @@ hipError_t mix_forward(int w, int B, int NM, const float* Sr, const float* Si, c
                        float* Yr, float* Yi, hipStream_t st);
 hipError_t mix_backward(int w, int B, int NM, float* Sr, float* Si, const float* Gr, const float* Gi, const float* Rr,
                         const float* Ri, float* dRr, float* dRi, hipStream_t st);
+// The end of a Fourier layer or of its adjoint (fno_layer.hip), bit-identical
+// to a complex and a pointwise GEMM: shapes for which layer_fits holds,
+//   out[b][m][z][p] = sum_c W[m][c] x[b][c][z][p] + Re sum_kz (Ar + i sa Ai)[kz][z] (Sr + i Si)[b][m][kz][p]
+// with W[m][c] at m*sm + c*sk, then by mode
+//   kLayerBias: + bias[m]; kLayerGelu: + bias[m], stored to pre unless that is null, gelu;
+//   kLayerNone: as it is;  kLayerGrad: times gelu'(dact).
+constexpr int kLayerBias = 0, kLayerGelu = 1, kLayerNone = 2, kLayerGrad = 3;
+struct LayerOut {
+    int mode, w, B, KZ, Z, P;
+    const float* x;
+    const float* W;
+    int sm, sk;
+    const float *Ar, *Ai;
+    float sa;
+    const float *Sr, *Si;
+    float* out;
+    const float* bias = nullptr;
+    const float* dact = nullptr;
+    float* pre = nullptr;
+};
+bool layer_fits(int w, int KZ, int Z, long long P);
+hipError_t layer_out(const LayerOut& a, hipStream_t st);
 // The projection width -> hidden -> d_out of a prediction and its backward
 // pass (fno_head.hip), bit-identical to the pointwise GEMMs: shapes for which
 // head_fits holds, S points a sample, weights [c][h] and [h][o], biases b1, b2.

@@ -315,6 +315,47 @@ def test_projection_matches_the_pointwise_gemms_bitwise(grid, width, d_out):
         assert np.all(np.isfinite(g[k])) and np.array_equal(g[k], g_w[k]), k
 
 
+# Widths 16 and 32 end their layers in a kernel of its own; inside a width of 48 whose
+# further channels have zero weights the layers go through the GEMMs, and those channels
+# stay zero: outputs, loss and the gradients of the shared channels are the same
+# bit for bit.  Planes with a last tile of 8 points and of whole tiles; z of less
+# than, of whole and of ragged groups of 16; 1 to all 16 modes.
+@pytest.mark.parametrize("grid,mz", [((12, 6, 10), 1), ((8, 8, 32), 16), ((20, 10, 50), 12)])
+@pytest.mark.parametrize("width", [16, 32])
+def test_layer_ends_match_the_gemms_bitwise(grid, mz, width):
+    cfg = F.FNOConfig(X=grid[0], Y=grid[1], Z=grid[2], width=width, modes=(3, 2, mz), layers=3, d_in=3, d_hidden=24,
+                      d_out=2)
+    rng = np.random.default_rng(23)
+    p = F.init_params(cfg, seed=23)
+    for k in p:
+        if k in ("Pb", "Q1b", "Q2b") or k.startswith("b"):
+            p[k] = 0.3 * rng.standard_normal(p[k].shape)
+        if k.startswith("R"):
+            p[k] = p[k] * width * width * 0.3
+    a = rng.standard_normal((2, 3, cfg.Z, cfg.Y, cfg.X)).astype(np.float32)
+    t = rng.standard_normal((2, 2, cfg.Z, cfg.Y, cfg.X)).astype(np.float32)
+
+    def net(w):
+        return G.FNO(cfg.X, cfg.Y, cfg.Z, width=w, modes=cfg.modes, layers=3, d_in=3, d_hidden=24, d_out=2, max_batch=2)
+
+    def embed(small, large):   # every axis of the width's length grows, zeros beyond
+        out = np.zeros(large)
+        out[tuple(slice(n) for n in small.shape)] = small
+        return out
+
+    res = []
+    for w in (width, 48):
+        n = net(w)
+        n.set_params({k: embed(np.asarray(p[k]), shape) for k, shape in G.param_shapes(n.cfg)})
+        loss, g = n.gradients(a, t)
+        res.append((n.forward(a), loss, G.unflatten(n.cfg, g)))
+        n.close()
+    (out, loss, g), (out_w, loss_w, g_w) = res
+    assert np.array_equal(out, out_w) and loss == loss_w
+    for k in g:
+        assert np.all(np.isfinite(g[k])) and np.array_equal(g[k], g_w[k][tuple(slice(n) for n in g[k].shape)]), k
+
+
 def test_adam_steps_reduce_loss():
     p, a, t, net = _setup(seed=2)
     losses = [net.train_step(a, t, 3e-3) for _ in range(30)]
