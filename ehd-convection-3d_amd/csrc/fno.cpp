@@ -907,12 +907,7 @@ int ehd_fno_train_step_indices(ehd_fno* f, int batch, const int* idx, float lr, 
             return set_error(EHD_EINVAL, "sample index %d outside 0..%d", idx[i], f->ds_n - 1);
     }
     // gather the batch on the device; the step then runs on it as on a resident batch
-    for (int i = 0; i < batch; ++i) {
-        HIPCHK(hipMemcpyAsync(f->in + i * sin, f->ds_in + (size_t)idx[i] * sin, sin * sizeof(float),
-                              hipMemcpyDeviceToDevice, f->st));
-        HIPCHK(hipMemcpyAsync(f->tgt + i * sout, f->ds_tgt + (size_t)idx[i] * sout, sout * sizeof(float),
-                              hipMemcpyDeviceToDevice, f->st));
-    }
+    FCHK(gather(f->ds_in, f->ds_tgt, idx, batch, (long long)sin, (long long)sout, f->in, f->tgt, f->st));
     f->resident = batch;
     return ehd_fno_train_step(f, batch, nullptr, nullptr, lr, loss);
 }

@@ -16,7 +16,7 @@
 // input channels; 128 hidden in four steps; d_out; 32 consecutive points of a
 // slice of 2048), operands rounded to bf16 where the GEMMs staged them, FP32
 // epilogues.  At 8 samples of 64x64x64 points, width 32, 2.0 ms of GEMMs and
-// sums became 0.28 ms forward and 0.57 backward (0.08 for a prediction of 4).
+// sums became 0.28 ms forward and 0.51 backward (0.08 for a prediction of 4).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>

@@ -111,9 +111,13 @@ hipError_t channel_sum(const float* g, float* db, int B, int C, long long S, boo
 // the same sums of g, to the last bit, from the sums of its quads, quads[b][tile of 32 points][c][8]
 // (S a multiple of 4, C of 8)
 hipError_t channel_sum_quads(const float* quads, float* db, int B, int C, long long S, float* part, hipStream_t st);
-// grad = 2 (out - tgt) / n, part[mse_blocks()] = partial sums of (out - tgt)^2
+// grad = 2 (out - tgt) / n, part[mse_blocks()] = partial sums of (out - tgt)^2; n a multiple of 4
 int mse_blocks();
 hipError_t mse(const float* out, const float* tgt, float* grad, double* part, long long n, hipStream_t st);
+// in[b], tgt[b] = samples idx[b] (on the host) of ds_in and ds_tgt, nin and ntgt floats each
+// (multiples of 4)
+hipError_t gather(const float* ds_in, const float* ds_tgt, const int* idx, int B, long long nin, long long ntgt,
+                  float* in, float* tgt, hipStream_t st);
 // Adam (Kingma & Ba 2015), t counts from 1
 hipError_t adam(float* p, const float* g, float* m, float* v, long long n, float lr, float b1, float b2, float eps,
                 int t, hipStream_t st);

@@ -378,6 +378,32 @@ def test_resident_batch_steps_match_host_batches():
         n2.train_step(None, None, 2e-3, batch=a.shape[0])
 
 
+# The gather takes 64 samples a launch; the loss and its gradient, like the gather,
+# work on quads (samples of 6 and 4 of them, fewer than the threads; of 300 and 200).
+@pytest.mark.parametrize("grid", [(2, 2, 2), (10, 8, 5)])
+@pytest.mark.parametrize("batch", [64, 65, 130])
+def test_large_gathered_batches_match_host_batches(grid, batch):
+    nets = [G.FNO(*grid, width=4, modes=(1, 1, 1), layers=2, d_in=3, d_hidden=8, d_out=2, max_batch=130)
+            for _ in range(2)]
+    rng = np.random.default_rng(4)
+    p = (0.3 * rng.standard_normal(nets[0].n)).astype(np.float32)
+    a = rng.standard_normal((9, 3) + grid[::-1]).astype(np.float32)
+    t = rng.standard_normal((9, 2) + grid[::-1]).astype(np.float32)
+    idx = rng.integers(0, 9, batch).tolist()
+    for n in nets:
+        n.set_params(G.unflatten(n.cfg, p))
+    nets[1].set_dataset(a, t)
+    loss = nets[0].train_step(a[idx], t[idx], 1e-3)
+    assert nets[1].train_step_indices(idx, 1e-3) == loss
+    assert np.array_equal(nets[0].get_params(), nets[1].get_params())
+    out = nets[0].forward(a[idx])
+    nets[1].set_params(G.unflatten(nets[1].cfg, p))
+    first = nets[1].forward(a[idx]).astype(np.float64)
+    ref = np.mean((first - t[idx].astype(np.float64)) ** 2)
+    # float differences carry 2^-24 of the larger of the two each, their squares twice that: far within 1e-6
+    assert abs(loss / ref - 1) < 1e-6 and out.shape == first.shape
+
+
 def test_resident_dataset_steps_match_host_batches():
     """Steps on mini-batches gathered on the device from a resident training
     set give bit for bit what the same steps on host copies of those samples
