@@ -68,8 +68,8 @@ struct ehd_fno {
     Cbuf Vz, Vy, Ym, Wx, Wy;      // spectral temporaries (reused by the backward pass)
     float *dv0 = nullptr, *dv1 = nullptr, *dh = nullptr;
     double* part = nullptr;
-    bool head = false;            // the projection's own kernels (head_fits): no h and dh
-    bool layer = false;           // the layers' last step in one kernel (layer_fits)
+    bool head = false;            // the projection's own kernels (head_fits); in training from head_min samples on
+    int head_min = 0;             // (head_batch), h and dh are for fewer
     float* quads = nullptr;       // sums of four points of the hidden gradient
     float* wscr2 = nullptr;       // split-K partial sums of the projection's second weight gradient
     float* wscr = nullptr;        // split-K partial sums of the weight gradients
@@ -388,6 +388,30 @@ int pointwise_dw(ehd_fno* f, int B, int cin, int cout, const float* X, const flo
     return EHD_OK;
 }
 
+// V[b][c][kz][ky][x] = the transforms of v along z and y by the tables A and B
+// (their imaginary parts times s), operands checked like the GEMMs'
+int dft_begin(ehd_fno* f, int B, const Cbuf& A, const Cbuf& Bt, int s, const float* v, const Cbuf& V)
+{
+    const long long BC = (long long)B * f->c.width, Z = f->c.Z, Y = f->c.Y, X = f->c.X, KZ = f->KZ, KY = f->KY;
+    for (const float* p : {A.r, A.i})
+        if (!in_range(f, p, KZ * Z - 1)) return set_error(EHD_EINVAL, "transform operands");
+    for (const float* p : {Bt.r, Bt.i})
+        if (!in_range(f, p, KY * Y - 1)) return set_error(EHD_EINVAL, "transform operands");
+    for (const float* p : {V.r, V.i})
+        if (!in_range(f, p, BC * KZ * KY * X - 1)) return set_error(EHD_EINVAL, "transform operands");
+    if (!in_range(f, v, BC * f->ZP - 1)) return set_error(EHD_EINVAL, "transform operands");
+    f->work.flops += 2.0 * BC * X * KZ * Y * (2.0 * Z + 4.0 * KY);
+    f->work.bytes += 4.0 * ((double)BC * (f->ZP + 2.0 * KZ * KY * X) + 2.0 * (KZ * Z + KY * Y));
+    f->work.launches += 1;
+    FCHK(dft_zy(v, A.r, A.i, Bt.r, Bt.i, (float)s, V.r, V.i, (int)BC, f->KZ, f->KY, f->c.X, f->c.Y, f->c.Z, f->st));
+    return EHD_OK;
+}
+
+bool layer_kernel(const ehd_fno* f, int B) { return layer_fits(f->c.width, B, f->KZ, f->c.Z, f->P); }
+
+// a prediction or (train) the forward and backward pass of a step
+bool head_kernels(const ehd_fno* f, int B, bool train) { return f->head && (!train || B >= f->head_min); }
+
 // The last step of layer l (a.mode kLayerBias or kLayerGelu) or of its adjoint:
 // the transform along z of S added to the pointwise product with x, operands
 // checked like the GEMMs'
@@ -426,23 +450,28 @@ int spectral_fwd(ehd_fno* f, int l, int B, const float* v, float* out, float bet
     const float* Rr = f->p + f->oRr[l];
     const float* Ri = f->p + f->oRi[l];
     Cbuf& S = f->S[l];
-    {   // 1. Vz = AzT v (real input)
-        Geo g;
-        g.M = KZ; g.N = (int)P; g.K = Z;
-        g.am = Z; g.ak = 1;
-        g.bk = P; g.bn = 1; g.b1 = Z * P;
-        g.cm = P; g.cn = 1; g.c1 = KZ * P;
-        g.nb1 = (int)BC;
-        FCHK(xgemm(f, g, f->AzT.r, f->AzT.i, v, nullptr, f->Vz.r, f->Vz.i, 1, 1, 1.f, 0.f, f->st));
-    }
-    {   // 2. Vy = ByT Vz along y, per (bc, kz)
-        Geo g;
-        g.M = KY; g.N = X; g.K = Y;
-        g.am = Y; g.ak = 1;
-        g.bk = X; g.bn = 1; g.b1 = (long long)Y * X;
-        g.cm = X; g.cn = 1; g.c1 = (long long)KY * X;
-        g.nb1 = (int)(BC * KZ);
-        FCHK(cgemm(f, g, f->ByT.r, f->ByT.i, f->Vz.r, f->Vz.i, f->Vy.r, f->Vy.i, 1, 1, 0.f, f->st));
+    if (dft_fits((int)BC, KZ, KY, X, Y, Z)) {   // 1., 2.
+        const int rc = dft_begin(f, B, f->AzT, f->ByT, 1, v, f->Vy);
+        if (rc) return rc;
+    } else {
+        {   // 1. Vz = AzT v (real input)
+            Geo g;
+            g.M = KZ; g.N = (int)P; g.K = Z;
+            g.am = Z; g.ak = 1;
+            g.bk = P; g.bn = 1; g.b1 = Z * P;
+            g.cm = P; g.cn = 1; g.c1 = KZ * P;
+            g.nb1 = (int)BC;
+            FCHK(xgemm(f, g, f->AzT.r, f->AzT.i, v, nullptr, f->Vz.r, f->Vz.i, 1, 1, 1.f, 0.f, f->st));
+        }
+        {   // 2. Vy = ByT Vz along y, per (bc, kz)
+            Geo g;
+            g.M = KY; g.N = X; g.K = Y;
+            g.am = Y; g.ak = 1;
+            g.bk = X; g.bn = 1; g.b1 = (long long)Y * X;
+            g.cm = X; g.cn = 1; g.c1 = (long long)KY * X;
+            g.nb1 = (int)(BC * KZ);
+            FCHK(cgemm(f, g, f->ByT.r, f->ByT.i, f->Vz.r, f->Vz.i, f->Vy.r, f->Vy.i, 1, 1, 0.f, f->st));
+        }
     }
     {   // 3. S = Vy Cx along x
         Geo g;
@@ -483,7 +512,7 @@ int spectral_fwd(ehd_fno* f, int l, int B, const float* v, float* out, float bet
         g.nb1 = (int)(BC * KZ);
         FCHK(cgemm(f, g, f->Byi.r, f->Byi.i, f->Wx.r, f->Wx.i, f->Wy.r, f->Wy.i, 1, 1, 0.f, f->st));
     }
-    if (!f->layer) {   // 7. out = Re(Azi^T Wy) along z
+    if (!layer_kernel(f, B)) {   // 7. out = Re(Azi^T Wy) along z
         Geo g;
         g.M = Z; g.N = (int)P; g.K = KZ;
         g.am = 1; g.ak = Z;
@@ -506,23 +535,28 @@ int spectral_bwd(ehd_fno* f, int l, int B, const float* du, float* dv, float bet
     float* dRr = f->g + f->oRr[l];
     float* dRi = f->g + f->oRi[l];
     Cbuf& S = f->S[l];
-    {   // 7b. G_Wy = conj(Azi) du  (real du)
-        Geo g;
-        g.M = KZ; g.N = (int)P; g.K = Z;
-        g.am = Z; g.ak = 1;
-        g.bk = P; g.bn = 1; g.b1 = Z * P;
-        g.cm = P; g.cn = 1; g.c1 = KZ * P;
-        g.nb1 = (int)BC;
-        FCHK(xgemm(f, g, f->Azi.r, f->Azi.i, du, nullptr, f->Wy.r, f->Wy.i, -1, 1, 1.f, 0.f, f->st));
-    }
-    {   // 6b. G_Wx = conj(Byi) G_Wy along y
-        Geo g;
-        g.M = KY; g.N = X; g.K = Y;
-        g.am = Y; g.ak = 1;
-        g.bk = X; g.bn = 1; g.b1 = (long long)Y * X;
-        g.cm = X; g.cn = 1; g.c1 = (long long)KY * X;
-        g.nb1 = (int)(BC * KZ);
-        FCHK(cgemm(f, g, f->Byi.r, f->Byi.i, f->Wy.r, f->Wy.i, f->Wx.r, f->Wx.i, -1, 1, 0.f, f->st));
+    if (dft_fits((int)BC, KZ, KY, X, Y, Z)) {   // 7b., 6b.
+        const int rc = dft_begin(f, B, f->Azi, f->Byi, -1, du, f->Wx);
+        if (rc) return rc;
+    } else {
+        {   // 7b. G_Wy = conj(Azi) du  (real du)
+            Geo g;
+            g.M = KZ; g.N = (int)P; g.K = Z;
+            g.am = Z; g.ak = 1;
+            g.bk = P; g.bn = 1; g.b1 = Z * P;
+            g.cm = P; g.cn = 1; g.c1 = KZ * P;
+            g.nb1 = (int)BC;
+            FCHK(xgemm(f, g, f->Azi.r, f->Azi.i, du, nullptr, f->Wy.r, f->Wy.i, -1, 1, 1.f, 0.f, f->st));
+        }
+        {   // 6b. G_Wx = conj(Byi) G_Wy along y
+            Geo g;
+            g.M = KY; g.N = X; g.K = Y;
+            g.am = Y; g.ak = 1;
+            g.bk = X; g.bn = 1; g.b1 = (long long)Y * X;
+            g.cm = X; g.cn = 1; g.c1 = (long long)KY * X;
+            g.nb1 = (int)(BC * KZ);
+            FCHK(cgemm(f, g, f->Byi.r, f->Byi.i, f->Wy.r, f->Wy.i, f->Wx.r, f->Wx.i, -1, 1, 0.f, f->st));
+        }
     }
     {   // 5b. G_Ym = G_Wx Cxi^H along x
         Geo g;
@@ -572,7 +606,7 @@ int spectral_bwd(ehd_fno* f, int l, int B, const float* du, float* dv, float bet
         g.nb1 = (int)(BC * KZ);
         FCHK(cgemm(f, g, f->ByT.r, f->ByT.i, f->Vy.r, f->Vy.i, f->Vz.r, f->Vz.i, -1, 1, 0.f, f->st));
     }
-    if (!f->layer) {   // 1b. dv (+)= Re(AzT^H G_Vz) = AzT_r^T G_r + AzT_i^T G_i
+    if (!layer_kernel(f, B)) {   // 1b. dv (+)= Re(AzT^H G_Vz) = AzT_r^T G_r + AzT_i^T G_i
         Geo g;
         g.M = Z; g.N = (int)P; g.K = KZ;
         g.am = 1; g.ak = Z;
@@ -595,7 +629,7 @@ int forward(ehd_fno* f, int B, bool keep)
     if ((rc = pointwise(f, B, f->c.d_in, w, f->p + f->oPw, f->in, f->v[0], 0.f, ep))) return rc;
     for (int l = 0; l < L; ++l) {
         if ((rc = spectral_fwd(f, l, B, f->v[l], f->v[l + 1], 0.f))) return rc;
-        if (f->layer) {
+        if (layer_kernel(f, B)) {
             LayerOut a{};
             a.mode = l < L - 1 ? kLayerGelu : kLayerBias;
             a.bias = f->p + f->ob[l];
@@ -611,7 +645,7 @@ int forward(ehd_fno* f, int B, bool keep)
         }
         if ((rc = pointwise(f, B, w, w, f->p + f->oW[l], f->v[l], f->v[l + 1], 1.f, el))) return rc;
     }
-    if (f->head) {
+    if (head_kernels(f, B, keep)) {
         if (!head_operands(f, B, {f->v[L]}, {f->out})) return set_error(EHD_EINVAL, "projection operands");
         head_work(f, B, 1, w + O + (keep ? H : 0));
         FCHK(head_forward(w, B, O, f->ZP, f->v[L], f->p + f->oQ1w, f->p + f->oQ1b, f->p + f->oQ2w, f->p + f->oQ2b,
@@ -638,7 +672,7 @@ int backward(ehd_fno* f, int B)
     float* dv = f->dv0;
     float* dn = f->dv1;
     FCHK(channel_sum(f->dout, f->g + f->oQ2b, B, O, ZP, false, f->red, f->st));
-    if (f->head) {
+    if (head_kernels(f, B, true)) {
         const long long ns = (long long)B * f->nsplit, n1 = (long long)w * H, n2 = (long long)H * O;
         if (!head_operands(f, B, {f->v[L], dv}, {f->dout}) || f->nsplit != head_slices(ZP) ||
             !in_range(f, f->wscr, ns * n1 - 1) || !in_range(f, f->wscr2, ns * n2 - 1) ||
@@ -663,7 +697,7 @@ int backward(ehd_fno* f, int B)
         if ((rc = pointwise_dw(f, B, w, w, f->v[l], dv, f->g + f->oW[l]))) return rc;
         FCHK(channel_sum(dv, f->g + f->ob[l], B, w, ZP, false, f->red, f->st));
         if ((rc = spectral_bwd(f, l, B, dv, dn, 0.f))) return rc;
-        if (f->layer) {
+        if (layer_kernel(f, B)) {
             LayerOut a{};
             a.mode = l >= 1 ? kLayerGrad : kLayerNone;
             a.dact = l >= 1 ? f->u[l - 1] : nullptr;
@@ -772,10 +806,11 @@ int ehd_fno_create(const ehd_fno_config* cfg, ehd_fno** out)
         (rc = falloc(f, &f->tgt, B * c.d_out * f->ZP)) || (rc = falloc(f, &f->dout, B * c.d_out * f->ZP)) ||
         (rc = falloc(f, &f->dv0, act)) || (rc = falloc(f, &f->dv1, act)))
         return bail(rc);
-    f->layer = layer_fits(c.width, f->KZ, c.Z, f->P);
     f->head = head_fits(c.width, c.d_hidden, c.d_out, f->ZP);
-    if (f->head ? (rc = falloc(f, &f->quads, B * c.d_hidden * (head_points(f->ZP) / 4)))
-                : (rc = falloc(f, &f->h, B * c.d_hidden * f->ZP)) || (rc = falloc(f, &f->dh, B * c.d_hidden * f->ZP)))
+    f->head_min = head_batch(f->ZP);
+    const long long Bh = f->head ? std::min<long long>(B, f->head_min - 1) : B;   // samples of h and dh
+    if ((f->head && B > Bh && (rc = falloc(f, &f->quads, B * c.d_hidden * (head_points(f->ZP) / 4)))) ||
+        (Bh > 0 && ((rc = falloc(f, &f->h, Bh * c.d_hidden * f->ZP)) || (rc = falloc(f, &f->dh, Bh * c.d_hidden * f->ZP)))))
         return bail(rc);
     f->v.assign(c.layers + 1, nullptr);
     for (auto& p : f->v)

@@ -317,6 +317,13 @@ hipError_t head_forward(int w, int B, int O, long long S, const float* v, const 
     return hipGetLastError();
 }
 
+// A workgroup walks a slice of 2048 points; with fewer than 128 of them the
+// GEMMs, which spread a slice over several workgroups, are faster.  Training steps,
+// kernel against GEMMs: width 32, 32x32x24 with 1, 4 samples (12, 48 slices) 0.98/0.84,
+// 1.27/1.19 ms, 64x64x64 with 1 (128) 1.80/1.81, with 2 2.32/2.56; width 16, 48x48x64 with 1
+// (72) 1.06/1.04, 32x32x48 with 8 (192) 1.52/1.60.
+int head_batch(long long S) { return (int)((128 + head_slices(S) - 1) / head_slices(S)); }
+
 long long head_points(long long S) { return (S + PT - 1) / PT * PT; }
 
 int head_slices(long long S) { return (int)((S + SLICE - 1) / SLICE); }

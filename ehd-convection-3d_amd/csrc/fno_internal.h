@@ -55,6 +55,12 @@ hipError_t mix_forward(int w, int B, int NM, const float* Sr, const float* Si, c
                        float* Yr, float* Yi, hipStream_t st);
 hipError_t mix_backward(int w, int B, int NM, float* Sr, float* Si, const float* Gr, const float* Gi, const float* Rr,
                         const float* Ri, float* dRr, float* dRi, hipStream_t st);
+// The transforms along z and y of real v[bc][z][y][x] (fno_dft.hip), bit-identical to two complex GEMMs:
+// shapes for which dft_fits holds,
+//   out[bc][kz][ky][x] = sum_y (Br + i s Bi)[ky][y] sum_z (Ar + i s Ai)[kz][z] v
+bool dft_fits(int BC, int KZ, int KY, int X, int Y, int Z);
+hipError_t dft_zy(const float* v, const float* Ar, const float* Ai, const float* Br, const float* Bi, float s,
+                  float* outr, float* outi, int BC, int KZ, int KY, int X, int Y, int Z, hipStream_t st);
 // The end of a Fourier layer or of its adjoint (fno_layer.hip), bit-identical
 // to a complex and a pointwise GEMM: shapes for which layer_fits holds,
 //   out[b][m][z][p] = sum_c W[m][c] x[b][c][z][p] + Re sum_kz (Ar + i sa Ai)[kz][z] (Sr + i Si)[b][m][kz][p]
@@ -75,7 +81,7 @@ struct LayerOut {
     const float* dact = nullptr;
     float* pre = nullptr;
 };
-bool layer_fits(int w, int KZ, int Z, long long P);
+bool layer_fits(int w, int B, int KZ, int Z, long long P);
 hipError_t layer_out(const LayerOut& a, hipStream_t st);
 // The projection width -> hidden -> d_out of a prediction and its backward
 // pass (fno_head.hip), bit-identical to the pointwise GEMMs: shapes for which
@@ -86,6 +92,7 @@ hipError_t layer_out(const LayerOut& a, hipStream_t st);
 //             B head_slices(S) slices, and the sums of four consecutive points of
 //             the hidden layer's gradient, quads[b][tile of 32 points][h][8]
 bool head_fits(int w, int hidden, int O, long long S);
+int head_batch(long long S);   // from this batch on the backward kernel is the faster one
 long long head_points(long long S);   // in whole tiles
 int head_slices(long long S);
 hipError_t head_forward(int w, int B, int O, long long S, const float* v, const float* W1, const float* b1,

@@ -226,14 +226,20 @@ hipError_t launch(const LayerOut& a, hipStream_t st)
 
 }  // namespace
 
-bool layer_fits(int w, int KZ, int Z, long long P)
+// 512 workgroups, two on every compute unit, run at a time; where the last such
+// round is less than seven eighths full the GEMMs, which spread the same work
+// wider, are the faster ones.  Training steps at width 32, kernel against
+// GEMMs: 64x64x64 with 2, 3, 4 samples (256, 384, 512 workgroups) 2.42/2.32,
+// 2.97/2.87, 3.20/3.40 ms; 48x48x64 with 6, 8 (432, 576) 3.24/3.23, 4.20/4.01 ms.
+bool layer_fits(int w, int B, int KZ, int Z, long long P)
 {
-    return (w == 16 || w == 32) && KZ <= KM && P % 4 == 0 && Z * P < (1 << 25);
+    const long long blocks = (P + PT - 1) / PT * B, rounds = (blocks + 511) / 512;
+    return (w == 16 || w == 32) && KZ <= KM && P % 4 == 0 && Z * P < (1 << 25) && 8 * blocks >= 7 * 512 * rounds;
 }
 
 hipError_t layer_out(const LayerOut& a, hipStream_t st)
 {
-    if (a.B < 1 || a.P < 1 || a.Z < 1 || a.KZ < 1 || !layer_fits(a.w, a.KZ, a.Z, a.P) ||
+    if (a.B < 1 || a.P < 1 || a.Z < 1 || a.KZ < 1 || !layer_fits(a.w, a.B, a.KZ, a.Z, a.P) ||
         (a.mode <= kLayerGelu && !a.bias) || (a.mode == kLayerGrad && !a.dact))
         return hipErrorInvalidValue;
     return a.w == 32 ? launch<2>(a, st) : launch<1>(a, st);

@@ -284,10 +284,11 @@ def test_gradients_of_every_width_and_batch_path_match_oracle(width, batch):
 # A projection of 128 hidden channels takes kernels of its own; with 32 more channels
 # whose weights are zero it goes through the pointwise GEMMs, and adds only zeros: outputs,
 # loss and every gradient are the same bit for bit.  Points: 20 beyond the last
-# whole tile of 32; two slices of 2048, the second part full; ragged in both.
-@pytest.mark.parametrize("grid", [(6, 6, 5), (16, 16, 10), (18, 14, 9)])
+# whole tile of 32; two slices of 2048, the second part full; ragged in both; too few
+# slices for the backward kernel.
+@pytest.mark.parametrize("grid,batch", [((6, 6, 5), 128), ((16, 16, 10), 64), ((18, 14, 9), 64), ((18, 14, 9), 3)])
 @pytest.mark.parametrize("width,d_out", [(16, 1), (32, 2), (16, 8), (32, 5)])
-def test_projection_matches_the_pointwise_gemms_bitwise(grid, width, d_out):
+def test_projection_matches_the_pointwise_gemms_bitwise(grid, batch, width, d_out):
     cfg = F.FNOConfig(X=grid[0], Y=grid[1], Z=grid[2], width=width, modes=(2, 3, 2), layers=2, d_in=3, d_hidden=128,
                       d_out=d_out)
     rng = np.random.default_rng(17)
@@ -298,12 +299,12 @@ def test_projection_matches_the_pointwise_gemms_bitwise(grid, width, d_out):
     wide["Q1w"] = np.concatenate([p["Q1w"], np.zeros((width, 32))], axis=1)
     wide["Q1b"] = np.concatenate([p["Q1b"], np.zeros(32)])
     wide["Q2w"] = np.concatenate([p["Q2w"], np.zeros((32, d_out))], axis=0)
-    a = rng.standard_normal((3, 3, cfg.Z, cfg.Y, cfg.X)).astype(np.float32)
-    t = rng.standard_normal((3, d_out, cfg.Z, cfg.Y, cfg.X)).astype(np.float32)
+    a = rng.standard_normal((batch, 3, cfg.Z, cfg.Y, cfg.X)).astype(np.float32)
+    t = rng.standard_normal((batch, d_out, cfg.Z, cfg.Y, cfg.X)).astype(np.float32)
     res = []
     for hidden, q in ((128, p), (160, wide)):
         net = G.FNO(cfg.X, cfg.Y, cfg.Z, width=width, modes=cfg.modes, layers=2, d_in=3, d_hidden=hidden, d_out=d_out,
-                    max_batch=3)
+                    max_batch=batch)
         net.set_params(q)
         loss, g = net.gradients(a, t)
         res.append((net.forward(a), loss, G.unflatten(net.cfg, g)))
@@ -319,10 +320,11 @@ def test_projection_matches_the_pointwise_gemms_bitwise(grid, width, d_out):
 # further channels have zero weights the layers go through the GEMMs, and those channels
 # stay zero: outputs, loss and the gradients of the shared channels are the same
 # bit for bit.  Planes with a last tile of 8 points and of whole tiles; z of less
-# than, of whole and of ragged groups of 16; 1 to all 16 modes.
-@pytest.mark.parametrize("grid,mz", [((12, 6, 10), 1), ((8, 8, 32), 16), ((20, 10, 50), 12)])
+# than, of whole and of ragged groups of 16; 1 to all 16 modes; batches that fill
+# rounds of 512 workgroups.
+@pytest.mark.parametrize("grid,mz,batch", [((12, 6, 10), 1, 341), ((16, 16, 32), 16, 64), ((20, 10, 50), 12, 73)])
 @pytest.mark.parametrize("width", [16, 32])
-def test_layer_ends_match_the_gemms_bitwise(grid, mz, width):
+def test_layer_ends_match_the_gemms_bitwise(grid, mz, batch, width):
     cfg = F.FNOConfig(X=grid[0], Y=grid[1], Z=grid[2], width=width, modes=(3, 2, mz), layers=3, d_in=3, d_hidden=24,
                       d_out=2)
     rng = np.random.default_rng(23)
@@ -332,11 +334,11 @@ def test_layer_ends_match_the_gemms_bitwise(grid, mz, width):
             p[k] = 0.3 * rng.standard_normal(p[k].shape)
         if k.startswith("R"):
             p[k] = p[k] * width * width * 0.3
-    a = rng.standard_normal((2, 3, cfg.Z, cfg.Y, cfg.X)).astype(np.float32)
-    t = rng.standard_normal((2, 2, cfg.Z, cfg.Y, cfg.X)).astype(np.float32)
+    a = rng.standard_normal((batch, 3, cfg.Z, cfg.Y, cfg.X)).astype(np.float32)
+    t = rng.standard_normal((batch, 2, cfg.Z, cfg.Y, cfg.X)).astype(np.float32)
 
     def net(w):
-        return G.FNO(cfg.X, cfg.Y, cfg.Z, width=w, modes=cfg.modes, layers=3, d_in=3, d_hidden=24, d_out=2, max_batch=2)
+        return G.FNO(cfg.X, cfg.Y, cfg.Z, width=w, modes=cfg.modes, layers=3, d_in=3, d_hidden=24, d_out=2, max_batch=batch)
 
     def embed(small, large):   # every axis of the width's length grows, zeros beyond
         out = np.zeros(large)
@@ -376,6 +378,33 @@ def test_resident_batch_steps_match_host_batches():
     n2.forward(a)
     with pytest.raises(Exception):
         n2.train_step(None, None, 2e-3, batch=a.shape[0])
+
+
+# Up to 16 modes along z the transforms along z and y share a kernel; with 17 modes, the
+# further ones of zero weights, they go through the GEMMs: outputs, loss and the
+# gradients of the shared modes are the same bit for bit.  Rows of less than, of
+# whole and of ragged groups of 16; y and z of one and two steps of 32; 258
+# channels of all samples make 256 workgroups.
+@pytest.mark.parametrize("grid", [(12, 6, 34), (16, 32, 34), (36, 40, 70)])
+@pytest.mark.parametrize("mz", [1, 16])
+def test_transforms_match_the_gemms_bitwise(grid, mz):
+    def net(m):
+        return G.FNO(*grid, width=43, modes=(3, 3, m), layers=2, d_in=2, d_hidden=8, d_out=2, max_batch=6)
+
+    rng = np.random.default_rng(31)
+    a, t = (rng.standard_normal((6, 2) + grid[::-1]).astype(np.float32) for _ in range(2))
+    small, large = net(mz), net(17)
+    p = {k: 0.3 * rng.standard_normal(shape) for k, shape in G.param_shapes(small.cfg)}
+    small.set_params(p)
+    for k in p:
+        if k.startswith("R"):
+            p[k] = np.concatenate([p[k], np.zeros((17 - mz,) + p[k].shape[1:])])
+    large.set_params(p)
+    (loss, g), (loss_l, g_l) = small.gradients(a, t), large.gradients(a, t)
+    assert loss == loss_l and np.array_equal(small.forward(a), large.forward(a))
+    g, g_l = G.unflatten(small.cfg, g), G.unflatten(large.cfg, g_l)
+    for k in g:
+        assert np.all(np.isfinite(g[k])) and np.array_equal(g[k], g_l[k][:mz] if k.startswith("R") else g_l[k]), k
 
 
 # The gather takes 64 samples a launch; the loss and its gradient, like the gather,
