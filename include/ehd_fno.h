@@ -99,8 +99,9 @@ int ehd_fno_cgemm_strided(int M, int N, int K, int nb, const float* Ar, const fl
                           float* Cr, float* Ci, const long long cs[3], long long c_len, int sa, int sb, float alpha,
                           float beta);
 
-/* Work of the GEMMs issued since the last reset (forward, gradients and
- * training steps): algorithmic FLOPs (2 M N K per real product; a complex
+/* Work of the GEMMs, and of the kernels that run several of them in one pass,
+ * issued since the last reset (forward, gradients and training steps):
+ * algorithmic FLOPs (2 M N K per real product; a complex
  * product counts as its four real ones), algorithmic HBM bytes (A and B read
  * once, C written once and read too when accumulated, all FP32), launches.
  * reset != 0 clears the counters after reading. */
