@@ -1,7 +1,9 @@
 // fno.cpp -- the Fourier-neural-operator surrogate on the GPU (include/ehd_fno.h).
 //
-// Every contraction is one call of the strided bf16 matrix-core GEMM
-// (fno_kernels.hip): the truncated DFTs are dense matrices applied along one
+// Every contraction can run as one call of the strided bf16 matrix-core GEMM
+// (fno_kernels.hip); shapes and batches for which a fused kernel is the faster
+// one (fno_dft.hip, fno_mix.hip, fno_layer.hip, fno_head.hip) take that, with
+// the same bits.  As GEMMs: the truncated DFTs are dense matrices applied along one
 // axis (z: real -> complex, y and x: complex -> complex), a complex product is
 // one launch over separate real and imaginary planes (each plane read once,
 // each result plane written once), and transposes or conjugates are stride

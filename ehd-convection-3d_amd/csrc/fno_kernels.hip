@@ -1,9 +1,9 @@
 // fno_kernels.hip -- the surrogate's GPU kernels: a strided, batched GEMM on
 // gfx950's bf16 matrix cores (v_mfma_f32_16x16x32_bf16, FP32 accumulation)
-// that carries every contraction of the Fourier neural operator (the
+// that can carry every contraction of the Fourier neural operator (the
 // truncated DFTs written as matrices, the per-mode channel mixing, the
 // pointwise layers and all their adjoints), plus the elementwise kernels
-// (loss, column sums, Adam); bias and GELU run in the GEMM epilogue.
+// (loss, column sums, Adam, the gather of a batch); bias and GELU run in the GEMM epilogue.
 //
 // Operands are FP32 in memory and rounded to bf16 (nearest even) when staged
 // into LDS; accumulation and the epilogue are FP32.  Any element strides are

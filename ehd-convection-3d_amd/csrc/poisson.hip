@@ -988,7 +988,7 @@ __global__ void __launch_bounds__(256) fftx_inv_kernel(const PoissonJob* __restr
 // (1) and (3) for a small plane in one launch each: a block holds a whole
 // plane, transforms its row pairs, turns them into the nx/2+1 lines along y in
 // LDS and transforms those, or the other way round.  The same line programs
-// as the separate passes, so the same numbers bit for bit.  Two launches and
+// as the separate passes, so with the same plan the same numbers bit for bit.  Two launches and
 // a spectrum round trip less per direction: the whole solve takes, five launches
 // / three, FP32S 32x32x16 22.5 / 19.0 us, 64x64x64 24.1 / 18.2; FP64 64x64x32
 // 28.1 / 22.2 us.
