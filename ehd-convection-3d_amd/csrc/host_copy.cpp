@@ -172,11 +172,23 @@ private:
     std::atomic<bool> stop_{false};
 };
 
+// On every way out that is not a return of EHD_OK, no copy on the stream
+// outlives the memory that it writes: declared after all of that.
+struct Drain {
+    hipStream_t st;
+    bool done = false;
+    ~Drain()
+    {
+        if (!done) (void)hipStreamSynchronize(st);
+    }
+};
+
 // without staging memory or threads: as the runtime does it
 int download_plain(const HostCopy* c, int count, hipStream_t st)
 {
     std::vector<float> f;
     std::vector<double> mean;
+    Drain drain{st};
     for (int a = 0; a < count; ++a) {
         const bool raw = c[a].kind == HostCopy::kFloat || c[a].kind == HostCopy::kDouble;
         void* to = c[a].host;
@@ -192,11 +204,13 @@ int download_plain(const HostCopy* c, int count, hipStream_t st)
         HIPCHK(hipStreamSynchronize(st));
         if (!raw) deliver(c[a], f.data(), 0, c[a].n, mean.data());
     }
+    drain.done = true;
     return EHD_OK;
 }
 
 int download_staged(const HostCopy* c, int count, hipStream_t st, Staging& S)
 {
+    Drain drain{st};
     std::vector<Piece> pieces;
     size_t total = 0;
     for (int a = 0; a < count; ++a) {
@@ -228,6 +242,7 @@ int download_staged(const HostCopy* c, int count, hipStream_t st, Staging& S)
             move(k, at);
             at += (pieces[k].n * width(c[pieces[k].array]) + 63) & ~(size_t)63;
         }
+        drain.done = true;
         return EHD_OK;
     }
     auto slot = [&](int k) { return S.mem + (size_t)(k % kSlots) * kSlot; };
@@ -257,10 +272,8 @@ int download_staged(const HostCopy* c, int count, hipStream_t st, Staging& S)
         if (e == hipSuccess && !crew.empty())
             for (int k = std::max(0, np - kSlots); k < np; ++k) crew.wait(k);
     }
-    if (e != hipSuccess) {
-        (void)hipStreamSynchronize(st);   // no copy into a slot outlives the call
-        return set_error(EHD_EHIP, "device to host copy failed: %s", hipGetErrorString(e));
-    }
+    if (e != hipSuccess) return set_error(EHD_EHIP, "device to host copy failed: %s", hipGetErrorString(e));
+    drain.done = true;
     return EHD_OK;
 }
 
@@ -272,7 +285,6 @@ int download(const HostCopy* c, int count, hipStream_t st)
         Lease lease;
         return lease.s ? download_staged(c, count, st, *lease.s) : download_plain(c, count, st);
     } catch (const std::bad_alloc&) {
-        (void)hipStreamSynchronize(st);
         return set_error(EHD_ENOMEM, "host allocation failed");
     }
 }

@@ -1,0 +1,41 @@
+"""Field and parameter reads (csrc/host_copy.cpp) on a stand-in for the HIP
+runtime (tests/host_copy/hip/hip_runtime.h), which lets a chosen call fail:
+the values delivered, and what is left behind when a copy fails."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "ehd-convection-3d_amd", "csrc")
+HERE = os.path.join(ROOT, "tests", "host_copy")
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not on PATH")
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("host_copy") / "harness")
+    r = subprocess.run(["g++", "-std=c++17", "-O2", "-g", "-Wall", "-I", HERE, os.path.join(HERE, "harness.cpp"),
+                        os.path.join(CSRC, "host_copy.cpp"), os.path.join(CSRC, "ehd_error.cpp"), "-o", exe,
+                        "-lpthread"], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr
+
+    def scenario(*args):
+        r = subprocess.run([exe, *args], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout + r.stderr
+    return scenario
+
+
+def test_small_and_large_reads_are_exact(run):
+    run("exact")
+
+
+@pytest.mark.parametrize("call", ["hipMemcpyAsync", "hipEventRecord", "hipEventSynchronize"])
+def test_a_failed_copy_leaves_none_on_the_stream(run, call):
+    run("failing", call)
+
+
+def test_lack_of_host_memory_leaves_no_copy_on_the_stream(run):
+    run("no_memory")
