@@ -80,6 +80,7 @@ struct Lease {
         if (s && !s->make()) {
             delete s;
             s = nullptr;
+            (void)hipGetLastError();   // the copies go without: the next check of a launch must not find it
         }
     }
     ~Lease()

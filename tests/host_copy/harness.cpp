@@ -99,6 +99,22 @@ void no_memory()
     CHECK(download(g.c, 2, &other) == EHD_OK && g.right());
 }
 
+// Without staging memory the copies go the plain way, and the failure that the
+// call got over is not found by the next check of the thread's last error.
+void no_staging(const std::string& call)
+{
+    for (size_t n : kSizes)
+        for (long k = 1; k <= (call == "hipHostMalloc" ? 1 : 8); ++k) {
+            Fields f(n);
+            fake::Stream st;
+            fake::fail(call, k);
+            CHECK(download(f.c, 2, &st) == EHD_OK && f.right());
+            fake::failing.clear();
+            CHECK(hipGetLastError() == hipSuccess);
+            CHECK(st.run == st.queued && fake::pinned.empty());
+        }
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -107,6 +123,7 @@ int main(int argc, char** argv)
     if (what == "exact") exact();
     else if (what == "failing") failing(argv[2]);
     else if (what == "no_memory") no_memory();
+    else if (what == "no_staging") no_staging(argv[2]);
     else CHECK(!"scenario");
     CHECK(fake::pinned.empty());
     std::puts("ok");

@@ -39,3 +39,8 @@ def test_a_failed_copy_leaves_none_on_the_stream(run, call):
 
 def test_lack_of_host_memory_leaves_no_copy_on_the_stream(run):
     run("no_memory")
+
+
+@pytest.mark.parametrize("call", ["hipHostMalloc", "hipEventCreateWithFlags"])
+def test_reads_without_staging_memory_are_exact_and_leave_no_error(run, call):
+    run("no_staging", call)
