@@ -33,9 +33,10 @@ struct Staging {
     int device = -1;
 
     double* mean() const { return (double*)(mem + kSlots * kSlot); }
-    bool make()
+    // with dev current: an event can only be recorded on a stream of its own device
+    bool make(int dev)
     {
-        if (hipGetDevice(&device) != hipSuccess) return false;
+        device = dev;
         if (hipHostMalloc((void**)&mem, kSlots * kSlot + kMaxMean * sizeof(double), hipHostMallocDefault) != hipSuccess) {
             mem = nullptr;
             return false;
@@ -59,14 +60,18 @@ std::mutex g_mu;
 Staging* g_kept[2] = {nullptr, nullptr};
 long long g_owners = 0;
 
-// a staging buffer of the current device for one call, given back (or freed,
-// when two are kept already or no owner is left) at the end of it
+// a staging buffer of the stream's device (the calling thread's may be another)
+// for one call, given back (or freed, when two are kept already or no owner is
+// left) at the end of it
 struct Lease {
     Staging* s = nullptr;
-    Lease()
+    explicit Lease(hipStream_t st)
     {
-        int dev = -1;
-        if (hipGetDevice(&dev) != hipSuccess) return;
+        int dev = -1, current = -1;
+        if (hipStreamGetDevice(st, &dev) != hipSuccess || hipGetDevice(&current) != hipSuccess) {
+            (void)hipGetLastError();   // the copies go without staging: the next check of a launch must not find it
+            return;
+        }
         {
             std::lock_guard<std::mutex> lk(g_mu);
             for (Staging*& k : g_kept)
@@ -77,11 +82,13 @@ struct Lease {
                 }
         }
         s = new (std::nothrow) Staging();
-        if (s && !s->make()) {
+        if (current != dev && hipSetDevice(dev) != hipSuccess) dev = -1;
+        if (s && (dev < 0 || !s->make(dev))) {
             delete s;
             s = nullptr;
-            (void)hipGetLastError();   // the copies go without: the next check of a launch must not find it
+            (void)hipGetLastError();
         }
+        if (current != dev && dev >= 0) (void)hipSetDevice(current);
     }
     ~Lease()
     {
@@ -283,7 +290,7 @@ int download_staged(const HostCopy* c, int count, hipStream_t st, Staging& S)
 int download(const HostCopy* c, int count, hipStream_t st)
 {
     try {
-        Lease lease;
+        Lease lease(st);
         return lease.s ? download_staged(c, count, st, *lease.s) : download_plain(c, count, st);
     } catch (const std::bad_alloc&) {
         return set_error(EHD_ENOMEM, "host allocation failed");

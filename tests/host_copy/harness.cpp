@@ -115,6 +115,20 @@ void no_staging(const std::string& call)
         }
 }
 
+// A stream of another device than the thread's current one: the events and the
+// staging memory are the stream's device's, the current device stays.
+void other_device()
+{
+    for (size_t n : kSizes) {
+        Fields f(n), g(n);
+        fake::Stream far, near;
+        far.device = 1;
+        CHECK(download(f.c, 2, &far) == EHD_OK && f.right());
+        CHECK(fake::current == 0);
+        CHECK(download(g.c, 2, &near) == EHD_OK && g.right());
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -124,6 +138,7 @@ int main(int argc, char** argv)
     else if (what == "failing") failing(argv[2]);
     else if (what == "no_memory") no_memory();
     else if (what == "no_staging") no_staging(argv[2]);
+    else if (what == "other_device") other_device();
     else CHECK(!"scenario");
     CHECK(fake::pinned.empty());
     std::puts("ok");

@@ -44,3 +44,7 @@ def test_lack_of_host_memory_leaves_no_copy_on_the_stream(run):
 @pytest.mark.parametrize("call", ["hipHostMalloc", "hipEventCreateWithFlags"])
 def test_reads_without_staging_memory_are_exact_and_leave_no_error(run, call):
     run("no_staging", call)
+
+
+def test_a_stream_of_another_device_is_read(run):
+    run("other_device")
