@@ -57,11 +57,14 @@ struct Staging {
 };
 
 std::mutex g_mu;
-Staging* g_kept[2] = {nullptr, nullptr};
+// A buffer costs milliseconds to allocate and to free: eight are kept (128 MB
+// pinned at most), one for each device of a node or each of as many readers.
+constexpr int kKept = 8;
+Staging* g_kept[kKept] = {};
 long long g_owners = 0;
 
 // a staging buffer of the stream's device (the calling thread's may be another)
-// for one call, given back (or freed, when two are kept already or no owner is
+// for one call, given back (or freed, when kKept are kept already or no owner is
 // left) at the end of it
 struct Lease {
     Staging* s = nullptr;
@@ -305,11 +308,11 @@ void staging_retain()
 
 void staging_release()
 {
-    Staging* drop[2] = {nullptr, nullptr};
+    Staging* drop[kKept] = {};
     {
         std::lock_guard<std::mutex> lk(g_mu);
         if (--g_owners == 0)
-            for (int i = 0; i < 2; ++i) std::swap(drop[i], g_kept[i]);
+            for (int i = 0; i < kKept; ++i) std::swap(drop[i], g_kept[i]);
     }
     for (Staging* s : drop) delete s;
 }

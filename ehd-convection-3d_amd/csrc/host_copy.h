@@ -28,7 +28,7 @@ constexpr size_t kMaxMean = 4096;
 // count <= 16 arrays, at most one of them with a mean.
 int download(const HostCopy* c, int count, hipStream_t st);
 
-// The staging buffers are kept from call to call (at most two of them) while
+// The staging buffers are kept from call to call (at most eight of them) while
 // any box or network is alive: the owners count themselves in and out.
 void staging_retain();
 void staging_release();

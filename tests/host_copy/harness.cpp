@@ -129,6 +129,23 @@ void other_device()
     }
 }
 
+// Readers in turn on several devices keep a staging buffer each; with more of
+// them than are kept the pinned memory stays bounded.
+void kept(int devices)
+{
+    staging_retain();
+    for (int round = 0; round < 5; ++round)
+        for (int d = 0; d < devices; ++d) {
+            Fields f(400);
+            fake::Stream st;
+            st.device = d;
+            CHECK(download(f.c, 2, &st) == EHD_OK && f.right());
+            CHECK(fake::pinned.size() <= 8);
+        }
+    if (devices <= 8) CHECK(fake::calls["hipHostMalloc"] == devices);
+    staging_release();
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -139,6 +156,7 @@ int main(int argc, char** argv)
     else if (what == "no_memory") no_memory();
     else if (what == "no_staging") no_staging(argv[2]);
     else if (what == "other_device") other_device();
+    else if (what == "kept") kept(std::atoi(argv[2]));
     else CHECK(!"scenario");
     CHECK(fake::pinned.empty());
     std::puts("ok");

@@ -48,3 +48,8 @@ def test_reads_without_staging_memory_are_exact_and_leave_no_error(run, call):
 
 def test_a_stream_of_another_device_is_read(run):
     run("other_device")
+
+
+@pytest.mark.parametrize("devices", [1, 3, 8, 9])
+def test_staging_memory_is_kept_and_bounded(run, devices):
+    run("kept", str(devices))
