@@ -146,6 +146,18 @@ void kept(int devices)
     staging_release();
 }
 
+// A read waits for the stream it was queued on, so that the runtime has done
+// with its commands: left to it, they were on the bill of the box's close.
+void waited()
+{
+    for (size_t n : kSizes) {
+        Fields f(n);
+        fake::Stream st;
+        CHECK(download(f.c, 2, &st) == EHD_OK && f.right());
+        CHECK(st.waited == st.queued);
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -157,6 +169,7 @@ int main(int argc, char** argv)
     else if (what == "no_staging") no_staging(argv[2]);
     else if (what == "other_device") other_device();
     else if (what == "kept") kept(std::atoi(argv[2]));
+    else if (what == "waited") waited();
     else CHECK(!"scenario");
     CHECK(fake::pinned.empty());
     std::puts("ok");

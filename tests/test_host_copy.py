@@ -53,3 +53,7 @@ def test_a_stream_of_another_device_is_read(run):
 @pytest.mark.parametrize("devices", [1, 3, 8, 9])
 def test_staging_memory_is_kept_and_bounded(run, devices):
     run("kept", str(devices))
+
+
+def test_a_read_leaves_nothing_to_its_streams_owner(run):
+    run("waited")
