@@ -50,7 +50,7 @@ struct ehd_box {
     unsigned lbm_chunk = 0;              // FP32S LBM XCD tile order (lbm_xcd_chunk)
     bool lbm_stream = false;             // streaming population accesses (lbm_streams)
     int tune_lpb = 0, tune_ylines = 0;   // Poisson lines per block (0: largest that fits)
-    bool debug_sync = false;   // synchronise and check after every launch (ehd_set_debug_sync)
+    int debug_sync = 0;        // 1, 2: synchronise and check after every launch (ehd_set_debug_sync)
     long long step = 0;
     double t = 0.0;
     double current_hs = 0.0;

@@ -193,7 +193,7 @@ PoissonGroup poisson_group_of(const ehd_box* b)
     g.twx = b->twx;
     g.twy = b->twy;
     g.jobs = b->pjob;
-    g.debug_sync = b->debug_sync ? 1 : 0;
+    g.debug_sync = b->debug_sync;
     return g;
 }
 
@@ -1012,7 +1012,7 @@ int ehd_run_to_steady(ehd_box* b, int check_every, double tol, long long max_ste
 int ehd_set_debug_sync(ehd_box* b, int on)
 {
     if (!b) return set_error(EHD_EINVAL, "null box");
-    b->debug_sync = on != 0;
+    b->debug_sync = on == 2 ? 2 : on != 0;
     return EHD_OK;
 }
 

@@ -132,7 +132,7 @@ struct PoissonGroup {
     const void* twx;             // twiddles of nx and ny, path type
     const void* twy;
     const PoissonJob* jobs;      // device array of njobs
-    int debug_sync;              // synchronise the stream and check after every pass
+    int debug_sync;              // synchronise the stream and check after every pass; 2: every transform a pass of its own
 };
 // name of the Poisson pass whose synchronised check failed last (debug_sync)
 const char* poisson_failed_pass();

@@ -988,10 +988,10 @@ __global__ void __launch_bounds__(256) fftx_inv_kernel(const PoissonJob* __restr
 // (1) and (3) for a small plane in one launch each: a block holds a whole
 // plane, transforms its row pairs, turns them into the nx/2+1 lines along y in
 // LDS and transforms those, or the other way round.  The same line programs
-// as the separate passes, so with the same plan the same numbers bit for bit.  Two launches and
-// a spectrum round trip less per direction: the whole solve takes, five launches
-// / three, FP32S 32x32x16 22.5 / 19.0 us, 64x64x64 24.1 / 18.2; FP64 64x64x32
-// 28.1 / 22.2 us.
+// and, in the planes that with_plane admits, the same plan as the separate
+// passes, so the same numbers bit for bit.  Two launches and a spectrum round
+// trip less: solves back to back, five launches / three, FP32S 32x32x16 16.6 /
+// 13.1 us, 64x64x64 22.3 / 16.9; FP64 64x64x32 26.1 / 20.6 us.
 constexpr int kPlaneThreads = 512;
 
 // A sign that the compiler does not know: the y pass takes its as an
@@ -1264,7 +1264,7 @@ int log2_ceil(int v)
 // Planes of up to 64 x 64 points take the one-launch transforms where their two
 // buffers fit.  Larger ones keep too few blocks busy for too long, five launches /
 // three: FP32S 96x96x64 26.3 / 39 us, 100x80x64 29.6 / 35.5, 128x128x64 33 / 47
-// (62x64x40, the slowest kind of plan within the line, 28.9 / 28.1).
+// (62x62x40, the slowest kind of plan within the line, 34.5 / 30.6).
 template <typename T, int N>
 size_t plane_lds(int nx, int ny)
 {
@@ -1296,22 +1296,6 @@ hipError_t launch_plane(const PoissonGroup& g, bool inverse, hipStream_t st)
     return hipGetLastError();
 }
 
-// The plane kernels' plan: a compile-time one where both sides have it and a
-// line's butterflies fit the block (f(constant N) of 32 or 64), else the
-// runtime plan, else none.  Planes of 48x48 keep the separate passes: the
-// forward plane kernel of their plan fuses other products into sums, and a
-// run's recorded history must not depend on which kernel serves it.
-template <typename T, class F>
-bool with_plane(int nx, int ny, const F& f)
-{
-    if (nx == 48 && ny == 48) return false;
-    if (nx == 32 && plane_fits<T, 32>(nx, ny)) f(std::integral_constant<int, 32>{});
-    else if (nx == 64 && plane_fits<T, 64>(nx, ny)) f(std::integral_constant<int, 64>{});
-    else if (plane_fits<T, 0>(nx, ny)) f(std::integral_constant<int, 0>{});
-    else return false;
-    return true;
-}
-
 // f(constant N) with the compile-time plan's length, 0 for a runtime plan
 template <class F>
 auto with_plan(int n, const F& f)
@@ -1327,6 +1311,28 @@ auto with_plan(int n, const F& f)
     case 512: return f(std::integral_constant<int, 512>{});
     default: return f(std::integral_constant<int, 0>{});
     }
+}
+
+// f(constant N) with the plane kernels' plan, if there is one: a plane takes
+// them only where both sides run the plan that their passes would run, so that
+// the potential is the passes' bit for bit and a run's history does not depend
+// on which of the two serves its planes.  That is a square with a compile-time
+// plan of powers of two (32 or 64; with a factor of three the forward plane
+// kernel fuses other products into sums than the passes do) and two sides
+// without one (the runtime plan).  Other pairs are left to the passes, whose
+// compile-time plans are mostly the faster ones too: a whole FP32S solve of 9
+// interior planes, plane kernels with the runtime plan / passes, 32x64 19.1 /
+// 18.3 us, 48x64 20.8 / 18.7, 32x128 21.9 / 18.9, 96x36 22.9 / 21.0; one side
+// of 32 or 64 beside a runtime plan 64x40 20.3 / 22.2, 100x32 20.7 / 23.7.
+template <typename T, class F>
+bool with_plane(int nx, int ny, const F& f)
+{
+    auto planned = [](int n) { return with_plan(n, [](auto N) { return decltype(N)::value > 0; }); };
+    if (nx == 32 && plane_fits<T, 32>(nx, ny)) f(std::integral_constant<int, 32>{});
+    else if (nx == 64 && plane_fits<T, 64>(nx, ny)) f(std::integral_constant<int, 64>{});
+    else if (!planned(nx) && !planned(ny) && plane_fits<T, 0>(nx, ny)) f(std::integral_constant<int, 0>{});
+    else return false;
+    return true;
 }
 
 // One Poisson solve for every job of a group (same nx, ny, precision; the
@@ -1354,6 +1360,7 @@ hipError_t poisson_t(const PoissonGroup& g, hipStream_t st)
     };
     hipError_t ec = hipSuccess;
     auto plane_pass = [&](bool inverse) {
+        if (g.debug_sync == 2) return false;
         return with_plane<T>(nx, ny, [&](auto n) { ec = launch_plane<T, decltype(n)::value>(g, inverse, st); });
     };
     if (plane_pass(false)) {

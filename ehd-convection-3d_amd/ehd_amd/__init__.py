@@ -320,7 +320,8 @@ class Box:
         _check(lib().ehd_set_nusselt_reference(self._h, float(current_hs)))
 
     def set_debug_sync(self, on: bool = True):
-        """Synchronise and check after every launch (faults named by phase and step)."""
+        """Synchronise and check after every launch (faults named by phase and step); 2: small planes'
+        transforms along x and y in launches of their own too."""
         _check(lib().ehd_set_debug_sync(self._h, int(on)))
 
     def profile_enable(self, on: bool = True, every: int = 1):

@@ -227,8 +227,9 @@ int ehd_profile_reset(ehd_box* b);
  * check, so that an asynchronous fault is reported by the launch that caused
  * it, named in ehd_last_error() (phase and step).  The reference checks
  * launches only with cudaGetLastError and no synchronisation (LBM.cu:36-57),
- * so its faults surface later.  Off by default; the results are the same
- * either way, only slower. */
+ * so its faults surface later.  on = 2 also runs the transforms of small
+ * planes, which share a launch along x and y, as one launch each.  Off by
+ * default; the results are the same either way, bit for bit, only slower. */
 int ehd_set_debug_sync(ehd_box* b, int on);
 
 int ehd_sync(ehd_box* b);

@@ -296,6 +296,30 @@ def test_poisson_runtime_plans_vs_oracle(shape, precision):
     test_poisson_vs_oracle(shape, precision)
 
 
+# The one-launch transforms of small planes give the separate passes' bits (debug
+# level 2 runs those): squares with a compile-time plan, pairs of runtime plans of
+# every radix (2..5, 7, 9, 11, 13, 16, a prime stage), and planes of which only
+# one side, or each side another, has a compile-time plan.
+@pytest.mark.parametrize("shape", [(32, 32), (64, 64), (48, 48), (36, 36), (24, 40), (2, 14), (18, 26), (22, 98),
+                                   (62, 62), (34, 38), (16, 20), (58, 62), (32, 64), (64, 32), (48, 32), (80, 48),
+                                   (32, 100), (64, 40), (64, 62), (16, 256), (32, 128)])
+@pytest.mark.parametrize("precision", [E.FP64, E.FP32S])
+def test_plane_transforms_match_the_passes_bitwise(shape, precision):
+    nx, ny, nz = *shape, 9
+    q = np.random.default_rng(7).standard_normal((nz, ny, nx))
+    phi = []
+    for level in (0, 1, 2):
+        with E.Box(E.make_params(nx, ny, nz, T=200.0, precision=precision)) as b:
+            b.init()
+            b.set_debug_sync(level)
+            b.write_charge(q)
+            b.poisson()
+            phi.append(b.read_fields(("phi",))["phi"])
+    assert np.all(np.isfinite(phi[0])) and np.ptp(phi[0]) > 0
+    assert_same(phi[1], phi[0], "checked after every launch")
+    assert_same(phi[2], phi[0], "every transform in a launch of its own")
+
+
 def test_diagnostics_current_vs_oracle():
     ob = oracle_box(16, 12, 10)
     ob.init_equilibrium()
