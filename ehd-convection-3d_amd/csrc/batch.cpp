@@ -288,16 +288,24 @@ int tune(ehd_batch* bt)
         const PoissonShape ps = poisson_shape(bt->prec, gr.g.nx, gr.g.ny, gr.g.max_n + 2);
         double best = 1e30;
         int bl = 0, by = 0;
+        auto time_group = [&](double* ms) {
+            return time_ms(bt, reps, [&]() -> int {
+                HIPCHK(launch_poisson_group(bt->prec, gr.g, bt->st));
+                return EHD_OK;
+            }, ms);
+        };
+        if (poisson_planes(bt->prec, gr.g.nx, gr.g.ny)) {   // nothing to choose
+            int rc = time_group(&bt->group_ms[gi]);
+            if (rc) return rc;
+            continue;
+        }
         for (int xl : x_candidates(ps.max_x_lines))
             for (int yl : {ps.max_y_lines, ps.max_y_lines / 2, ps.max_y_lines / 4}) {
                 if (yl < 1) continue;
                 gr.g.lpb = xl;
                 gr.g.ylines = yl;
                 double ms = 0;
-                int rc = time_ms(bt, reps, [&]() -> int {
-                    HIPCHK(launch_poisson_group(bt->prec, gr.g, bt->st));
-                    return EHD_OK;
-                }, &ms);
+                int rc = time_group(&ms);
                 if (rc) return rc;
                 if (ms < best) {
                     best = ms;
@@ -773,8 +781,9 @@ int ehd_batch_tuning(ehd_batch* bt, ehd_tuning* out)
         out->group[i].nx = g.g.nx;
         out->group[i].ny = g.g.ny;
         out->group[i].nboxes = (int)g.members.size();
-        out->group[i].x_lines = g.g.lpb ? g.g.lpb : ps.max_x_lines;
-        out->group[i].y_lines = g.g.ylines ? g.g.ylines : ps.max_y_lines;
+        const bool planes = poisson_planes(bt->prec, g.g.nx, g.g.ny);
+        out->group[i].x_lines = planes ? 0 : g.g.lpb ? g.g.lpb : ps.max_x_lines;
+        out->group[i].y_lines = planes ? 0 : g.g.ylines ? g.g.ylines : ps.max_y_lines;
         out->group[i].ms = i < bt->group_ms.size() ? bt->group_ms[i] : 0.0;
     }
     return EHD_OK;

@@ -142,6 +142,8 @@ struct PoissonShape {
 PoissonJob make_poisson_job(const LbmParams& P, const PoissonBufs& pb, const void* q, void* phi, double voltage,
                             double eps);
 PoissonShape poisson_shape(Prec prec, int nx, int ny, int nz);
+// whether the transforms of such planes share a launch along x and y, which takes no line counts
+bool poisson_planes(Prec prec, int nx, int ny);
 // writes the job table *dst and the twiddle tables of nx and ny (path type) on the device
 hipError_t launch_poisson_setup(Prec prec, const PoissonJob& job, PoissonJob* dst, void* twx, int nx, void* twy, int ny,
                                 hipStream_t st);

@@ -1451,6 +1451,12 @@ PoissonShape poisson_shape(Prec prec, int nx, int ny, int nz)
     return s;
 }
 
+bool poisson_planes(Prec prec, int nx, int ny)
+{
+    auto any = [](auto) {};
+    return prec == Prec::F64 ? with_plane<double>(nx, ny, any) : with_plane<float>(nx, ny, any);
+}
+
 hipError_t launch_poisson_setup(Prec prec, const PoissonJob& job, PoissonJob* dst, void* twx, int nx, void* twy, int ny,
                                 hipStream_t st)
 {

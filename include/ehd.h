@@ -288,7 +288,8 @@ typedef struct ehd_tuning {
     double lbm_ms;            /* timed LBM launch (tuning run), 0 if not tuned */
     int ngroups;              /* Poisson groups (distinct nx, ny) */
     struct {
-        int nx, ny, nboxes, x_lines, y_lines;   /* lines per workgroup of the x / y FFT passes */
+        int nx, ny, nboxes, x_lines, y_lines;   /* lines per workgroup of the x / y FFT passes (0: small planes,
+                                                    one workgroup transforms a whole plane) */
         double ms;                               /* timed Poisson chain of the group, 0 if not tuned */
     } group[16];
     int lbm_chunk;            /* XCD tile order of the LBM launch: tiles per XCD run (0: linear order) */

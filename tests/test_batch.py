@@ -85,6 +85,16 @@ def test_batch_tuning_report_and_state_checks():
             bt.step(1)
 
 
+@pytest.mark.parametrize("flags", [0, E.BATCH_TUNE])
+def test_tuner_counts_lines_only_where_passes_have_them(flags):
+    """64x64 planes are transformed whole; 48x48 and 80x80 ones in passes of lines."""
+    with E.Batch(_params(E.FP32S), flags=flags) as bt:
+        t = bt.tuning()
+    lines = {t.group[i].nx: (t.group[i].x_lines, t.group[i].y_lines) for i in range(t.ngroups)}
+    assert lines[64] == (0, 0) and min(lines[48] + lines[80]) > 0
+    assert all((t.group[i].ms > 0) == bool(flags) for i in range(t.ngroups))
+
+
 def test_batch_steady_detector():
     """Subcritical boxes (T below the threshold) relax to the no-flow state;
     every box reports its own convergence step."""
