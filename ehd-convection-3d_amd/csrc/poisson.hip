@@ -1288,6 +1288,11 @@ hipError_t launch_plane(const PoissonGroup& g, bool inverse, hipStream_t st)
     const cplx<T>*twx = (const cplx<T>*)g.twx, *twy = (const cplx<T>*)g.twy;
     const int lgx = log2_ceil(g.ny / 2), lgy = log2_ceil(g.nx / 2 + 1);
     const PlanArg<N> plx = plan_arg<N>(g.nx), ply = plan_arg<N>(g.ny);
+    if (sh > kMaxLds) {   // more than a launch may ask for by itself
+        const void* kernel = inverse ? (const void*)plane_inv_kernel<T, N> : (const void*)plane_fwd_kernel<T, N>;
+        const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);
+        if (e != hipSuccess) return e;
+    }
     if (inverse)
         plane_inv_kernel<T, N><<<grid, kPlaneThreads, sh, st>>>(g.jobs, twx, twy, plx, ply, g.nx, g.ny, lgx, lgy,
                                                                 g.split_mean ? 0 : 1);
