@@ -47,6 +47,7 @@ struct ehd_batch {
     Prec prec = Prec::F32S;
     hipStream_t st = nullptr;
     int flags = 0;
+    bool graph = false;       // steady steps replay a captured graph (replays_graphs)
     // FP32S: one item table per buffer parity
     void* ditems[2] = {nullptr, nullptr};
     unsigned total_tiles = 0;
@@ -165,6 +166,19 @@ void drop_graphs(ehd_batch* bt)
             (void)hipGraphExecDestroy(e);
             e = nullptr;
         }
+}
+
+// EHD_BATCH_GRAPH is a matter of speed, so it holds only on the runtime (major
+// and minor version) that the library was built for.  Where another library
+// brought its own into the process first, torch with the 7.0 runtime in a
+// process of this build for 7.2, a batch with a graph ended in a segmentation
+// fault on the host whose cause is not known; there the steps are launched one
+// by one.
+bool replays_graphs(int flags)
+{
+    int v = 0;
+    return (flags & EHD_BATCH_GRAPH) != 0 && hipRuntimeGetVersion(&v) == hipSuccess &&
+           v / 100000 == HIP_VERSION / 100000;
 }
 
 // Capture the two steady steps (direct = ebuf = false, no macroscopic
@@ -325,11 +339,10 @@ int tune(ehd_batch* bt)
     // each, run as the batch will run it (the captured steady pair replayed,
     // or eager)
     if (!bt->side.empty() && !(bt->flags & EHD_BATCH_CHAINS)) {
-        const bool graph = (bt->flags & EHD_BATCH_GRAPH) != 0;
         for (int mode = 0; mode < 2; ++mode) {
             bt->chains = (mode == 1);
             int rc;
-            if (graph) {
+            if (bt->graph) {
                 if ((rc = capture_pair(bt, 0))) return rc;
                 rc = time_ms(bt, reps, [&]() -> int {
                     HIPCHK(hipGraphLaunch(bt->exec[0], bt->st));
@@ -378,6 +391,7 @@ int ehd_batch_create(const ehd_params* params, int nboxes, int flags, ehd_batch*
         return code;
     };
     bt->flags = flags;
+    bt->graph = replays_graphs(flags);
     bt->prec = params[0].precision == EHD_FP64 ? Prec::F64 : Prec::F32S;
     if (hipStreamCreateWithFlags(&bt->st, hipStreamNonBlocking) != hipSuccess)
         return bail(set_error(EHD_EHIP, "hipStreamCreate failed"));
@@ -644,7 +658,6 @@ int ehd_batch_step(ehd_batch* bt, int nsteps)
     for (ehd_box* b : bt->boxes) HIPCHK(hipStreamSynchronize(b->st));
     int cur = bt->boxes[0]->cur;
     bool direct = bt->boxes[0]->direct, ebuf = bt->boxes[0]->ebuf;
-    const bool graph = (bt->flags & EHD_BATCH_GRAPH) != 0;
     int i = 0;
     auto advance = [&](int n) {
         for (ehd_box* b : bt->boxes)
@@ -655,7 +668,7 @@ int ehd_batch_step(ehd_batch* bt, int nsteps)
     };
     while (i < nsteps) {
         const bool last = (i == nsteps - 1);
-        if (graph && !direct && !ebuf && i + 2 <= nsteps - 1) {
+        if (bt->graph && !direct && !ebuf && i + 2 <= nsteps - 1) {
             if (!bt->exec[cur] && (rc = capture_pair(bt, cur))) return rc;
             HIPCHK(hipGraphLaunch(bt->exec[cur], bt->st));
             i += 2;

@@ -274,7 +274,8 @@ int ehd_poisson_noalloc(const ehd_params* p, const double* q, double* phi, void*
  * per process (main.cu). */
 typedef struct ehd_batch ehd_batch;
 
-#define EHD_BATCH_GRAPH 1   /* replay the steady steps from a captured HIP graph */
+#define EHD_BATCH_GRAPH 1   /* replay the steady steps from a captured HIP graph (the same steps launched one by one
+                               where the process has a HIP runtime of another version than the library's) */
 #define EHD_BATCH_TUNE  2   /* time the launch shapes at creation and keep the fastest */
 #define EHD_BATCH_CHAINS 4  /* one LBM launch and Poisson chain per (nx, ny) group, the groups on
                                concurrent streams (with EHD_BATCH_TUNE and without this flag the

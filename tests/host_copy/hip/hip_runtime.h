@@ -17,8 +17,10 @@
 
 typedef int hipError_t;
 constexpr hipError_t hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2, hipErrorInvalidHandle = 400;
+constexpr int HIP_VERSION = 70200000;   // the runtime that the code is built for
+enum hipStreamCaptureMode { hipStreamCaptureModeThreadLocal = 1 };
 enum hipMemcpyKind { hipMemcpyHostToDevice = 1, hipMemcpyDeviceToHost = 2 };
-constexpr unsigned hipHostMallocDefault = 0, hipEventDisableTiming = 2;
+constexpr unsigned hipHostMallocDefault = 0, hipEventDisableTiming = 2, hipStreamNonBlocking = 1;
 
 namespace fake {
 
@@ -48,6 +50,7 @@ inline std::recursive_mutex mu;
 inline std::map<std::string, long> calls;     // how often a call was made
 inline std::string failing;                   // this call fails
 inline long failing_from = 0;                 // from this call of it on (counting from 1)
+inline int version = HIP_VERSION;             // of the runtime that is there
 inline thread_local int current = 0;          // current device
 inline thread_local hipError_t last = hipSuccess;
 inline std::map<char*, size_t> pinned;        // pinned allocations alive
@@ -176,3 +179,85 @@ inline hipError_t hipMemcpyAsync(void* to, const void* from, size_t n, hipMemcpy
     ++s->queued;
     return hipSuccess;
 }
+
+// ---- what a batch uses beside copies: plain memory, events without time, graphs that only count ----
+
+struct fakeGraph {
+};
+typedef fakeGraph* hipGraph_t;
+typedef fakeGraph* hipGraphExec_t;
+
+inline hipError_t hipRuntimeGetVersion(int* v)
+{
+    *v = fake::version;
+    return fake::enter("hipRuntimeGetVersion");
+}
+
+template <class T>
+hipError_t hipMalloc(T** p, size_t n)
+{
+    *p = (T*)std::malloc(n);
+    return hipSuccess;
+}
+
+inline hipError_t hipFree(void* p)
+{
+    std::free(p);
+    return hipSuccess;
+}
+
+inline hipError_t hipMemcpy(void* to, const void* from, size_t n, hipMemcpyKind)
+{
+    std::memcpy(to, from, n);
+    return hipSuccess;
+}
+
+inline hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned)
+{
+    *s = new fake::Stream;
+    return hipSuccess;
+}
+
+inline hipError_t hipStreamDestroy(hipStream_t s)
+{
+    delete s;
+    return hipSuccess;
+}
+
+inline hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+
+inline hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0); }
+
+inline hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t)
+{
+    *ms = 1.f;
+    return hipSuccess;
+}
+
+inline hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return fake::enter("hipStreamBeginCapture"); }
+
+inline hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g)
+{
+    *g = new fakeGraph;
+    return hipSuccess;
+}
+
+inline hipError_t hipGraphDestroy(hipGraph_t g)
+{
+    delete g;
+    return hipSuccess;
+}
+
+inline hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, void*, char*, size_t)
+{
+    *e = new fakeGraph;
+    return hipSuccess;
+}
+
+inline hipError_t hipGraphExecDestroy(hipGraphExec_t e)
+{
+    delete e;
+    return hipSuccess;
+}
+
+inline hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return fake::enter("hipGraphLaunch"); }

@@ -1,6 +1,8 @@
-"""Field and parameter reads (csrc/host_copy.cpp) on a stand-in for the HIP
-runtime (tests/host_copy/hip/hip_runtime.h), which lets a chosen call fail:
-the values delivered, and what is left behind when a copy fails."""
+"""Host code on a stand-in for the HIP runtime (tests/host_copy/hip/hip_runtime.h).
+
+Field and parameter reads (csrc/host_copy.cpp), where a chosen call can fail:
+the values delivered, and what is left behind when a copy fails.  Batches
+(csrc/batch.cpp) on runtimes of several versions: when steps replay a graph."""
 import os
 import shutil
 import subprocess
@@ -14,13 +16,18 @@ HERE = os.path.join(ROOT, "tests", "host_copy")
 pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not on PATH")
 
 
+def _build(folder, harness, source):
+    exe = str(folder / "harness")
+    r = subprocess.run(["g++", "-std=c++17", "-O2", "-g", "-Wall", "-I", HERE, os.path.join(HERE, harness),
+                        os.path.join(CSRC, source), os.path.join(CSRC, "ehd_error.cpp"), "-o", exe, "-lpthread"],
+                       capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr
+    return exe
+
+
 @pytest.fixture(scope="module")
 def run(tmp_path_factory):
-    exe = str(tmp_path_factory.mktemp("host_copy") / "harness")
-    r = subprocess.run(["g++", "-std=c++17", "-O2", "-g", "-Wall", "-I", HERE, os.path.join(HERE, "harness.cpp"),
-                        os.path.join(CSRC, "host_copy.cpp"), os.path.join(CSRC, "ehd_error.cpp"), "-o", exe,
-                        "-lpthread"], capture_output=True, text=True, timeout=300)
-    assert r.returncode == 0, r.stderr
+    exe = _build(tmp_path_factory.mktemp("host_copy"), "harness.cpp", "host_copy.cpp")
 
     def scenario(*args):
         r = subprocess.run([exe, *args], capture_output=True, text=True, timeout=120)
@@ -57,3 +64,23 @@ def test_staging_memory_is_kept_and_bounded(run, devices):
 
 def test_a_read_leaves_nothing_to_its_streams_owner(run):
     run("waited")
+
+
+@pytest.fixture(scope="module")
+def batch_harness(tmp_path_factory):
+    return _build(tmp_path_factory.mktemp("batch"), "batch_harness.cpp", "batch.cpp")
+
+
+# 11 steps: the direct one, pairs of steady ones, and the last, which runs eagerly;
+# two boxes of other planes, so the tuner captures a pair of each kind of step
+@pytest.mark.parametrize("tune", [0, 2])
+@pytest.mark.parametrize("version,replays", [(70200000, True), (70254321, True), (70051831, False), (60443483, False),
+                                             (80000000, False)])
+def test_batches_replay_graphs_only_on_the_runtime_they_were_built_for(batch_harness, version, replays, tune):
+    for flags, graph in ((1 | tune, replays), (tune, False)):
+        r = subprocess.run([batch_harness, str(version), str(flags)], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stderr
+        captures, played, launches = (int(w) for w in r.stdout.split()[::2])
+        assert (captures > 0) == graph and played == (4 if graph else 0)
+        # the tuner may keep one LBM launch for both boxes or one each
+        assert graph or launches in (11, 22)
