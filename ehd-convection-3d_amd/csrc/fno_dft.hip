@@ -186,7 +186,10 @@ dft_zy_kernel(const float* __restrict__ v, const float* __restrict__ Ar, const f
 }  // namespace
 
 // Two workgroups must share a compute unit's LDS for the loads of one to cover
-// the other's second transform, and they must fill the chip: a workgroup takes
+// the other's second transform.  That, not the 16 rows of the first product,
+// bounds the modes along z: a mode takes 5 KB beside the tables, so at most 15
+// of them fit (Y, Z <= 32, KY <= 16), at Y = Z = 64 at most 14 with KY <= 16 and
+// 13 with KY <= 32; at Y = 128 11 with KY = 24.  And the workgroups must fill the chip: one takes
 // a whole column, where the GEMMs split the planes further.  Training steps,
 // kernel against GEMMs: width 32, 64x64x64 with 1, 4 samples (64, 256
 // workgroups) 2.07/2.05, 3.20/3.31 ms, 48x48x64 with 6 (384) 3.24/3.24; width

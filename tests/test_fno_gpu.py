@@ -407,6 +407,37 @@ def test_transforms_match_the_gemms_bitwise(grid, mz):
         assert np.all(np.isfinite(g[k])) and np.array_equal(g[k], g_l[k][:mz] if k.startswith("R") else g_l[k]), k
 
 
+# The same over the sizes of the kernel: its three forms by the pieces of a wave (up
+# to 3, 6 and 8), one to three tiles of 16 along ky, whole and ragged, the
+# mode counts of the trained network and the most that fit.  The network with
+# 17 modes runs one launch more a layer, so the smaller one does take the kernel; with
+# 16 modes it does not (its LDS holds at most 15).
+@pytest.mark.parametrize("grid,my,mz", [((12, 16, 34), 8, 8), ((36, 24, 34), 12, 12), ((64, 64, 64), 12, 12),
+                                        ((20, 32, 34), 10, 14), ((34, 48, 40), 24, 10), ((12, 36, 70), 17, 9)])
+def test_transform_kernels_forms_match_the_gemms_bitwise(grid, my, mz):
+    def net(m):
+        return G.FNO(*grid, width=43, modes=(3, my, m), layers=2, d_in=2, d_hidden=8, d_out=2, max_batch=6)
+
+    rng = np.random.default_rng(37)
+    a, t = (rng.standard_normal((6, 2) + grid[::-1]).astype(np.float32) for _ in range(2))
+    nets = [net(m) for m in (mz, 16, 17)]
+    p = {k: 0.3 * rng.standard_normal(shape) for k, shape in G.param_shapes(nets[0].cfg)}
+    out, launches, grads = [], [], []
+    for n, m in zip(nets, (mz, 16, 17)):
+        n.set_params({k: np.concatenate([v, np.zeros((m - mz,) + v.shape[1:])]) if k.startswith("R") else v
+                      for k, v in p.items()})
+        n.gemm_work(reset=True)
+        out.append(n.forward(a))
+        launches.append(n.gemm_work(reset=True).launches)
+        loss, g = n.gradients(a, t)
+        grads.append(dict(G.unflatten(n.cfg, g), loss=np.float64(loss)))
+        n.close()
+    assert launches[0] + 2 == launches[1] == launches[2]
+    assert np.all(np.isfinite(out[0])) and np.array_equal(out[0], out[2])
+    for k, v in grads[0].items():
+        assert np.all(np.isfinite(v)) and np.array_equal(v, grads[2][k][:mz] if k.startswith("R") else grads[2][k]), k
+
+
 # The gather takes 64 samples a launch; the loss and its gradient, like the gather,
 # work on quads (samples of 6 and 4 of them, fewer than the threads; of 300 and 200).
 @pytest.mark.parametrize("grid", [(2, 2, 2), (10, 8, 5)])
