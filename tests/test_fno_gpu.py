@@ -281,6 +281,42 @@ def test_gradients_of_every_width_and_batch_path_match_oracle(width, batch):
     assert max(errs.values()) < 5e-2, errs
 
 
+# Widths 16 and 32 mix the modes in kernels of their own up to 16 samples, forward and
+# backward; inside a width of 48 whose further channels have zero weights the batched
+# GEMMs do it, and those channels stay zero: outputs, loss and the gradients of the shared
+# channels are the same bit for bit.  One sample to two groups of 8; modes that are and
+# are not whole groups of 16.  The backward kernel's two products are one launch, as
+# GEMMs two.
+@pytest.mark.parametrize("modes", [(3, 3, 1), (4, 2, 3), (5, 4, 3)])
+@pytest.mark.parametrize("batch", [1, 2, 8, 9, 16])
+@pytest.mark.parametrize("width", [16, 32])
+def test_mixing_matches_the_gemms_bitwise(width, batch, modes):
+    cfg, p, net, a, t = _small_net(width, modes, batch, seed=29)
+    wide = G.FNO(cfg.X, cfg.Y, cfg.Z, width=48, modes=modes, layers=2, d_in=cfg.d_in, d_hidden=cfg.d_hidden,
+                 d_out=cfg.d_out, max_batch=batch)
+
+    def embed(small, large):
+        out = np.zeros(large)
+        out[tuple(slice(n) for n in small.shape)] = small
+        return out
+
+    wide.set_params({k: embed(np.asarray(p[k]), shape) for k, shape in G.param_shapes(wide.cfg)})
+    res = []
+    for n in (net, wide):
+        n.gemm_work(reset=True)
+        loss, g = n.gradients(a, t)
+        res.append((n.gemm_work(reset=True).launches, loss, n.forward(a), G.unflatten(n.cfg, g)))
+        n.close()
+    (launches, loss, out, g), (launches_w, loss_w, out_w, g_w) = res
+    # the transforms' kernel, from 256 channels of all samples on, is a launch less a layer and direction
+    transforms = 4 * ((48 * batch >= 256) - (width * batch >= 256))
+    assert launches + 2 == launches_w + transforms
+    assert loss == loss_w and np.array_equal(out, out_w)
+    for k in g:
+        shared = g_w[k][tuple(slice(n) for n in g[k].shape)]
+        assert np.all(np.isfinite(g[k])) and np.any(g[k]) and np.array_equal(g[k], shared), k
+
+
 # A projection of 128 hidden channels takes kernels of its own; with 32 more channels
 # whose weights are zero it goes through the pointwise GEMMs, and adds only zeros: outputs,
 # loss and every gradient are the same bit for bit.  Points: 20 beyond the last
