@@ -113,6 +113,26 @@ def test_batch_steady_detector():
         assert all(x.step == max(r.steps for r in res) for x in d)
 
 
+@pytest.mark.parametrize("flags", [0, E.BATCH_GRAPH | E.BATCH_TUNE, E.BATCH_GRAPH | E.BATCH_CHAINS])
+@pytest.mark.parametrize("precision,shape", [(E.FP32S, (90, 152, 72)), (E.FP64, (122, 62, 64))])
+def test_batch_with_padded_rows_matches_single_boxes(precision, shape, flags):
+    """A box beyond 384 MB, whose populations keep padded rows, beside one that does not: as alone, bit for bit."""
+    params = [E.make_params(*s, T=T, C_=10.0, lam=0.25, precision=precision, init_mode=E.INIT_HYDROSTATIC, seed=seed,
+                            amp=1e-3) for s, T, seed in ((shape, 400.0, 31), ((50, 64, 20), 300.0, 32))]
+    nsteps = (1, 6)
+    with E.Batch(params, flags=flags) as bt:
+        bt.init()
+        for n in nsteps:
+            bt.step(n)
+        got = [_state(b) for b in bt.boxes]
+    for i, p in enumerate(params):
+        with E.Box(p) as b:
+            b.init()
+            for n in nsteps:
+                b.step(n)
+            _assert_same_state(got[i], _state(b), f"box {i} ({p.nx}x{p.ny}x{p.nz})")
+
+
 @pytest.mark.parametrize("flags", [E.BATCH_GRAPH | E.BATCH_TUNE, E.BATCH_GRAPH | E.BATCH_CHAINS])
 def test_batch_with_a_256_wide_box_matches_single_boxes(flags):
     """The bench box's plane size (256 x 256: one LBM tile per x-row, the

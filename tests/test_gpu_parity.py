@@ -177,6 +177,40 @@ def test_lbm_steps_with_padded_rows_bitexact(shape):
     test_lbm_steps_bitexact(dict(shape=shape, uw=0.05, exf=40.0))
 
 
+# A state that repeats along y does so on: a box of twice the rows, whose state is
+# beyond 384 MB and keeps padded rows (90 -> 96, 252 -> 256 floats), steps as the box
+# of one period does, which does not.  Whole potentials make the planes' means
+# exact, so every value is the same bit for bit.
+@pytest.mark.parametrize("shape", [(90, 76, 72), (252, 36, 56)])
+def test_fp32s_steps_with_padded_rows_match_unpadded_bitwise(shape):
+    nx, ny, nz = shape
+    assert 432 * nx * ny * nz <= 384 << 20 < 2 * 432 * nx * ny * nz
+    rng = np.random.default_rng(13)
+    one = rng.standard_normal((9, nz, ny, nx))
+    one[0] = 1600.0 + 1e-3 * one[0]
+    one[1] = 1e-4 * np.abs(one[1])
+    one[2] = rng.integers(0, 10000, (nz, ny, nx))
+    one[3:6] *= 1e-3
+    one[6:] *= 1e3
+    fields, pops = [], []
+    for f9 in (one, np.concatenate([one, one], axis=2)):
+        p = E.make_params(nx, f9.shape[2], nz, T=200.0, lam=0.25, uw=0.05, exf=40.0, precision=E.FP32S,
+                          init_mode=E.INIT_FIELDS)
+        with E.Box(p) as b:
+            b.init(f9)
+            for _ in range(3):
+                b.lbm_step()
+            fields.append(b.read_fields())
+            pops.append(b.read_populations())
+    for k, v in fields[0].items():
+        assert np.all(np.isfinite(v)), k
+        assert_same(fields[1][k][:, :ny], v, f"{k}, first period")
+        assert_same(fields[1][k][:, ny:], v, f"{k}, second period")
+    for got, ref, n in zip(pops[1], pops[0], ("f0", "f1", "h0", "h1")):
+        assert_same(got[..., :ny, :], ref, f"{n}, first period")
+        assert_same(got[..., ny:, :], ref, f"{n}, second period")
+
+
 @pytest.mark.parametrize("shape,precision,size", [((122, 62, 64), E.FP64, 8), ((90, 154, 70), E.FP32S, 4)])
 def test_checkpoint_with_padded_rows_bitexact(tmp_path, shape, precision, size):
     """The file holds the same rows as an unpadded box's, and restarts bit for bit."""
