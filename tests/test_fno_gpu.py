@@ -500,6 +500,27 @@ def test_large_gathered_batches_match_host_batches(grid, batch):
     assert abs(loss / ref - 1) < 1e-6 and out.shape == first.shape
 
 
+@pytest.mark.parametrize("batch", [3, 65])
+def test_prediction_after_a_gathered_batch_is_the_host_batchs(batch):
+    """Predictions before and after one step on a gathered batch: the values of a network trained on the same batch
+    from the host, and not those of before."""
+    nets = [G.FNO(10, 8, 5, width=4, modes=(1, 1, 1), layers=2, d_in=3, d_hidden=8, d_out=2, max_batch=65)
+            for _ in range(2)]
+    rng = np.random.default_rng(6)
+    p = (0.3 * rng.standard_normal(nets[0].n)).astype(np.float32)
+    a = rng.standard_normal((9, 3, 5, 8, 10)).astype(np.float32)
+    t = rng.standard_normal((9, 2, 5, 8, 10)).astype(np.float32)
+    idx = rng.integers(0, 9, batch).tolist()
+    for n in nets:
+        n.set_params(G.unflatten(n.cfg, p))
+    nets[1].set_dataset(a, t)
+    before = nets[0].forward(a[idx])
+    nets[0].train_step(a[idx], t[idx], 1e-3)
+    nets[1].train_step_indices(idx, 1e-3)
+    out, gathered = (n.forward(a[idx]) for n in nets)
+    assert np.all(np.isfinite(out)) and np.array_equal(gathered, out) and not np.array_equal(out, before)
+
+
 def test_resident_dataset_steps_match_host_batches():
     """Steps on mini-batches gathered on the device from a resident training
     set give bit for bit what the same steps on host copies of those samples
