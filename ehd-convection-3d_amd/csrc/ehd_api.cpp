@@ -750,7 +750,20 @@ int ehd_read_fields(ehd_box* b, double* rho, double* q, double* phi, double* ux,
         HIPCHK(launch_efield(b->prec, b->lp, b->phi, b->phibar, b->ex, b->ey, b->ez, b->st));
     for (const auto& e : {std::make_pair(ex, b->ex), std::make_pair(ey, b->ey), std::make_pair(ez, b->ez)})
         if (e.first) c[n++] = HostCopy{HostCopy::kDouble, e.first, e.second, S};
-    return n > 0 ? download(c, n, b->st) : EHD_OK;
+    if (n == 0) return EHD_OK;
+    // A wait for a stream has a thread of the runtime finish the commands queued on
+    // it, some microseconds for each.  Left undone, the first hipFree of the box's
+    // close waited for that, behind whatever threads the program had started
+    // meanwhile (torch's spinning pool); done at the end of the read, it ran beside
+    // those threads and held them up.  So the steps' commands are finished beside
+    // the copies, the copies' own beside the last deliveries.  Passes of FP32S steps, a
+    // read and its conversion by torch / the close after one, mean ms, without the
+    // two waits, with one at the end, and so: 90x154x45 (200 steps) 21.7 / 6.5,
+    // 30.8 / 3.1, 22.2 / 2.2; 64x64x64 (200) 8.7 / 6.4, 12.7 / 1.3, 8.6 / 1.3.  With
+    // the wait beside the deliveries alone 170x48x66 (300) 59 / 3.0, with both 31 /
+    // 3.1, without 31 / 6.8.
+    HIPCHK(hipStreamSynchronize(b->st));
+    return download(c, n, b->st);
 }
 
 int ehd_write_phi(ehd_box* b, const double* phi)

@@ -280,16 +280,14 @@ int download_staged(const HostCopy* c, int count, hipStream_t st, Staging& S)
                 e = send(sent++);
             }
         }
+        // Everything has arrived.  The stream is waited for too, which has a thread
+        // of the runtime finish the copies' commands, here beside the last
+        // deliveries; left undone, that was on the bill of whatever the owner of the
+        // stream did next (ehd_read_fields).
+        if (e == hipSuccess) e = hipStreamSynchronize(st);
         if (e == hipSuccess && !crew.empty())
             for (int k = std::max(0, np - kSlots); k < np; ++k) crew.wait(k);
     }
-    // Waiting for the stream, not only for its last event, is where the runtime
-    // finishes the copies' commands; left undone, the first hipFree of the
-    // box's close waited for that, behind whatever threads the program had
-    // started meanwhile (torch's spinning pool).  FP32S 90x154x45, 200 steps and
-    // a read, the fields converted by torch / close: 21.3 / 5.2 ms without this
-    // wait, 21.4 / 2.1 with it; 122x122x101 FP64, create to close 36.4 / 32.0 ms.
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) return set_error(EHD_EHIP, "device to host copy failed: %s", hipGetErrorString(e));
     drain.done = true;
     return EHD_OK;
