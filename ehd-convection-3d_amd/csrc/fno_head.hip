@@ -30,7 +30,6 @@ namespace {
 constexpr int H = 128, HT = H / 16;   // hidden channels and their 16-channel tiles
 constexpr int PT = 32;                // points of a tile, two 16-point halves
 constexpr int HP = H + 8;             // pitch of a point's hidden channels (bf16)
-constexpr int QP = PT + 8;            // pitch of a hidden channel's points (bf16)
 constexpr int SLICE = 2048;           // points of one partial weight gradient
 
 // LDS written by some lanes of a wave is read by others of the same wave

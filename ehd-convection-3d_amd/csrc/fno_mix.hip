@@ -10,7 +10,7 @@
 // operands once, and each of its waves then streams one mode's weights from
 // memory straight into MFMA operands.  Bound by the
 // weights' traffic: 22 us forward (3.9 TB/s), 37 us for the two adjoints together
-// (4.6 TB/s), which were 75 us each.
+// (4.2 TB/s), which were 75 us each.
 //
 // The products are those of the GEMMs bit for bit: operands rounded to bf16
 // once, one 16x16x32 step over k (channels or batch, at most 32), the real

@@ -531,7 +531,7 @@ hipError_t launch_lbm_f64(const LbmParams& P, const PopBufs& pb, const MacroBufs
 // last-level cache (256 MB) and a row of the lattice is whole cache lines; a
 // streamed part of a line reaches memory on its own.  Measured, us per launch,
 // streaming / plain:
-//   rows of whole lines: FP32S 64x64x64 (226 MB) 23.5 / 21.9, 96x96x64 (255 MB) 52 / 52,
+//   rows of whole lines: FP32S 64x64x64 (113 MB) 23.5 / 21.9, 96x96x64 (255 MB) 52 / 52,
 //     112x112x64 (347 MB) 76 / 76, 128x128x64 (453 MB) 82 / 92, 256x256x128 629 / 692;
 //     FP64 64x64x64 (226 MB) 46 / 39, 72x72x64 (287 MB) 66 / 62,
 //     128x128x32 (453 MB) 86 / 91, 256x256x128 1343 / 1390
